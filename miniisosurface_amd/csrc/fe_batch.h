@@ -37,6 +37,16 @@ struct BatchJob {
     int64_t mask_base;   // first sign-mask word
 };
 
+/* The job's volume pointer, read from memory as what it is, a pointer to device memory: as a plain
+ * pointer its loads become flat ones, for which LDS operations wait too. */
+__device__ __forceinline__ const float* job_volume(const BatchJob& J)
+{
+    typedef const __attribute__((address_space(1))) float* GlobalFloats;
+    GlobalFloats p;
+    __builtin_memcpy(&p, &J.vol, sizeof(p));
+    return (const float*)p;
+}
+
 /* the job whose item range holds `item`: the largest j < njobs with prefix[j] <= item */
 __device__ __forceinline__ int find_job(const int64_t* __restrict__ prefix, int njobs, int64_t item)
 {
@@ -79,43 +89,6 @@ __device__ __forceinline__ void run_queue(uint64_t* __restrict__ ticket, const i
     }
 }
 
-/* The XCD-aware variant of run_queue for pass 4. A persistent block b runs on XCD b mod 8 (the
- * dispatcher hands workgroups to the 8 XCDs in turn), and each XCD takes its items from a queue of
- * its own (ticket x): within job j, XCD x owns the dispatch indices b = 8 t + x < n_j, which
- * emit_block_order maps to the job's row blocks as it maps the single-volume kernel's blocks, so
- * each XCD's L2 sees tiles of neighbouring rows, and all XCDs move through a job's planes
- * together. xprefix[x stride + j]: XCD x's items before job j (jobs [0, njobs) are drawn from).
- * body(job, dispatch index). */
-template <class Body>
-__device__ __forceinline__ void run_queue_xcd(uint64_t* __restrict__ tickets, const int64_t* __restrict__ xprefix,
-                                              int64_t stride, int njobs, int chunk, Body body)
-{
-    __shared__ int64_t s_base;
-    __shared__ int s_job;
-    const int x = (int)(blockIdx.x & 7u);
-    const int64_t* __restrict__ pre = xprefix + (int64_t)x * stride;
-    const int64_t nitems = pre[njobs];
-    for (;;) {
-        __syncthreads();   // every thread has read the previous ticket
-        if (threadIdx.x == 0) {
-            const int64_t b = (int64_t)__hip_atomic_fetch_add((unsigned long long*)&tickets[x],
-                                                              (unsigned long long)chunk, __ATOMIC_RELAXED,
-                                                              __HIP_MEMORY_SCOPE_AGENT);
-            s_base = b;
-            s_job = b < nitems ? find_job(pre, njobs, b) : 0;
-        }
-        __syncthreads();
-        const int64_t base = s_base;
-        if (base >= nitems) break;
-        int j = __builtin_amdgcn_readfirstlane(s_job);
-        const int64_t end = base + chunk < nitems ? base + chunk : nitems;
-        for (int64_t it = base; it < end; ++it) {
-            while (it >= pre[j + 1]) ++j;
-            body(j, 8 * (it - pre[j]) + x);
-        }
-    }
-}
-
 /* clears the queue tickets and the scan's tile status (a kernel, so it can sit in a graph) */
 __global__ __launch_bounds__(256) void k_batch_zero(uint64_t* __restrict__ words, int64_t n)
 {
@@ -139,9 +112,9 @@ __device__ __forceinline__ void batch_classify_item(const BatchJob* __restrict__
     };
     // an item is 4 kShortRows rows of a short-row job (batch_classify_rows), else 4 rows
     if (J.g.W <= 4)
-        fe_classify_short_rows_n(J.vol, J.g, n, sink, blk);
+        fe_classify_short_rows_n(job_volume(J), J.g, n, sink, blk);
     else
-        fe_classify_block_n(J.vol, J.g, n, sink, blk);
+        fe_classify_block_n(job_volume(J), J.g, n, sink, blk);
 }
 
 __global__ __launch_bounds__(256) void k_batch_classify(const BatchJob* __restrict__ jobs,
@@ -203,17 +176,23 @@ __device__ __forceinline__ void batch_emit_item(const uint64_t* __restrict__ s_c
                                                 uint32_t* __restrict__ tris, int j, int64_t blk)
 {
     const BatchJob& J = jobs[j];
+    const float* __restrict__ vol = job_volume(J);
     const uint64_t vbias = voff[J.row_base];
     if (J.unit)
-        fe_emit_rows_block<uint32_t, true>(s_case, s_w, J.vol, mask + J.mask_base, J.g, J.iso, counts + J.row_base,
+        fe_emit_rows_block<uint32_t, true>(s_case, s_w, vol, mask + J.mask_base, J.g, J.iso, counts + J.row_base,
                                            voff + J.row_base, toff + J.row_base, pts, nrm, tris, vbias, blk);
     else
-        fe_emit_rows_block<uint32_t, false>(s_case, s_w, J.vol, mask + J.mask_base, J.g, J.iso, counts + J.row_base,
+        fe_emit_rows_block<uint32_t, false>(s_case, s_w, vol, mask + J.mask_base, J.g, J.iso, counts + J.row_base,
                                             voff + J.row_base, toff + J.row_base, pts, nrm, tris, vbias, blk);
 }
 
 /* Pass 4 for the first nemit jobs, from the one queue (items [0, nitems), tickets[0]) or, with
- * xprefix, the XCD queues (run_queue_xcd, tickets[0 .. 8)). */
+ * xprefix, from one queue per XCD (tickets[0 .. 8)): a persistent block b runs on XCD b mod 8 (the
+ * dispatcher hands workgroups to the 8 XCDs in turn), and within job j, XCD x owns the dispatch
+ * indices b = 8 t + x < n_j, which emit_block_order maps to the job's row blocks as it maps the
+ * single-volume kernel's blocks, so each XCD's L2 sees tiles of neighbouring rows, and all XCDs move
+ * through a job's planes together. xprefix[x (njobs + 1) + j]: XCD x's items before job j. Both take
+ * their items through one loop, so that the kernel holds pass 4 once. */
 __device__ __forceinline__ void batch_emit_queue(const uint64_t* __restrict__ s_case, EmitRowsLds* s_w,
                                                  const BatchJob* __restrict__ jobs, const int64_t* __restrict__ prefix,
                                                  int njobs, int64_t nitems, int chunk,
@@ -224,15 +203,12 @@ __device__ __forceinline__ void batch_emit_queue(const uint64_t* __restrict__ s_
                                                  uint32_t* __restrict__ tris, uint64_t* __restrict__ tickets,
                                                  const int64_t* __restrict__ xprefix, int nemit)
 {
-    if (xprefix)
-        run_queue_xcd(tickets, xprefix, (int64_t)njobs + 1, nemit, chunk, [&](int j, int64_t b) {
-            batch_emit_item(s_case, s_w, jobs, mask, counts, voff, toff, pts, nrm, tris, j,
-                            emit_block_order(b, prefix[j + 1] - prefix[j], jobs[j].g));
-        });
-    else
-        run_queue(tickets, prefix, njobs, nitems, chunk, [&](int j, int64_t blk) {
-            batch_emit_item(s_case, s_w, jobs, mask, counts, voff, toff, pts, nrm, tris, j, blk);
-        });
+    const int x = xprefix ? (int)(blockIdx.x & 7u) : 0;
+    const int64_t* __restrict__ pre = xprefix ? xprefix + (int64_t)x * (njobs + 1) : prefix;
+    run_queue(tickets + x, pre, xprefix ? nemit : njobs, xprefix ? pre[nemit] : nitems, chunk, [&](int j, int64_t it) {
+        const int64_t blk = xprefix ? emit_block_order(8 * it + x, prefix[j + 1] - prefix[j], jobs[j].g) : it;
+        batch_emit_item(s_case, s_w, jobs, mask, counts, voff, toff, pts, nrm, tris, j, blk);
+    });
 }
 
 /* Pass 4 for the first jobs (items [0, nitems)); writes nothing when their output exceeds the
@@ -253,7 +229,7 @@ __global__ __launch_bounds__(256) void k_batch_emit(const BatchJob* __restrict__
     // need: vertices and triangles of the emitted jobs (the totals, or the first vertex and
     // triangle of the first job not emitted)
     if (need[0] > cap_v || need[1] > cap_t) return;
-    s_case[threadIdx.x] = kCaseEdges[threadIdx.x];
+    s_case[threadIdx.x] = kCaseSlots.v[threadIdx.x];
     batch_emit_queue(s_case, s_w, jobs, prefix, njobs, nitems, chunk, mask, counts, voff, toff, pts, nrm, tris,
                      tickets, xprefix, nemit);
 }
@@ -283,7 +259,7 @@ __global__ __launch_bounds__(256) void k_batch_fused(const BatchJob* __restrict_
     cg::grid_group grid = cg::this_grid();
     __shared__ uint64_t s_case[256];
     __shared__ EmitRowsLds s_w[4];
-    s_case[threadIdx.x] = kCaseEdges[threadIdx.x];
+    s_case[threadIdx.x] = kCaseSlots.v[threadIdx.x];
     run_queue(state + 0, cls_prefix, ngroups, ncls, chunk,
               [&](int q, int64_t blk) { batch_classify_item(jobs, group_job, mask, q, blk); });
     grid.sync();

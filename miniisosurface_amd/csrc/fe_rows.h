@@ -8,10 +8,10 @@
  * contiguous range of the output, and its triangles one contiguous range too.
  *
  *   k_fe_count_rows  pass 1b + 2 (trims, x/y/z cut counts, triangle counts per row)
- *   k_fe_emit_rows   pass 4: vertices (cut edges compacted into LDS lists, x-edges then y/z-edges,
- *                    one vertex per lane, written at consecutive addresses), then triangles (active
- *                    cells listed in output order, resolved one triangle per lane, vertex ids from
- *                    row offsets plus popcount ranks held in LDS)
+ *   k_fe_emit_rows   pass 4: vertices (voxels with a cut edge listed in output order in LDS, one per
+ *                    lane, its up to three vertices from one set of voxel loads), and triangles
+ *                    (active cells listed in output order, one per lane its case and its twelve
+ *                    vertex ids into LDS, then one triangle per lane)
  */
 #ifndef MINIISO_FE_ROWS_H
 #define MINIISO_FE_ROWS_H
@@ -115,10 +115,12 @@ __device__ __forceinline__ uint32_t seg_reduce(uint32_t v, int Wp)
 
 __device__ __forceinline__ uint32_t seg_sum(uint32_t v, int Wp) { return seg_reduce<OpAdd>(v, Wp); }
 
-/* Sign-mask words around lane (row r, word w): rows (j,k) (j+1,k) (j,k+1) (j+1,k+1), each with
- * the next word for the +1 neighbours. Rows outside the grid read as zero. */
+/* Sign-mask words around lane (row r, word w): rows (j,k) (j+1,k) (j,k+1) (j+1,k+1). n holds the
+ * lowest bit of each row's next word (the +1 neighbour of bit 63), taken from the next lane, which
+ * holds that word of the same row, or 0 in the row's last word. Rows outside the grid read as zero. */
 struct LaneWords {
-    uint64_t m[4], n[4];
+    uint64_t m[4];
+    uint32_t n[4];
 };
 
 __device__ __forceinline__ LaneWords load_lane_words(const uint64_t* __restrict__ mask, const Geom& g, int64_t r,
@@ -128,16 +130,24 @@ __device__ __forceinline__ LaneWords load_lane_words(const uint64_t* __restrict_
     const int64_t W = g.W;
     const int64_t rows[4] = {r, r + 1, r + g.ny, r + g.ny + 1};
     const bool rok[4] = {ok, ok && has_y, ok && has_z, ok && has_y && has_z};
-    const bool nxt = w + 1 < W;
+    uint32_t low = 0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        L.m[q] = rok[q] ? mask[rows[q] * W + w] : 0ull;
-        L.n[q] = (rok[q] && nxt) ? mask[rows[q] * W + w + 1] : 0ull;
-    }
+    for (int q = 0; q < 4; ++q) L.m[q] = rok[q] ? mask[rows[q] * W + w] : 0ull;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) low |= ((uint32_t)L.m[q] & 1u) << q;
+    const uint32_t of_next = dpp_u32<kDppWaveShl1>(low);   // every lane takes part
+    low = w + 1 < W ? of_next : 0u;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) L.n[q] = __builtin_amdgcn_ubfe(low, q, 1);
     return L;
 }
 
-__device__ __forceinline__ uint64_t shifted(uint64_t m, uint64_t next) { return (m >> 1) | (next << 63); }
+/* the word's bits moved down by one, `next` (bit 0) moving in at the top */
+__device__ __forceinline__ uint64_t shifted(uint64_t m, uint32_t next)
+{
+    const uint32_t lo = (uint32_t)m, hi = (uint32_t)(m >> 32);
+    return (uint64_t)__builtin_amdgcn_alignbit(next, hi, 1) << 32 | __builtin_amdgcn_alignbit(hi, lo, 1);
+}
 
 /* The 8 corner words of a lane: sign bits at i (m) and at i+1 (s) of the 4 rows. */
 struct CornerWords {
@@ -228,8 +238,8 @@ __device__ __forceinline__ void fe_count_rows_block(const uint64_t* __restrict__
     const int64_t j = jk.j, k = jk.k;
     const bool has_y = j < g.ny - 1, has_z = k < g.nz - 1;
     const LaneWords L = load_lane_words(mask, g, r, rl.w, ok, has_y, has_z);
-    // the words and bit 0 of the next words (corner i + 1 of bit 63), as far as the lane loaded them
-    const uint64_t any = L.m[0] | L.m[1] | L.m[2] | L.m[3] | ((L.n[0] | L.n[1] | L.n[2] | L.n[3]) & 1ull);
+    // the words and bit 0 of the next words (corner i + 1 of bit 63)
+    const uint64_t any = L.m[0] | L.m[1] | L.m[2] | L.m[3] | (uint64_t)(L.n[0] | L.n[1] | L.n[2] | L.n[3]);
     if (__ballot(any != 0ull) == 0ull) {
         // every voxel the wavefront's rows see is below the isovalue (most wavefronts at a
         // sparse, high isovalue): no cut edge, no triangle, an empty trim
@@ -429,58 +439,60 @@ __device__ __forceinline__ void vertex_yz(const float* __restrict__ v, const Geo
     edge_finish<Unit>(g, axis, i, j, k, w, ga, gb, p, nrm);
 }
 
-/* A vertex-list entry: output position (wavefront-relative) << 14 | axis << 12 | lane << 6 | bit,
- * the lane (q, w) and bit b naming row q of the wavefront and i = 64 w + b. The row is row j0 + q
- * of plane k0, carried into the following planes. */
+/* Flying Edges corner coordinates of the edges from an origin (i,j,k) below the last index of each
+ * axis (fe_edge_corners), and the end of edge_point with them: p = a + w (b - a), where b - a is 1 or
+ * spacing along the edge and a - a (0, or NaN) across it. */
 template <bool Unit>
-__device__ __forceinline__ void emit_vertex(const float* __restrict__ plane, const Geom& g, float iso, uint32_t ent,
-                                            int j0, int k0, int wp_log2, bool xgroup, float p[3], float nrm[3])
-{
-    const int ny = (int)g.ny;
-    const int src = (int)((ent >> 6) & 63);
-    int j = j0 + (src >> wp_log2), dk = 0;
-    while (j >= ny) {
-        j -= ny;
-        ++dk;
+struct CornerCoords {
+    float A[3];
+    __device__ __forceinline__ CornerCoords(const Geom& g, int i, int j, int k)
+    {
+        if (Unit) {
+            A[0] = (float)i; A[1] = (float)j; A[2] = (float)(k + (int)g.kofs);
+        } else {
+            A[0] = g.org[0] + (float)i * g.sp[0];
+            A[1] = g.org[1] + (float)j * g.sp[1];
+            A[2] = g.org[2] + (float)(k + (int)g.kofs) * g.sp[2];
+        }
     }
-    const int i = ((src & ((1 << wp_log2) - 1)) << 6) | (int)(ent & 63);
-    const uint32_t off = (uint32_t)dk * (uint32_t)(g.nx * g.ny) + (uint32_t)j * (uint32_t)g.nx + (uint32_t)i;
-    if (xgroup)
-        vertex_x<Unit>(plane + off, g, iso, i, j, k0 + dk, p, nrm);
-    else
-        vertex_yz<Unit>(plane + off, g, iso, (int)((ent >> 12) & 3), i, j, k0 + dk, p, nrm);
-}
+    __device__ __forceinline__ void finish(const Geom& g, int axis, float w, const float ga[3], const float gb[3],
+                                           float p[3], float nrm[3]) const
+    {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            if (Unit)
+                p[c] = A[c] + (c == axis ? w : w * 0.0f);
+            else
+                p[c] = A[c] + w * ((c == axis ? A[c] + g.sp[c] : A[c]) - A[c]);
+            nrm[c] = ga[c] + w * (gb[c] - ga[c]);
+        }
+    }
+};
 
 /* ------------------------------------------------------------------ pass 4: fused emit */
-constexpr int kEmitVertCap = 512;   // vertex-list entries per wavefront and round
-constexpr int kEmitCellCap = 512;   // active-cell entries per wavefront and round
+constexpr int kEmitCellCap = 240;   // active-cell entries per wavefront and round
 constexpr int kEmitTriCap = 64 * 5; // triangles of one group of 64 cells (at most 5 each)
-constexpr int kStageVerts = 320;    // vertices staged per wavefront and output window
+constexpr int kIdStride = 7;        // dwords per cell of ids: odd, so that cells spread over the banks
+constexpr int kOriginCap = 640;     // origin entries per wavefront and round
 
-/* LDS of one wavefront. The triangles use the 8 edge-combination cut words and id bases of each
- * lane, the cell list and the triangle map; the vertices before them use the same bytes for their
- * list and staging window (sv), or, without staging, the vertex list (u.vlist). */
+/* LDS of one wavefront. words: the mask bits of a lane's four rows by 32-voxel halves (half h of lane
+ * l at 2 l + h, followed by the next half's for the corner i + 1; a row that is not there repeats
+ * row 0, so that it shows no cut). rank: per half, the id ranks of the eight edge combinations before
+ * it, 16 bits each, (0,1) (2,3) (4,5) (6,7). origins: the vertices' list. t: the triangles' cell list
+ * and, for the current 64 cells, their ids and the map of their triangles. Four blocks share a CU; a
+ * fifth (the list in t's bytes, made again after the triangles) measured 1.48 against 1.445 ms at
+ * 1024^3, three 1.73. */
 struct EmitRowsLds {
-    union {
-        struct {
-            uint64_t cut[8][64];
-            uint32_t base[8][64];
-            union {
-                uint32_t vlist[kEmitVertCap];
-                struct {
-                    uint32_t cells[kEmitCellCap];
-                    uint32_t map[kEmitTriCap];
-                } t;
-            } u;
-        };
-        struct {
-            uint32_t list[kStageVerts];
-            float stage[6 * kStageVerts];   // points, then normals, of the window's vertices
-        } sv;
-    };
+    uint4 rank[128];
+    uint32_t words[4][130];
+    uint16_t origins[kOriginCap];
+    struct {
+        uint32_t ids[64 * kIdStride];
+        uint32_t map[kEmitTriCap];
+        uint16_t cells[kEmitCellCap];
+    } t;
 };
-static_assert(sizeof(EmitRowsLds) == 8 * 64 * 8 + 8 * 64 * 4 + (kEmitCellCap + kEmitTriCap) * 4,
-              "the staging window fits in the triangles' bytes");
+static_assert(sizeof(EmitRowsLds) * 4 + 256 * 8 <= 40960, "four blocks of pass 4 share a CU's 160 KB");
 
 /* case of the cell at bit b of a 32-bit half: h[q] holds corner v_q's bits (the case's bit order) */
 __device__ __forceinline__ uint32_t case_of_half(const uint32_t h[8], int b)
@@ -492,375 +504,421 @@ __device__ __forceinline__ uint32_t case_of_half(const uint32_t h[8], int b)
 }
 
 /* Pass 4 for the (row, word) lane layout in one launch: each wavefront writes the vertices of its
- * rows (one vertex per lane from LDS lists), then the triangles of its cell rows (active cells
- * listed per lane, resolved one cell and then one triangle per lane). */
+ * rows, then the triangles of its cell rows. */
 
 /* Per-wavefront state of pass 4 in the lane-row layout: rows r0 .. r0 + rpw - 1, lane (q, w)
- * holding word w of row r0 + q and the words of its three neighbour rows. */
+ * holding word w of row r0 + q. */
 struct EmitRows {
     RowLanes rl;
-    int lane, wv;
-    int64_t r0, r;
-    bool ok, emit, has_y, has_z;   // emit: the row is in the range pass 4 writes
-    LaneWords L;
-    uint64_t v0, t0, vb, eb;
-    int64_t k0;   // the wavefront's first row is (j0, k0)
+    int lane, wv, wp_log2;
+    int64_t r0;
+    uint64_t v0, v2, t0;           // first vertex of row r0 and of row r0 + ny, first triangle of row r0
+    uint64_t origins, act;         // this lane's voxels with a cut edge that pass 4 writes; its active cells
+    int64_t k0;                    // the wavefront's first row is (j0, k0)
     int j0;
 };
 
-__device__ __forceinline__ bool emit_rows_setup(EmitRows& E, const uint64_t* __restrict__ mask, const Geom& g,
-                                                const RowCounts* __restrict__ counts,
+/* Loads the wavefront's mask words and row state and fills words and rank. False: nothing to write.
+ * The row state comes from one lane per row and reaches the others by lane moves: a load that 64
+ * lanes make of their row's entry costs the L1 one access per four lanes, 1024^3 about 100 of a
+ * wavefront's 1320. */
+__device__ __forceinline__ bool emit_rows_setup(EmitRows& E, EmitRowsLds* s_w, const uint64_t* __restrict__ mask,
+                                                const Geom& g, const RowCounts* __restrict__ counts,
                                                 const uint64_t* __restrict__ voff, const uint64_t* __restrict__ toff,
                                                 int64_t blk)
 {
     E.lane = lane_id();
     E.wv = wave_in_block();
     E.rl = row_lanes(g.W);
+    const RowLanes& rl = E.rl;
     const int64_t R = g.ny * g.nz;
-    E.r0 = (blk * 4 + E.wv) * E.rl.rpw;
+    E.r0 = (blk * 4 + E.wv) * rl.rpw;
     if (E.r0 >= R) return false;
-    E.r = E.r0 + E.rl.q;
-    E.ok = E.r < R && E.rl.w < g.W;
-    {
-        // a wavefront whose rows have no vertex and no triangle leaves before reading mask words
-        // (most of them at a sparse isovalue)
-        bool some = false;
-        if (E.ok && E.rl.w == 0) {
-            const RowCounts c = counts[E.r];
-            some = (c.x | c.y | c.z | c.t) != 0u;
-        }
-        if (__ballot(some) == 0ull) return false;
-    }
-    E.emit = E.ok && E.r >= g.emit_lo && E.r < g.emit_hi;
-    const RowJK jk = split_row(E.r0, E.rl.q, g.ny);
-    E.has_y = jk.j < g.ny - 1;
-    E.has_z = jk.k < g.nz - 1;
-    E.L = load_lane_words(mask, g, E.r, E.rl.w, E.ok, E.has_y, E.has_z);
+    const int64_t r = E.r0 + rl.q;
+    const bool ok = r < R && rl.w < g.W;
+    const bool first = ok && rl.w == 0;        // the lane that holds the row's state
+    // a wavefront whose rows have no vertex and no triangle leaves before reading mask words
+    // (most of them at a sparse isovalue)
+    RowCounts c{0u, 0u, 0u, 0u};
+    if (first) c = counts[r];
+    if (__ballot((c.x | c.y | c.z | c.t) != 0u) == 0ull) return false;
+    const RowJK jk = split_row(E.r0, rl.q, g.ny);
+    const bool has_y = jk.j < g.ny - 1, has_z = jk.k < g.nz - 1;
+    const LaneWords L = load_lane_words(mask, g, r, rl.w, ok, has_y, has_z);
     E.v0 = voff[E.r0];
     E.t0 = toff[E.r0];
-    E.vb = low_bits(g.nx - 64 * E.rl.w);
-    E.eb = low_bits(g.nx - 1 - 64 * E.rl.w);
     E.k0 = uniform_div(E.r0, g.ny);
     E.j0 = (int)(E.r0 - E.k0 * g.ny);
+    // the row's vertex offset and, in the plane above, that row's, from v0 and v2 (below 2^16: at
+    // most 65 rows of 64 words in all hold 3 * 64 * 65 voxels' edges)
+    const bool up = E.r0 + g.ny < R;
+    E.v2 = up ? voff[E.r0 + g.ny] : 0ull;
+    uint32_t own = 0, above = 0, above_x = 0;
+    if (first) {
+        own = (uint32_t)(voff[r] - E.v0);
+        if (r + g.ny < R) {
+            above = (uint32_t)(voff[r + g.ny] - E.v2);
+            above_x = counts[r + g.ny].x;
+        }
+    }
+    // first ids of the row's x-edges (a, low), z-edges (a, high), y-edges (b); x- and y-edges above (c)
+    uint32_t a = own | (own + c.x + c.y) << 16, b = own + c.x, cc = above | (above + above_x) << 16;
+    const int head = rl.q << (6 - __builtin_ctz((unsigned)rl.rpw)), next = head + rl.Wp;
+    uint32_t a1 = (uint32_t)__shfl((int)a, next & 63), c1 = (uint32_t)__shfl((int)cc, next & 63);
+    if (next >= 64) {
+        // the row after the wavefront's last one
+        const int64_t rn = E.r0 + rl.rpw;
+        a1 = c1 = 0;
+        if (rn < R) {
+            const uint32_t o = (uint32_t)(voff[rn] - E.v0);
+            const RowCounts cn = counts[rn];
+            a1 = o | (o + cn.x + cn.y) << 16;
+        }
+        if (rn + g.ny < R) c1 = (uint32_t)(voff[rn + g.ny] - E.v2);
+    }
+    a = (uint32_t)__shfl((int)a, head);
+    b = (uint32_t)__shfl((int)b, head);
+    cc = (uint32_t)__shfl((int)cc, head);
+    E.wp_log2 = 6 - __builtin_ctz((unsigned)rl.rpw);
+
+    const uint64_t vb = low_bits(g.nx - 64 * rl.w), eb = low_bits(g.nx - 1 - 64 * rl.w);
+    const uint64_t cw[8] = {(L.m[0] ^ shifted(L.m[0], L.n[0])) & eb, (L.m[1] ^ shifted(L.m[1], L.n[1])) & eb,
+                            (L.m[2] ^ shifted(L.m[2], L.n[2])) & eb, (L.m[3] ^ shifted(L.m[3], L.n[3])) & eb,
+                            (L.m[0] ^ L.m[1]) & vb, (L.m[2] ^ L.m[3]) & vb,
+                            (L.m[0] ^ L.m[2]) & vb, (L.m[1] ^ L.m[3]) & vb};
+    const uint32_t base[4] = {(a & 0xFFFFu) | a1 << 16, (cc & 0xFFFFu) | c1 << 16, b | (cc & 0xFFFF0000u),
+                              a >> 16 | (a1 & 0xFFFF0000u)};
+    uint32_t lo[4], hi[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        // two combinations per segmented scan and per dword
+        lo[q] = base[q] + seg_excl_scan((uint32_t)__popcll(cw[2 * q]) | (uint32_t)__popcll(cw[2 * q + 1]) << 16, rl.Wp,
+                                        rl.w);
+        hi[q] = lo[q] + ((uint32_t)__popc((uint32_t)cw[2 * q]) | (uint32_t)__popc((uint32_t)cw[2 * q + 1]) << 16);
+    }
+    EmitRowsLds& S = s_w[E.wv];
+    S.rank[2 * E.lane] = uint4{lo[0], lo[1], lo[2], lo[3]};
+    S.rank[2 * E.lane + 1] = uint4{hi[0], hi[1], hi[2], hi[3]};
+    const uint64_t m[4] = {L.m[0], has_y ? L.m[1] : L.m[0], has_z ? L.m[2] : L.m[0], L.m[3]};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        S.words[q][2 * E.lane] = (uint32_t)m[q];
+        S.words[q][2 * E.lane + 1] = (uint32_t)(m[q] >> 32);
+    }
+    const bool emit = ok && r >= g.emit_lo && r < g.emit_hi;
+    E.origins = emit ? cw[0] | (m[0] ^ m[1]) | (m[0] ^ m[2]) : 0ull;
+    E.act = emit && has_y && has_z ? active_cells(L, eb) : 0ull;
+    wave_sync();
     return true;
 }
 
-/* Vertices of the wavefront's rows, [x][y][z] cuts per row, through an LDS list of kEmitVertCap
- * entries. Voxel offsets are 32-bit from plane k0. With vmap, vertex id v is written at vmap[v]. */
-template <bool Unit, typename Index = uint32_t>
-__device__ __forceinline__ void emit_rows_vertices(const EmitRows& E, uint32_t* list, const float* __restrict__ vol,
-                                                   const Geom& g, float iso, float* __restrict__ pts,
-                                                   float* __restrict__ nrm, const Index* __restrict__ vmap = nullptr)
+/* bits below position b (0 .. 31) */
+__device__ __forceinline__ uint32_t bits_below(uint32_t b) { return __builtin_amdgcn_ubfe(0xFFFFFFFFu, 0, b); }
+
+/* Appends the positions (lane << 6 | bit) of a lane's set bits to list, from entry `first` on as far
+ * as they fall in [win, win + Cap). */
+template <int Cap>
+__device__ __forceinline__ void list_bits(uint64_t bits, uint32_t first, uint32_t win, int lane, uint16_t* list)
 {
-    const RowLanes& rl = E.rl;
-    const LaneWords& L = E.L;
-    const int lane = E.lane;
-    const uint64_t v0 = E.v0, vb = E.vb, eb = E.eb;
-    const bool has_y = E.has_y, has_z = E.has_z;
-    const int j0 = E.j0;
-    const int64_t k0 = E.k0;
-    const float* __restrict__ plane = vol + k0 * (g.nx * g.ny);
-    const uint64_t live = E.emit ? ~0ull : 0ull;
-    const uint64_t cut[3] = {(L.m[0] ^ shifted(L.m[0], L.n[0])) & eb & live,
-                             has_y ? ((L.m[0] ^ L.m[1]) & vb & live) : 0ull,
-                             has_z ? ((L.m[0] ^ L.m[2]) & vb & live) : 0ull};
-    const uint32_t c0 = __popcll(cut[0]), c1 = __popcll(cut[1]), c2 = __popcll(cut[2]);
-    // x and y counts share one segmented scan (row totals below 2^16)
-    const uint32_t p01 = c0 | c1 << 16;
-    const uint32_t inc01 = seg_incl<OpAdd>(p01, rl.Wp, rl.w);
-    const uint32_t tot01 = (uint32_t)__shfl((int)inc01, (lane & ~(rl.Wp - 1)) + rl.Wp - 1);
-    const uint32_t ex01 = inc01 - p01;
-    const uint32_t X = tot01 & 0xFFFFu, Y = tot01 >> 16;
-    const uint32_t lane_tot = c0 + c1 + c2;
-    const uint32_t incl = wave_incl_scan_u32(lane_tot);
-    const uint32_t before_row = __shfl(incl - lane_tot, rl.q * rl.Wp);
-    const uint32_t pos0 = before_row + (ex01 & 0xFFFFu);
-    const uint32_t pos1 = before_row + X + (ex01 >> 16);
-    const uint32_t pos2 = before_row + X + Y + seg_excl_scan(c2, rl.Wp, rl.w);
-    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-    // Two lists, x-edges and then y/z-edges, so that the lanes of one step take the same load
-    // pattern; each entry carries its output position. The x-edges are listed in lane order,
-    // which is output order within each row, so that a step stores runs of consecutive vertices
-    // (they mostly fit one step, whose gathers then touch the same lines in any order; 1024^3:
-    // 1.594 against 1.615 ms). For rows of 16 words and more, the y/z-edges run word-major (word
-    // w of all the wavefront's rows, then word w + 1), so that each of their steps gathers from a
-    // narrow x-range of neighbouring rows and shares cache lines (1024^3: 1.65 against 1.69 ms);
-    // for shorter rows in output order, so that one step's stores are contiguous (512^3 gyroid:
-    // 0.425 against 0.44 ms; 256^3 and 384^3 likewise).
-    const bool word_major = rl.Wp >= 16;
-    const int wp_log2 = __builtin_ctz((unsigned)rl.Wp), rpw_log2 = 6 - wp_log2;
-    const int tl = word_major ? rl.w * rl.rpw + rl.q : lane;                  // y/z list position of this lane
-    const int from = word_major ? ((lane & (rl.rpw - 1)) << wp_log2) + (lane >> rpw_log2) : lane;   // lane at position `lane`
-    const uint32_t c12t = (uint32_t)__shfl((int)(c1 + c2), from);
-    const uint32_t xincl = wave_incl_scan_u32(c0), yzincl_t = wave_incl_scan_u32(c12t);
-    const uint32_t xtotal = (uint32_t)__builtin_amdgcn_readlane((int)xincl, 63);
-    const uint32_t xfirst = xincl - c0;
-    const uint32_t yzfirst = (uint32_t)__shfl((int)(yzincl_t - c12t), tl);
+    uint32_t p = first - win;
 #pragma unroll
-    for (int grp = 0; grp < 2; ++grp) {
-        const uint32_t gtotal = grp ? total - xtotal : xtotal;
-        const uint32_t gfirst = grp ? yzfirst : xfirst;
-        for (uint32_t win = 0; win < gtotal; win += kEmitVertCap) {
-            const uint32_t wend = win + kEmitVertCap;
-            uint32_t idx = gfirst;
+    for (int h = 0; h < 2; ++h) {
+        const uint32_t ent = (uint32_t)lane << 6 | (uint32_t)h << 5;
+        for (uint32_t a = h ? (uint32_t)(bits >> 32) : (uint32_t)bits; a; a &= a - 1, ++p)
+            if (p < (uint32_t)Cap) list[p] = (uint16_t)(ent | (uint32_t)__builtin_ctz(a));
+    }
+}
+
+/* The voxels around an inner origin (i,j,k): its row from i - 1 to i + 2, the rows j + 1 and k + 1
+ * from i - 1 to i + 1, the rows j - 1 and k - 1 from i to i + 1; then, for a y-edge, (j + 2),
+ * (j + 1, k - 1), for a z-edge, (k + 2), (j - 1, k + 1), and for either, (j + 1, k + 1), each at i. */
+struct Around {
+    Vox4 r;
+    Vox3 yp, zp;
+    Vox2 ym, zm, y2, yz, z2, zy, d;
+};
+
+/* The first voxel of a pair, the second one kept as read (the compiler would narrow the load). */
+__device__ __forceinline__ float of_pair(const Vox2& v)
+{
+    asm volatile("" ::"v"(v.y));
+    return v.x;
+}
+
+/* Vertices: one origin -- a voxel with a cut edge along x, y or z -- per lane; its up to three vertices
+ * share the voxels around it. The gathers are bound by the L1, which takes one access per 128-byte
+ * line and four lanes (a 4-byte gather mostly one per lane, so single voxels are read in pairs): 3.6
+ * accesses per vertex by origin against 6.1 with an edge per lane (value noise at 1024^3, counted
+ * from the mask; all of pass 4, from the L1's counter: 5.5 against 8.8). Pass 4 at 1024^3, with the
+ * triangles of emit_rows_triangles: 1.59 -> 1.37-1.40 ms; 512^3 gyroid 0.41 -> 0.34-0.36 ms. Vertices are
+ * stored from the lanes: put in windows of 192 at their place in LDS and stored in 16-byte pieces
+ * they took the same time at 1024^3 and 3% more at 512^3, where a wavefront has several windows. */
+
+/* One step of the vertices: a lane's origin, its cut edges and their ids (from v0), its voxels. */
+struct VertexStep {
+    uint32_t ent, at[3];
+    bool any, inner, cut[3];
+    int j, k;
+    Around a;
+};
+
+/* Where the wavefront's rows lie, and its origins: in output order, so that a step's x-, y- and z-edge
+ * vertices leave in runs of neighbouring ids (1024^3: 1.405 ms against 1.445 ms with word w of all rows
+ * before word w + 1, whose gathers share more lines). */
+struct VertexRows {
+    const float* __restrict__ row0;   // voxel (0, j0, k0)
+    bool rows_inner;                  // every row at least one row from a near face, two from a far one
+    uint32_t n, first;                // the wavefront's origins; this lane's first in their order
+};
+
+__device__ __forceinline__ VertexRows vertex_rows(const EmitRows& E, const float* __restrict__ vol, const Geom& g)
+{
+    VertexRows R;
+    R.row0 = vol + E.r0 * g.nx;
+    R.rows_inner = E.j0 >= 1 && E.j0 + E.rl.rpw <= (int)g.ny - 2 && E.k0 >= 1 && E.k0 <= (int)g.nz - 3;
+    const uint32_t cnt = (uint32_t)__popcll(E.origins);
+    const uint32_t incl = wave_incl_scan_u32(cnt);
+    R.n = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+    R.first = incl - cnt;
+    return R;
+}
+
+/* base + off bytes, off per lane and base the same in every lane: a scalar base and a 32-bit offset */
+template <typename T>
+__device__ __forceinline__ T load_at(const float* __restrict__ base, uint32_t off)
+{
+    T t;
+    __builtin_memcpy(&t, reinterpret_cast<const char*>(base) + off, sizeof(T));
+    return t;
+}
+
+/* Takes this lane's origin (list entry e, if below n) and requests its voxels. */
+__device__ __forceinline__ void vertex_load(VertexStep& V, const EmitRows& E, const EmitRowsLds& S, const VertexRows& R,
+                                            const Geom& g, uint32_t e, uint32_t n)
+{
+    const int nx = (int)g.nx, ny = (int)g.ny, nz = (int)g.nz;
+    const int64_t sy = g.nx, sz = g.nx * g.ny;
+    V.any = e < n;
+    V.ent = V.any ? (uint32_t)S.origins[e] : 0u;
+    const uint32_t h2 = V.ent >> 5, b = V.ent & 31;
+    const int i = (int)(V.ent & ((64u << E.wp_log2) - 1u)), q = (int)(V.ent >> (6 + E.wp_log2));
+    const uint32_t w0 = S.words[0][h2], n0 = S.words[0][h2 + 1];
+    const uint32_t x = w0 ^ __builtin_amdgcn_alignbit(n0, w0, 1), y = w0 ^ S.words[1][h2], z = w0 ^ S.words[2][h2];
+    const uint4 rk = S.rank[h2];
+    const uint32_t below = bits_below(b);
+    V.cut[0] = V.any && ((x >> b) & 1u) && i < nx - 1;
+    V.cut[1] = V.any && ((y >> b) & 1u);
+    V.cut[2] = V.any && ((z >> b) & 1u);
+    V.at[0] = (rk.x & 0xFFFFu) + (uint32_t)__popc(x & below);
+    V.at[1] = (rk.z & 0xFFFFu) + (uint32_t)__popc(y & below);
+    V.at[2] = (rk.w & 0xFFFFu) + (uint32_t)__popc(z & below);
+    V.j = E.j0 + q;
+    V.k = (int)E.k0;
+    V.inner = V.any && (uint32_t)(i - 1) < (nx > 3 ? (uint32_t)(nx - 3) : 0u);
+    if (!R.rows_inner) {
+        while (V.j >= ny) {
+            V.j -= ny;
+            ++V.k;
+        }
+        V.inner = V.inner && V.j >= 1 && V.j <= ny - 3 && V.k >= 1 && V.k <= nz - 3;
+    }
+    if (V.inner) {
+        const float* __restrict__ v = R.row0;
+        const uint32_t off = 4 * ((uint32_t)q * (uint32_t)nx + (uint32_t)i);   // below 2^20
+        Around& a = V.a;
+        a.r = load_at<Vox4>(v - 1, off);
+        a.yp = load_at<Vox3>(v + sy - 1, off);
+        a.zp = load_at<Vox3>(v + sz - 1, off);
+        a.ym = load_at<Vox2>(v - sy, off);
+        a.zm = load_at<Vox2>(v - sz, off);
+        if (V.cut[1]) {
+            a.y2 = load_at<Vox2>(v + 2 * sy, off);
+            a.yz = load_at<Vox2>(v + sy - sz, off);
+        }
+        if (V.cut[2]) {
+            a.z2 = load_at<Vox2>(v + 2 * sz, off);
+            a.zy = load_at<Vox2>(v + sz - sy, off);
+        }
+        if (V.cut[1] || V.cut[2]) a.d = load_at<Vox2>(v + sy + sz, off);
+    }
+}
+
+/* Computes and stores the step's vertices. */
+template <bool Unit, bool Map, typename Index>
+__device__ __forceinline__ void vertex_store(const VertexStep& V, const EmitRows& E, const VertexRows& R, const Geom& g,
+                                             float iso, float* __restrict__ pts, float* __restrict__ nrm,
+                                             const Index* __restrict__ vmap)
+{
+    const int i = (int)(V.ent & ((64u << E.wp_log2) - 1u)), q = (int)(V.ent >> (6 + E.wp_log2));
+    auto put = [&](uint32_t v, const float p[3], const float nn[3]) {
+        const Vox3 vp{p[0], p[1], p[2]}, vn{nn[0], nn[1], nn[2]};
+        if (Map) {
+            const uint64_t id = (uint64_t)vmap[E.v0 + v];
+            __builtin_memcpy(pts + 3 * id, &vp, sizeof(vp));
+            __builtin_memcpy(nrm + 3 * id, &vn, sizeof(vn));
+        } else {
+            const uint32_t off = 12 * v;   // below 2^20
+            __builtin_memcpy(reinterpret_cast<char*>(pts + 3 * E.v0) + off, &vp, sizeof(vp));
+            __builtin_memcpy(reinterpret_cast<char*>(nrm + 3 * E.v0) + off, &vn, sizeof(vn));
+        }
+    };
+    if (V.inner) {
+        const Around& a = V.a;
+        const float ga[3] = {central<Unit>(a.r.x, a.r.z, g.sp[0]), central<Unit>(a.ym.x, a.yp.y, g.sp[1]),
+                             central<Unit>(a.zm.x, a.zp.y, g.sp[2])};
+        const CornerCoords<Unit> cc(g, i, V.j, V.k);
+        const float num = iso - a.r.y;
+        float p[3], nn[3];
+        if (V.cut[0]) {
+            const float gb[3] = {central<Unit>(a.r.y, a.r.w, g.sp[0]), central<Unit>(a.ym.y, a.yp.z, g.sp[1]),
+                                 central<Unit>(a.zm.y, a.zp.z, g.sp[2])};
+            cc.finish(g, 0, num / (a.r.z - a.r.y), ga, gb, p, nn);
+            put(V.at[0], p, nn);
+        }
+        if (V.cut[1]) {
+            const float gb[3] = {central<Unit>(a.yp.x, a.yp.z, g.sp[0]), central<Unit>(a.r.y, of_pair(a.y2), g.sp[1]),
+                                 central<Unit>(of_pair(a.yz), of_pair(a.d), g.sp[2])};
+            cc.finish(g, 1, num / (a.yp.y - a.r.y), ga, gb, p, nn);
+            put(V.at[1], p, nn);
+        }
+        if (V.cut[2]) {
+            const float gb[3] = {central<Unit>(a.zp.x, a.zp.z, g.sp[0]), central<Unit>(of_pair(a.zy), of_pair(a.d), g.sp[1]),
+                                 central<Unit>(a.r.y, of_pair(a.z2), g.sp[2])};
+            cc.finish(g, 2, num / (a.zp.y - a.r.y), ga, gb, p, nn);
+            put(V.at[2], p, nn);
+        }
+    } else if (V.any) {
+        const float* __restrict__ v = R.row0 + ((uint32_t)q * (uint32_t)g.nx + (uint32_t)i);
 #pragma unroll
-            for (int a = grp; a < (grp ? 3 : 1); ++a) {
-                uint64_t bits = cut[a];
-                uint32_t p = a == 0 ? pos0 : (a == 1 ? pos1 : pos2);
-                if (idx + (uint32_t)__popcll(bits) <= win || idx >= wend) {
-                    idx += (uint32_t)__popcll(bits);
-                    continue;
-                }
-                while (bits && idx < wend) {
-                    const int b = __builtin_ctzll(bits);
-                    bits &= bits - 1;
-                    if (idx >= win) list[idx - win] = p << 14 | (uint32_t)a << 12 | (uint32_t)lane << 6 | (uint32_t)b;
-                    ++idx;
-                    ++p;
-                }
-                idx += (uint32_t)__popcll(bits);
-            }
-            wave_sync();
-            const uint32_t n = min((uint32_t)kEmitVertCap, gtotal - win);
-            for (uint32_t e = lane; e < n; e += 64) {
-                const uint32_t ent = list[e];
-                float pp[3], nn[3];
-                emit_vertex<Unit>(plane, g, iso, ent, j0, (int)k0, wp_log2, grp == 0, pp, nn);
-                uint64_t vid = v0 + (ent >> 14);
-                if (vmap) vid = (uint64_t)vmap[vid];
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    pts[3 * vid + c] = pp[c];
-                    nrm[3 * vid + c] = nn[c];
-                }
-            }
-            wave_sync();
+        for (int ax = 0; ax < 3; ++ax) {
+            if (!V.cut[ax]) continue;
+            float p[3], nn[3];
+            fe_edge_point<Unit>(v, g, iso, ax, i, V.j, V.k, p, nn);
+            put(V.at[ax], p, nn);
         }
     }
 }
 
-/* Vertices of the wavefront's rows through an LDS staging window. The wavefront's vertices form
- * one contiguous output range [v0, v0 + total), written kStageVerts vertices at a time: in each
- * window the lanes list their cut edges whose output position falls in it (x-edges in lane order,
- * y/z-edges word-major for rows of 16 words and more, the order in which the gathers share cache
- * lines best), compute one vertex each, and put its point and normal at the vertex's place in the
- * staging buffer; the window then goes out as consecutive dwords, every store of the wavefront
- * covering 256 contiguous bytes. Stored straight from the lanes, a wavefront's vertices land in
- * runs of a few vertices (one row's cut edges of one axis, or fewer in word-major order), and
- * cache lines at the runs' ends are written partially, several times over. */
-template <bool Unit>
-__device__ __forceinline__ void emit_rows_vertices_staged(const EmitRows& E, EmitRowsLds& S,
-                                                          const float* __restrict__ vol, const Geom& g, float iso,
-                                                          float* __restrict__ pts, float* __restrict__ nrm)
-{
-    const RowLanes& rl = E.rl;
-    const LaneWords& L = E.L;
-    const int lane = E.lane;
-    const uint64_t v0 = E.v0, vb = E.vb, eb = E.eb;
-    const int j0 = E.j0;
-    const int64_t k0 = E.k0;
-    const float* __restrict__ plane = vol + k0 * (g.nx * g.ny);
-    const uint64_t live = E.emit ? ~0ull : 0ull;
-    const uint64_t cut[3] = {(L.m[0] ^ shifted(L.m[0], L.n[0])) & eb & live,
-                             E.has_y ? ((L.m[0] ^ L.m[1]) & vb & live) : 0ull,
-                             E.has_z ? ((L.m[0] ^ L.m[2]) & vb & live) : 0ull};
-    const uint32_t c0 = __popcll(cut[0]), c1 = __popcll(cut[1]), c2 = __popcll(cut[2]);
-    // output positions (wavefront-relative) of the lane's first x-, y- and z-edge vertex: rows in
-    // order, [x][y][z] within a row, words in order within an axis
-    const uint32_t p01 = c0 | c1 << 16;
-    const uint32_t inc01 = seg_incl<OpAdd>(p01, rl.Wp, rl.w);
-    const uint32_t tot01 = (uint32_t)__shfl((int)inc01, (lane & ~(rl.Wp - 1)) + rl.Wp - 1);
-    const uint32_t ex01 = inc01 - p01;
-    const uint32_t X = tot01 & 0xFFFFu, Y = tot01 >> 16;
-    const uint32_t lane_tot = c0 + c1 + c2;
-    const uint32_t incl = wave_incl_scan_u32(lane_tot);
-    const uint32_t before_row = __shfl(incl - lane_tot, rl.q * rl.Wp);
-    const uint32_t pos[3] = {before_row + (ex01 & 0xFFFFu), before_row + X + (ex01 >> 16),
-                             before_row + X + Y + seg_excl_scan(c2, rl.Wp, rl.w)};
-    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
-    const bool word_major = rl.Wp >= 16;
-    const int wp_log2 = __builtin_ctz((unsigned)rl.Wp), rpw_log2 = 6 - wp_log2;
-    const int tl = word_major ? rl.w * rl.rpw + rl.q : lane;
-    const int from = word_major ? ((lane & (rl.rpw - 1)) << wp_log2) + (lane >> rpw_log2) : lane;
-    uint32_t* list = S.sv.list;
-    float* stage = S.sv.stage;
-    for (uint32_t w0 = 0; w0 < total; w0 += kStageVerts) {
-        const uint32_t w1 = min(w0 + (uint32_t)kStageVerts, total);
-        uint32_t n[3];
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            const uint32_t lo = max(pos[a], w0), hi = min(pos[a] + (a == 0 ? c0 : (a == 1 ? c1 : c2)), w1);
-            n[a] = hi > lo ? hi - lo : 0u;
-        }
-        // list slots: the window's x-edges [0, xtot) in lane order, then its y/z-edges
-        const uint32_t xincl = wave_incl_scan_u32(n[0]);
-        const uint32_t xtot = (uint32_t)__builtin_amdgcn_readlane((int)xincl, 63);
-        const uint32_t n12t = (uint32_t)__shfl((int)(n[1] + n[2]), from);
-        const uint32_t yzincl_t = wave_incl_scan_u32(n12t);
-        const uint32_t wn = (uint32_t)__builtin_amdgcn_readlane((int)yzincl_t, 63) + xtot;
-        uint32_t slot[3];
-        slot[0] = xincl - n[0];
-        slot[1] = xtot + (uint32_t)__shfl((int)(yzincl_t - n12t), tl);
-        slot[2] = slot[1] + n[1];
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            if (!n[a]) continue;
-            uint64_t bits = cut[a];
-            uint32_t p = pos[a], s = slot[a];
-            while (bits && p < w1) {
-                const int b = __builtin_ctzll(bits);
-                bits &= bits - 1;
-                if (p >= w0) list[s++] = (p - w0) << 14 | (uint32_t)a << 12 | (uint32_t)lane << 6 | (uint32_t)b;
-                ++p;
-            }
-        }
-        wave_sync();
-#pragma unroll
-        for (int grp = 0; grp < 2; ++grp) {
-            for (uint32_t e = (grp ? xtot : 0u) + (uint32_t)lane; e < (grp ? wn : xtot); e += 64) {
-                const uint32_t ent = list[e];
-                float pp[3], nn[3];
-                emit_vertex<Unit>(plane, g, iso, ent, j0, (int)k0, wp_log2, grp == 0, pp, nn);
-                const uint32_t at = 3 * (ent >> 14);
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    stage[at + c] = pp[c];
-                    stage[3 * kStageVerts + at + c] = nn[c];
-                }
-            }
-        }
-        wave_sync();
-        const uint32_t nf = 3 * (w1 - w0);
-        float* __restrict__ dp = pts + 3 * (v0 + w0);
-        float* __restrict__ dn = nrm + 3 * (v0 + w0);
-        for (uint32_t f = (uint32_t)lane; f < nf; f += 64) {
-            dp[f] = stage[f];
-            dn[f] = stage[3 * kStageVerts + f];
-        }
-        wave_sync();
-    }
-}
-
-/* Triangles of the wavefront's cell rows: active cells listed per lane in output order, then
- * resolved one triangle per lane. Ids are written less vbias, or through remap. */
+/* Triangles of the wavefront's cell rows: active cells listed per lane in output order, then 64 at a
+ * time one cell per lane (its case and its twelve vertex ids, into LDS), then one triangle per lane
+ * (three ids from LDS, stored at consecutive addresses). Ids are written less vbias, or through
+ * remap.
+ * A cell needs the bits b and b + 1 of four rows and the ranks of eight edge combinations at b,
+ * which one alignbit and one popcount each give from the 32-bit half that holds b; ranks of the
+ * wavefront's own rows count from its first vertex v0, those of the plane above from v2, the first
+ * vertex of the row above the wavefront's first, so that both fit 16 bits. */
 template <typename Index, bool Remap>
 __device__ __forceinline__ void emit_rows_triangles(const EmitRows& E, EmitRowsLds& S, const uint64_t* __restrict__ s_case,
-                                                    const Geom& g, const RowCounts* __restrict__ counts,
-                                                    const uint64_t* __restrict__ voff, Index* __restrict__ tris,
-                                                    uint64_t vbias, const Index* __restrict__ remap)
+                                                    Index* __restrict__ tris, uint64_t vbias,
+                                                    const Index* __restrict__ remap)
 {
-    const RowLanes& rl = E.rl;
-    const LaneWords& L = E.L;
     const int lane = E.lane;
-    const int64_t r = E.r;
-    const bool ok = E.ok, has_y = E.has_y, has_z = E.has_z;
-    const uint64_t v0 = E.v0, t0 = E.t0, vb = E.vb, eb = E.eb;
-    const bool cells = ok && E.emit && has_y && has_z;
-    const CornerWords C = corner_words(L);
-    const uint64_t act = cells ? active_cells(C, eb) : 0ull;
-    const uint32_t ncell = (uint32_t)__popcll(act);
+    const uint64_t v0 = E.v0;
+    const uint32_t ncell = (uint32_t)__popcll(E.act);
     const uint32_t cincl = wave_incl_scan_u32(ncell);
     const uint32_t ctotal = (uint32_t)__builtin_amdgcn_readlane((int)cincl, 63);
     if (ctotal == 0) return;
-    {
-        uint64_t cw[8];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) cw[q] = (L.m[q] ^ shifted(L.m[q], L.n[q])) & eb;
-        cw[4] = (L.m[0] ^ L.m[1]) & vb;
-        cw[5] = (L.m[2] ^ L.m[3]) & vb;
-        cw[6] = (L.m[0] ^ L.m[2]) & vb;
-        cw[7] = (L.m[1] ^ L.m[3]) & vb;
-        uint64_t cb[8] = {v0, v0, v0, v0, v0, v0, v0, v0};
-        if (act) {
-            const int64_t rows[4] = {r, r + 1, r + g.ny, r + g.ny + 1};
-            combo_bases(counts, voff, rows, cb);
-        }
-#pragma unroll
-        for (int q = 0; q < 8; q += 2) {
-            // two combinations per segmented scan (row totals below 2^16)
-            const uint32_t ex = seg_excl_scan((uint32_t)__popcll(cw[q]) | (uint32_t)__popcll(cw[q + 1]) << 16, rl.Wp,
-                                              rl.w);
-            S.cut[q][lane] = cw[q];
-            S.cut[q + 1][lane] = cw[q + 1];
-            S.base[q][lane] = (uint32_t)(cb[q] - v0) + (ex & 0xFFFFu);
-            S.base[q + 1][lane] = (uint32_t)(cb[q + 1] - v0) + (ex >> 16);
-        }
-    }
-    uint32_t lo[8], hi[8];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        lo[2 * q] = (uint32_t)C.m[q];
-        hi[2 * q] = (uint32_t)(C.m[q] >> 32);
-        lo[2 * q + 1] = (uint32_t)C.s[q];
-        hi[2 * q + 1] = (uint32_t)(C.s[q] >> 32);
-    }
-    // corner order v0..v7 = m0 s0 s1 m1 m2 s2 s3 m3
-    const uint32_t clo[8] = {lo[0], lo[1], lo[3], lo[2], lo[4], lo[5], lo[7], lo[6]};
-    const uint32_t chi[8] = {hi[0], hi[1], hi[3], hi[2], hi[4], hi[5], hi[7], hi[6]};
     const uint32_t cfirst = cincl - ncell;
     const uint64_t vrel = v0 - vbias;
-    uint64_t slot = t0;
+    const uint32_t dv = (uint32_t)(E.v2 - v0);
+    Index* __restrict__ out = tris + 3 * E.t0;
     for (uint32_t win = 0; win < ctotal; win += kEmitCellCap) {
-        const uint32_t wend = win + kEmitCellCap;
-        // each lane lists the positions (lane, bit) of its active cells
-        if (ncell && cfirst < wend && cfirst + ncell > win) {
-            uint32_t p = cfirst;
-            for (uint64_t a = act; a && p < wend;) {
-                const int b = __builtin_ctzll(a);
-                a &= a - 1;
-                if (p >= win) S.u.t.cells[p - win] = (uint32_t)lane | (uint32_t)b << 6;
-                ++p;
-            }
-        }
+        list_bits<kEmitCellCap>(E.act, cfirst, win, lane, S.t.cells);
         wave_sync();
         const uint32_t n = min((uint32_t)kEmitCellCap, ctotal - win);
         for (uint32_t g0 = 0; g0 < n; g0 += 64) {
-            // one cell per lane: its case from the owner lane's corner words (read across lanes)
             const uint32_t idx = g0 + (uint32_t)lane;
-            uint32_t ent = idx < n ? S.u.t.cells[idx] : 0u;
-            {
-                const int src = (int)(ent & 63), b = (int)((ent >> 6) & 63);
-                uint32_t half[8];
+            const uint32_t ent = idx < n ? (uint32_t)S.t.cells[idx] : 0u;
+            const uint32_t h2 = ent >> 5, b = ent & 31;
+            uint32_t w[4], t[4], x[4];
 #pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const uint32_t l = (uint32_t)__shfl((int)clo[q], src), h = (uint32_t)__shfl((int)chi[q], src);
-                    half[q] = b >= 32 ? h : l;
-                }
-                ent |= case_of_half(half, b & 31) << 12;
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t lo = S.words[q][h2], hi = S.words[q][h2 + 1];
+                w[q] = lo;
+                t[q] = __builtin_amdgcn_alignbit(hi, lo, b);           // bits b and b + 1 of the row, at 0 and 1
+                x[q] = lo ^ __builtin_amdgcn_alignbit(hi, lo, 1);      // cut x-edges of the half
             }
-            const uint32_t nt = idx < n ? (uint32_t)case_tri_count(s_case[ent >> 12]) : 0u;
+            const uint4 rk = S.rank[h2];
+            const uint32_t cs = (t[0] & 3) | (t[1] & 3) << 2 | (t[2] & 3) << 4 | (t[3] & 3) << 6;
+            uint64_t packed = s_case[cs];
+            const uint32_t nt = idx < n ? (uint32_t)case_tri_count(packed) : 0u;
+            const uint32_t below = bits_below(b);
+            auto cnt = [&](uint32_t bits) { return (uint32_t)__popc(bits & below); };
+            uint32_t* id = S.t.ids + kIdStride * lane;
+            id[0] = rk.x + (cnt(x[0]) | cnt(x[1]) << 16);
+            id[4] = rk.y + (cnt(x[2]) | cnt(x[3]) << 16);
+            auto pair = [&](uint32_t r16, uint32_t bits, uint32_t cut) {
+                const uint32_t at = r16 + cnt(bits);
+                return at | (at + (cut & 1)) << 16;                    // at x = i and at x = i + 1
+            };
+            id[1] = pair(rk.z & 0xFFFFu, w[0] ^ w[1], t[0] ^ t[1]);
+            id[5] = pair(rk.z >> 16, w[2] ^ w[3], t[2] ^ t[3]);
+            id[2] = pair(rk.w & 0xFFFFu, w[0] ^ w[2], t[0] ^ t[2]);
+            id[3] = pair(rk.w >> 16, w[1] ^ w[3], t[1] ^ t[3]);
             const uint32_t tincl = wave_incl_scan_u32(nt);
             const uint32_t ttot = (uint32_t)__builtin_amdgcn_readlane((int)tincl, 63);
-            for (uint32_t tt = 0; tt < nt; ++tt) S.u.t.map[tincl - nt + tt] = ent | tt << 20;
+            // the group's triangles in output order: byte offset of the cell's ids | its 3 slots << 12
+            uint32_t* m = S.t.map + (tincl - nt);
+            for (uint32_t tt = 0; tt < nt; ++tt, packed >>= 12)
+                m[tt] = (uint32_t)(4 * kIdStride * lane) | (uint32_t)packed << 12;
             wave_sync();
             for (uint32_t e = lane; e < ttot; e += 64) {
-                const uint32_t me = S.u.t.map[e];
-                const int owner = (int)(me & 63);
-                const int b = (int)((me >> 6) & 63);
-                const uint64_t packed = s_case[(me >> 12) & 0xFF];
-                const int tt = (int)(me >> 20);
-                uint32_t id[3];
+                const uint32_t me = S.t.map[e];
+                const uint32_t at = me & 0xFFFu;
+                uint64_t id3[3];
 #pragma unroll
                 for (int s = 0; s < 3; ++s) {
-                    const int ed = case_edge(packed, 3 * tt + s);
-                    const int q = combo_of_edge(ed);
-                    const int p = b + edge_dx(ed);
-                    const uint64_t cwq = S.cut[q][owner];
-                    const uint64_t below = p == 64 ? cwq : (cwq & ((1ull << p) - 1ull));
-                    id[s] = S.base[q][owner] + (uint32_t)__popcll(below);
+                    const uint32_t slot = __builtin_amdgcn_ubfe(me, 12 + 4 * s, 4);
+                    const uint32_t up = (uint32_t)__builtin_amdgcn_sbfe((int)me, 15 + 4 * s, 1);   // slots 8 .. 11
+                    uint16_t rel;
+                    __builtin_memcpy(&rel, reinterpret_cast<const char*>(S.t.ids) + (at + 2 * slot), 2);
+                    id3[s] = vrel + ((uint32_t)rel + (up & dv));
                 }
                 if (Remap)
-                    store_tri<Index>(tris, slot + e, remap[vrel + id[0]], remap[vrel + id[1]], remap[vrel + id[2]]);
+                    store_tri<Index>(out, e, remap[id3[0]], remap[id3[1]], remap[id3[2]]);
                 else
-                    store_tri<Index>(tris, slot + e, vrel + id[0], vrel + id[1], vrel + id[2]);
+                    store_tri<Index>(out, e, id3[0], id3[1], id3[2]);
             }
-            slot += ttot;
+            out += 3 * ttot;
             wave_sync();
         }
     }
 }
 
-/* Lane-row block blk. s_case holds kCaseEdges; vertex ids are written less vbias (the first
+/* The wavefront's vertices and triangles. The first step's voxels are requested before the
+ * triangles, which work from LDS (1024^3: 1.44 ms against 1.48 ms with the vertices first). */
+template <typename Index, bool Unit, bool Map>
+__device__ __forceinline__ void emit_rows_both(const EmitRows& E, EmitRowsLds& S, const uint64_t* __restrict__ s_case,
+                                               const float* __restrict__ vol, const Geom& g, float iso,
+                                               float* __restrict__ pts, float* __restrict__ nrm,
+                                               Index* __restrict__ tris, uint64_t vbias,
+                                               const Index* __restrict__ vmap)
+{
+    const VertexRows R = vertex_rows(E, vol, g);
+    const uint32_t lane = (uint32_t)E.lane;
+    VertexStep V;
+    uint32_t n = min((uint32_t)kOriginCap, R.n);
+    list_bits<kOriginCap>(E.origins, R.first, 0, E.lane, S.origins);
+    wave_sync();
+    vertex_load(V, E, S, R, g, lane, n);
+    wave_sync();
+    emit_rows_triangles<Index, Map>(E, S, s_case, tris, vbias, vmap);
+    for (uint32_t win = 0;;) {
+        for (uint32_t e0 = 0; e0 < n; e0 += 64) {
+            vertex_store<Unit, Map, Index>(V, E, R, g, iso, pts, nrm, vmap);
+            if (e0 + 64 < n) vertex_load(V, E, S, R, g, e0 + 64 + lane, n);
+        }
+        win += kOriginCap;
+        if (win >= R.n) break;
+        n = min((uint32_t)kOriginCap, R.n - win);
+        wave_sync();
+        list_bits<kOriginCap>(E.origins, R.first, win, E.lane, S.origins);
+        wave_sync();
+        vertex_load(V, E, S, R, g, lane, n);
+    }
+}
+
+/* Lane-row block blk. s_case holds kCaseSlots; vertex ids are written less vbias (the first
  * vertex of this volume's output when several volumes share one buffer). With Remap, only the
  * triangles are written, each Flying Edges vertex id replaced by remap[id]. */
 template <typename Index, bool Unit, bool Remap = false>
@@ -873,9 +931,12 @@ __device__ __forceinline__ void fe_emit_rows_block(const uint64_t* __restrict__ 
                                                    uint64_t vbias, int64_t blk, const Index* __restrict__ remap = nullptr)
 {
     EmitRows E;
-    if (!emit_rows_setup(E, mask, g, counts, voff, toff, blk)) return;
-    if (!Remap) emit_rows_vertices_staged<Unit>(E, s_w[E.wv], vol, g, iso, pts, nrm);
-    emit_rows_triangles<Index, Remap>(E, s_w[E.wv], s_case, g, counts, voff, tris, vbias, remap);
+    if (!emit_rows_setup(E, s_w, mask, g, counts, voff, toff, blk)) return;
+    EmitRowsLds& S = s_w[E.wv];
+    if (Remap)
+        emit_rows_triangles<Index, true>(E, S, s_case, tris, vbias, remap);
+    else
+        emit_rows_both<Index, Unit, false>(E, S, s_case, vol, g, iso, pts, nrm, tris, vbias, remap);
 }
 
 /* The order in which pass 4's blocks take the rows, across the 8 XCDs. The hardware hands blocks
@@ -946,7 +1007,7 @@ __global__ __launch_bounds__(256) void k_fe_emit_rows(const float* __restrict__ 
     if (need && !output_fits<Index>(need, cap_v, cap_t)) return;
     __shared__ uint64_t s_case[256];
     __shared__ EmitRowsLds s_w[4];
-    s_case[threadIdx.x] = kCaseEdges[threadIdx.x];
+    s_case[threadIdx.x] = kCaseSlots.v[threadIdx.x];
     __syncthreads();
     const int64_t blk = emit_block_order(blockIdx.x, gridDim.x, g);
     fe_emit_rows_block<Index, Unit>(s_case, s_w, vol, mask, g, iso, counts, voff, toff, pts, nrm, tris, vbias, blk);
@@ -966,13 +1027,12 @@ __global__ __launch_bounds__(256) void k_mc_emit_rows(const float* __restrict__ 
 {
     __shared__ uint64_t s_case[256];
     __shared__ EmitRowsLds s_w[4];
-    s_case[threadIdx.x] = kCaseEdges[threadIdx.x];
+    s_case[threadIdx.x] = kCaseSlots.v[threadIdx.x];
     __syncthreads();
     const int64_t blk = emit_block_order(blockIdx.x, gridDim.x, g);
     EmitRows E;
-    if (!emit_rows_setup(E, mask, g, counts, voff, toff, blk)) return;
-    emit_rows_vertices<true, Index>(E, s_w[E.wv].u.vlist, vol, g, iso, pts, nrm, fe_to_mc);
-    emit_rows_triangles<Index, true>(E, s_w[E.wv], s_case, g, counts, voff, tris, 0, fe_to_mc);
+    if (!emit_rows_setup(E, s_w, mask, g, counts, voff, toff, blk)) return;
+    emit_rows_both<Index, true, true>(E, s_w[E.wv], s_case, vol, g, iso, pts, nrm, tris, 0, fe_to_mc);
 }
 
 /* Marching Cubes triangles: the Flying Edges triangle stream through the id map. */
@@ -986,7 +1046,7 @@ __global__ __launch_bounds__(256) void k_mc_triangles_rows(const uint64_t* __res
 {
     __shared__ uint64_t s_case[256];
     __shared__ EmitRowsLds s_w[4];
-    s_case[threadIdx.x] = kCaseEdges[threadIdx.x];
+    s_case[threadIdx.x] = kCaseSlots.v[threadIdx.x];
     __syncthreads();
     const int64_t blk = emit_block_order(blockIdx.x, gridDim.x, g);
     fe_emit_rows_block<Index, true, true>(s_case, s_w, nullptr, mask, g, 0.0f, counts, voff, toff, nullptr, nullptr,

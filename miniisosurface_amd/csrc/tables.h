@@ -106,6 +106,33 @@ static constexpr uint8_t kEdgeDx[12]   = {0, 1, 0, 0, 0, 1, 0, 0, 0, 1, 0, 1};
 static constexpr uint8_t kEdgeDy[12]   = {0, 0, 1, 0, 0, 0, 1, 0, 0, 0, 1, 1};
 static constexpr uint8_t kEdgeDz[12]   = {0, 0, 0, 0, 1, 1, 1, 1, 0, 0, 0, 0};
 
+/* The order in which pass 4 of the row kernels keeps a cell's twelve vertex ids: slots 0 .. 7 are
+ * the edges of grid plane k and the z-edges above it, slots 8 .. 11 the edges of plane k + 1; a y-
+ * or z-edge at x = i + 1 follows the one at x = i (rank plus that one's cut bit). */
+//                                         edge: 0  1  2  3  4  5   6  7   8  9  10 11
+static constexpr uint8_t kEdgeSlot[12] = {0, 3, 1, 2, 8, 11, 9, 10, 4, 5, 6, 7};
+
+/* kCaseEdges with slots in the place of edges, indexed by the corner bits as the mask words give
+ * them: bits 2 q and 2 q + 1 are x = i and x = i + 1 of row q = (j,k) (j+1,k) (j,k+1) (j+1,k+1). The
+ * corner numbering has rows 1 and 3 the other way round (v2, v3 and v6, v7). */
+struct CaseSlots {
+    uint64_t v[256];
+};
+constexpr CaseSlots make_case_slots()
+{
+    CaseSlots t{};
+    for (int c = 0; c < 256; ++c) {
+        const uint64_t e = kCaseEdges[(c & 0x33) | (c & 0x44) << 1 | (c & 0x88) >> 1];
+        const int ns = 3 * (int)(e >> 60);
+        uint64_t v = e;
+        for (int s = 0; s < ns; ++s)
+            v = (v & ~(0xFull << (4 * s))) | (uint64_t)kEdgeSlot[(e >> (4 * s)) & 0xF] << (4 * s);
+        t.v[c] = v;
+    }
+    return t;
+}
+static constexpr CaseSlots kCaseSlots = make_case_slots();
+
 MISO_HD constexpr int case_tri_count(uint64_t packed) { return (int)(packed >> 60); }
 
 MISO_HD constexpr int case_edge(uint64_t packed, int slot) { return (int)((packed >> (4 * slot)) & 0xF); }
