@@ -205,7 +205,8 @@ struct RowState {
 
     int launch_classify(float iso)
     {
-        hipLaunchKernelGGL(k_fe_classify, dim3(row_blocks()), dim3(256), 0, stream, d_vol, g, iso, d_mask);
+        hipLaunchKernelGGL(k_fe_classify, dim3(row_blocks()), dim3(256), 0, stream, d_vol, g, iso, d_mask,
+                           keep_from_row(g));
         HIPCALL(hipGetLastError());
         return MISO_OK;
     }

@@ -114,7 +114,7 @@ __device__ __forceinline__ void batch_classify_item(const BatchJob* __restrict__
     if (J.g.W <= 4)
         fe_classify_short_rows_n(job_volume(J), J.g, n, sink, blk);
     else
-        fe_classify_block_n(job_volume(J), J.g, n, sink, blk);
+        fe_classify_block_n(job_volume(J), J.g, n, sink, blk, INT64_MAX);
 }
 
 __global__ __launch_bounds__(256) void k_batch_classify(const BatchJob* __restrict__ jobs,

@@ -29,16 +29,26 @@ constexpr uint64_t kFlagPre = 2ull << 62;
 constexpr uint64_t kValMask = (1ull << 62) - 1;
 
 /* ------------------------------------------------------------------ pass 1a: sign mask */
+/* Voxels at the end of a volume that pass 1 leaves in the 256 MB cache beside the HBM, where pass 4,
+ * which takes the rows from the end (emit_block), finds them: 128 MB. Streamed past the caches as the
+ * rest is, pass 4 reads them from HBM again: 512^3 gyroid 496 us against 475 us, 333x257x190 144
+ * against 131, 1024^3 2.284 ms against 2.267. 256 MB: 482 us and 2.279 ms (pass 1 slows down by more
+ * than pass 4 gains); every voxel, and pass 4 from the start: 515 us and 2.340 ms. */
+constexpr int64_t kKeepVoxels = int64_t(1) << 25;
+
+inline int64_t keep_from_row(const Geom& g) { return g.ny * g.nz - (kKeepVoxels + g.nx - 1) / g.nx; }
+
 /* Rows 4 blk .. 4 blk + 3, one per wavefront. Each lane loads 4 consecutive voxels (one 16-byte
  * non-temporal load, so a wavefront step covers 256 voxels = 4 mask words); its 4 sign bits are placed at
  * bit 4 * (lane % 16) and OR-reduced over each 16-lane row with DPP, so lane 16 t + 15 ends up
- * holding mask word t of the step. Voxels past nx read as below the isovalue. Rows of at most
- * 256 voxels take one voxel per lane and __ballot instead (fewer instructions per short row).
+ * holding mask word t of the step. Rows from keep_row on are read with plain loads instead, so that
+ * they stay in the caches for pass 4 (kKeepVoxels). Voxels past nx read as below the isovalue. Rows
+ * of at most 256 voxels take one voxel per lane and __ballot instead (fewer instructions per short row).
  * The voxels are loaded once and classified against n isovalues of the same volume:
  * sink(t, iso, mask) names isovalue t and the mask array it writes (n = 1 for one extraction). */
 template <class Sink>
 __device__ __forceinline__ void fe_classify_block_n(const float* __restrict__ vol, const Geom& g, int n, Sink sink,
-                                                    int64_t blk)
+                                                    int64_t blk, int64_t keep_row)
 {
     const int lane = lane_id();
     const int64_t r = blk * kRowsPerBlock + (threadIdx.x >> 6);
@@ -80,7 +90,7 @@ __device__ __forceinline__ void fe_classify_block_n(const float* __restrict__ vo
             if (c0 + 256 * u >= g.nx) continue;    // wavefront-uniform: short rows skip whole steps
             const int64_t i = c0 + 256 * u + 4 * lane;
             if (i + 4 <= g.nx) {
-                const Vox4 q = load_vox4_stream(row + i);
+                const Vox4 q = r < keep_row ? load_vox4_stream(row + i) : load_vox<Vox4>(row + i);
                 v[u][0] = q.x; v[u][1] = q.y; v[u][2] = q.z; v[u][3] = q.w;
                 in[u] = 15u;
             } else {
@@ -164,15 +174,15 @@ __device__ __forceinline__ void fe_classify_short_rows_n(const float* __restrict
 }
 
 __device__ __forceinline__ void fe_classify_block(const float* __restrict__ vol, const Geom& g, float iso,
-                                                  uint64_t* __restrict__ mask, int64_t blk)
+                                                  uint64_t* __restrict__ mask, int64_t blk, int64_t keep_row)
 {
-    fe_classify_block_n(vol, g, 1, [&](int, float& is, uint64_t*& m) { is = iso; m = mask; }, blk);
+    fe_classify_block_n(vol, g, 1, [&](int, float& is, uint64_t*& m) { is = iso; m = mask; }, blk, keep_row);
 }
 
 __global__ __launch_bounds__(256) void k_fe_classify(const float* __restrict__ vol, Geom g, float iso,
-                                                     uint64_t* __restrict__ mask)
+                                                     uint64_t* __restrict__ mask, int64_t keep_row)
 {
-    fe_classify_block(vol, g, iso, mask, blockIdx.x);
+    fe_classify_block(vol, g, iso, mask, blockIdx.x, keep_row);
 }
 
 /* ------------------------------------------------------------------ pass 1b + 2: counts */

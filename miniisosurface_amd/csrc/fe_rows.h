@@ -991,6 +991,13 @@ __device__ __forceinline__ int64_t emit_block_order(int64_t b, int64_t n, const 
     return apply_block_order(g.bo, (uint32_t)b);
 }
 
+/* The row block of block b of a single-volume pass 4 of n blocks: the order above from the end, where
+ * the voxels lie that pass 1 read last (kKeepVoxels). */
+__device__ __forceinline__ int64_t emit_block(int64_t b, int64_t n, const Geom& g)
+{
+    return n - 1 - emit_block_order(b, n, g);
+}
+
 template <typename Index, bool Unit>
 __global__ __launch_bounds__(256) void k_fe_emit_rows(const float* __restrict__ vol,
                                                       const uint64_t* __restrict__ mask, Geom g, float iso,
@@ -1009,7 +1016,7 @@ __global__ __launch_bounds__(256) void k_fe_emit_rows(const float* __restrict__ 
     __shared__ EmitRowsLds s_w[4];
     s_case[threadIdx.x] = kCaseSlots.v[threadIdx.x];
     __syncthreads();
-    const int64_t blk = emit_block_order(blockIdx.x, gridDim.x, g);
+    const int64_t blk = emit_block(blockIdx.x, gridDim.x, g);
     fe_emit_rows_block<Index, Unit>(s_case, s_w, vol, mask, g, iso, counts, voff, toff, pts, nrm, tris, vbias, blk);
 }
 
@@ -1029,7 +1036,7 @@ __global__ __launch_bounds__(256) void k_mc_emit_rows(const float* __restrict__ 
     __shared__ EmitRowsLds s_w[4];
     s_case[threadIdx.x] = kCaseSlots.v[threadIdx.x];
     __syncthreads();
-    const int64_t blk = emit_block_order(blockIdx.x, gridDim.x, g);
+    const int64_t blk = emit_block(blockIdx.x, gridDim.x, g);
     EmitRows E;
     if (!emit_rows_setup(E, s_w, mask, g, counts, voff, toff, blk)) return;
     emit_rows_both<Index, true, true>(E, s_w[E.wv], s_case, vol, g, iso, pts, nrm, tris, 0, fe_to_mc);
@@ -1048,7 +1055,7 @@ __global__ __launch_bounds__(256) void k_mc_triangles_rows(const uint64_t* __res
     __shared__ EmitRowsLds s_w[4];
     s_case[threadIdx.x] = kCaseSlots.v[threadIdx.x];
     __syncthreads();
-    const int64_t blk = emit_block_order(blockIdx.x, gridDim.x, g);
+    const int64_t blk = emit_block(blockIdx.x, gridDim.x, g);
     fe_emit_rows_block<Index, true, true>(s_case, s_w, nullptr, mask, g, 0.0f, counts, voff, toff, nullptr, nullptr,
                                           tris, 0, blk, fe_to_mc);
 }
