@@ -20,14 +20,15 @@ struct miso_batch {
     BatchJob* d_jobs = nullptr;
     int64_t* d_cls_prefix = nullptr;
     int64_t* d_lane_prefix = nullptr;
-    int64_t R = 0, mask_words = 0, ntiles = 0;
+    int64_t R = 0, mask_words = 0;
+    ScanPlan scan{10, 0};
     uint64_t* d_mask = nullptr;
     RowCounts* d_counts = nullptr;
     RowTrim* d_trims = nullptr;
     uint64_t* d_voff = nullptr;
     uint64_t* d_toff = nullptr;
     uint64_t* d_state = nullptr;      // [0..2] queue tickets, [3] totals V, [4] totals T, [5..12] the XCD
-                                      // queues' tickets of pass 4, [13..] scan state
+                                      // queues' tickets of pass 4, [13..] scan tile sums
     int64_t state_words = 0;
     uint64_t* d_jobout = nullptr;     // 4 per job: first vertex, first triangle, vertices, triangles
     uint64_t* h_jobout = nullptr;     // pinned copy, then the two totals
@@ -53,7 +54,7 @@ struct miso_batch {
     uint64_t* tickets() { return d_state; }
     uint64_t* totals() { return d_state + 3; }
     uint64_t* xcd_tickets() { return d_state + 5; }
-    uint64_t* scan_state() { return d_state + 13; }
+    uint64_t* scan_sums() { return d_state + 13; }
 };
 
 namespace {
@@ -102,9 +103,10 @@ int enqueue_scan(miso_batch* b)
                        b->ngroups, ncls, b->chunk, b->d_mask, b->tickets() + 0);
     hipLaunchKernelGGL(k_batch_count, dim3(batch_grid(b, nlane)), dim3(256), 0, b->stream, (const BatchJob*)b->d_jobs,
                        (const int64_t*)b->d_lane_prefix, b->njobs, nlane, b->chunk, (const uint64_t*)b->d_mask,
-                       b->d_counts, b->d_trims, b->tickets() + 1);
-    hipLaunchKernelGGL(k_fe_scan, dim3((unsigned)b->ntiles), dim3(256), 0, b->stream, (const RowCounts*)b->d_counts,
-                       b->R, b->d_voff, b->d_toff, b->scan_state(), b->ntiles, b->totals());
+                       b->d_counts, b->d_trims, b->scan_sums(), b->scan.shift, b->tickets() + 1);
+    hipLaunchKernelGGL(k_fe_scan<uint32_t>, dim3((unsigned)b->scan.ntiles), dim3(256), 0, b->stream,
+                       (const RowCounts*)b->d_counts, b->R, b->d_voff, b->d_toff, (const uint64_t*)b->scan_sums(),
+                       b->scan.shift, b->scan.ntiles, b->totals(), (uint64_t*)nullptr, ScanMore());
     hipLaunchKernelGGL(k_batch_job_counts, dim3((unsigned)((b->njobs + 255) / 256)), dim3(256), 0, b->stream,
                        (const BatchJob*)b->d_jobs, b->njobs, b->R, (const uint64_t*)b->d_voff,
                        (const uint64_t*)b->d_toff, (const uint64_t*)b->totals(), b->d_jobout);
@@ -307,8 +309,8 @@ int batch_set_jobs(miso_batch* b, const miso_volume* vols, const float* isovals,
     b->lane_prefix.swap(lane);
     b->R = R;
     b->mask_words = mw;
-    b->ntiles = (R + kScanTile - 1) / kScanTile;
-    b->state_words = 13 + 1 + 2 * b->ntiles;
+    b->scan = plan_scan(R);
+    b->state_words = 13 + kTileSums * b->scan.ntiles;
     // pass 4's XCD queues: XCD x owns the dispatch indices 8 t + x of each job's row blocks
     b->xcd_prefix.assign(8 * (size_t)(njobs + 1), 0);
     for (int x = 0; x < 8; ++x)
@@ -372,12 +374,13 @@ int enqueue_fused(miso_batch* b)
     const int64_t* xprefix = xcd ? b->d_xcd_prefix : nullptr;
     int ngroups = b->ngroups, njobs = b->njobs, chunk = b->chunk;
     int64_t ncls = b->cls_prefix.back(), nlane = b->lane_prefix.back();
-    int64_t R = b->R, ntiles = b->ntiles;
+    int64_t R = b->R, ntiles = b->scan.ntiles;
+    int shift = b->scan.shift;
     uint64_t cap_v = b->cap_v, cap_t = b->cap_t;
     void* args[] = {&jobs,      &group_job, &cls_prefix, &ngroups,     &ncls,  &lane_prefix, &njobs,
                     &nlane,     &chunk,     &b->d_mask,  &b->d_counts, &b->d_trims, &b->d_voff, &b->d_toff,
-                    &b->d_state, &R,        &ntiles,     &b->d_jobout, &cap_v, &cap_t,     &b->d_pts,
-                    &b->d_nrm,  &b->d_tris, &xprefix};
+                    &b->d_state, &R,        &shift,      &ntiles,      &b->d_jobout, &cap_v, &cap_t,
+                    &b->d_pts,  &b->d_nrm,  &b->d_tris,  &xprefix};
     hipLaunchKernelGGL(k_batch_zero, dim3((unsigned)std::min<int64_t>(1024, (b->state_words + 255) / 256)), dim3(256),
                        0, b->stream, b->d_state, b->state_words);
     HIPCALL(hipLaunchCooperativeKernel((const void*)k_batch_fused, dim3((unsigned)grid), dim3(256), args, 0,

@@ -113,9 +113,9 @@ struct RowState {
     RowTrim* d_trims = nullptr;
     uint64_t* d_voff = nullptr;
     uint64_t* d_toff = nullptr;
-    uint64_t* d_scan = nullptr;
-    int64_t ntiles = 0;
-    uint64_t* d_totals = nullptr;
+    uint64_t* d_sums = nullptr;     // the scan's tile sums
+    ScanPlan scan{10, 0};
+    uint64_t* d_totals = nullptr;   // V, T; for Marching Cubes' edge order then the x, y and z totals
     uint64_t* h_totals = nullptr;   // pinned
 
     int init(const miso_volume* v, void* user_stream)
@@ -142,15 +142,15 @@ struct RowState {
         h_totals[0] = h_totals[1] = 0;
         if (!has_cells(g)) return MISO_OK;
         const int64_t R = g.ny * g.nz;
-        ntiles = (R + kScanTile - 1) / kScanTile;
+        scan = plan_scan(R);
         int rc = 0;
         if ((rc = dev_alloc(&d_mask, (size_t)(R * g.W)))) return rc;
         if ((rc = dev_alloc(&d_counts, (size_t)R))) return rc;
         if ((rc = dev_alloc(&d_trims, (size_t)R))) return rc;
         if ((rc = dev_alloc(&d_voff, (size_t)R))) return rc;
         if ((rc = dev_alloc(&d_toff, (size_t)R))) return rc;
-        if ((rc = dev_alloc(&d_scan, (size_t)(1 + 2 * ntiles)))) return rc;
-        if ((rc = dev_alloc(&d_totals, 2))) return rc;
+        if ((rc = dev_alloc(&d_sums, (size_t)scan.sum_words()))) return rc;
+        if ((rc = dev_alloc(&d_totals, 5))) return rc;
         return MISO_OK;
     }
 
@@ -164,7 +164,7 @@ struct RowState {
         dev_free(d_trims);
         dev_free(d_voff);
         dev_free(d_toff);
-        dev_free(d_scan);
+        dev_free(d_sums);
         dev_free(d_totals);
         if (h_totals) (void)hipHostFree(h_totals);
         h_totals = nullptr;
@@ -206,7 +206,7 @@ struct RowState {
     int launch_classify(float iso)
     {
         hipLaunchKernelGGL(k_fe_classify, dim3(row_blocks()), dim3(256), 0, stream, d_vol, g, iso, d_mask,
-                           keep_from_row(g));
+                           keep_from_row(g), d_sums, kTileSums * scan.ntiles);
         HIPCALL(hipGetLastError());
         return MISO_OK;
     }
@@ -215,20 +215,26 @@ struct RowState {
     {
         if (lane_rows())
             hipLaunchKernelGGL(k_fe_count_rows, dim3(lane_row_blocks()), dim3(256), 0, stream,
-                               (const uint64_t*)d_mask, g, d_counts, d_trims, d_scan, (int64_t)(1 + 2 * ntiles));
+                               (const uint64_t*)d_mask, g, d_counts, d_trims, d_sums, scan.shift);
         else
             hipLaunchKernelGGL(k_fe_count, dim3(row_blocks()), dim3(256), 0, stream, (const uint64_t*)d_mask, g,
-                               d_counts, d_trims, d_scan, (int64_t)(1 + 2 * ntiles));
+                               d_counts, d_trims, d_sums, scan.shift);
         HIPCALL(hipGetLastError());
         return MISO_OK;
     }
 
-    int launch_scan()
+    /* pass 3; the totals reach h_totals (if there is one) with the kernel's own writes */
+    int launch_scan(const ScanMore& more = ScanMore())
     {
-        hipLaunchKernelGGL(k_fe_scan, dim3((unsigned)ntiles), dim3(256), 0, stream, (const RowCounts*)d_counts,
-                           g.ny * g.nz, d_voff, d_toff, d_scan, ntiles, d_totals);
+        if (scan_is_wide(g.nx))
+            hipLaunchKernelGGL(k_fe_scan<uint64_t>, dim3((unsigned)scan.ntiles), dim3(256), 0, stream,
+                               (const RowCounts*)d_counts, g.ny * g.nz, d_voff, d_toff, (const uint64_t*)d_sums,
+                               scan.shift, scan.ntiles, d_totals, h_totals, more);
+        else
+            hipLaunchKernelGGL(k_fe_scan<uint32_t>, dim3((unsigned)scan.ntiles), dim3(256), 0, stream,
+                               (const RowCounts*)d_counts, g.ny * g.nz, d_voff, d_toff, (const uint64_t*)d_sums,
+                               scan.shift, scan.ntiles, d_totals, h_totals, more);
         HIPCALL(hipGetLastError());
-        HIPCALL(hipMemcpyAsync(h_totals, d_totals, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, stream));
         return MISO_OK;
     }
 };
@@ -237,75 +243,61 @@ struct RowState {
 struct McState {
     uint32_t* d_owned = nullptr;     // owned cut edges per cell row (grid-row indexed)
     uint64_t* d_moff = nullptr;      // Marching Cubes vertex offset per cell row
-    uint64_t* d_scan = nullptr;
-    uint64_t* d_total = nullptr;
-    int64_t ntiles = 0;
     void* d_map = nullptr;           // Flying Edges vertex id -> Marching Cubes vertex id
     uint64_t map_bytes = 0;
     int order = MISO_MC_ORDER_FIRST_VISIT;
     uint64_t* d_xyz = nullptr;       // edge order: per-row exclusive scans of the x, y, z counts
-    uint64_t* d_axstate = nullptr;   // their three scan states, then the three totals
 
     int init(const Geom& g)
     {
         const int64_t R = g.ny * g.nz;
-        ntiles = (R + kScanTile - 1) / kScanTile;
-        int rc = 0;
-        if ((rc = dev_alloc(&d_owned, (size_t)R))) return rc;
-        if ((rc = dev_alloc(&d_moff, (size_t)R))) return rc;
-        if ((rc = dev_alloc(&d_scan, (size_t)(1 + ntiles)))) return rc;
-        if ((rc = dev_alloc(&d_total, 1))) return rc;
-        return MISO_OK;
+        if (int rc = dev_alloc(&d_owned, (size_t)R)) return rc;
+        return dev_alloc(&d_moff, (size_t)R);
     }
 
-    /* the edge-order buffers, allocated on first use */
+    /* the edge-order buffer, allocated on first use */
     int init_edge_order(const Geom& g)
     {
-        if (d_xyz) return MISO_OK;
-        const int64_t R = g.ny * g.nz;
-        if (int rc = dev_alloc(&d_xyz, (size_t)(3 * R))) return rc;
-        return dev_alloc(&d_axstate, (size_t)(3 * (1 + ntiles) + 3));
+        return d_xyz ? MISO_OK : dev_alloc(&d_xyz, (size_t)(3 * g.ny * g.nz));
     }
 
     void release()
     {
         dev_free(d_owned);
         dev_free(d_moff);
-        dev_free(d_scan);
-        dev_free(d_total);
         dev_free(d_xyz);
-        dev_free(d_axstate);
         if (d_map) (void)hipFree(d_map);
         d_map = nullptr;
     }
 
-    /* first-visit order with the row-lane kernels: the owned-edge counts come with pass 2
-     * (k_fe_mc_count_rows), launched by launch_fe_count */
-    bool fused_count(const RowState& s) const { return order != MISO_MC_ORDER_EDGE && s.lane_rows(); }
-
-    /* pass 2 of the Flying Edges row state, with the owned-edge counts where fused_count */
+    /* pass 2 of the Flying Edges row state, in first-visit order with the owned-edge counts (with
+     * the row-lane kernels in the same pass over the mask words) */
     int launch_fe_count(RowState& s)
     {
-        if (!fused_count(s)) return s.launch_count();
-        hipLaunchKernelGGL(k_fe_mc_count_rows, dim3(s.lane_row_blocks()), dim3(256), 0, s.stream,
-                           (const uint64_t*)s.d_mask, s.g, s.d_counts, s.d_trims, s.d_scan,
-                           (int64_t)(1 + 2 * s.ntiles), d_owned, d_scan, (int64_t)(1 + ntiles));
+        if (order == MISO_MC_ORDER_EDGE) return s.launch_count();   // no first-visit offsets needed
+        if (!s.lane_rows()) {
+            if (int rc = s.launch_count()) return rc;
+            hipLaunchKernelGGL(k_mc_count, dim3(s.row_blocks()), dim3(256), 0, s.stream, (const uint64_t*)s.d_mask,
+                               s.g, (const RowCounts*)s.d_counts, d_owned, s.d_sums, s.scan.shift);
+        } else {
+            hipLaunchKernelGGL(k_fe_mc_count_rows, dim3(s.lane_row_blocks()), dim3(256), 0, s.stream,
+                               (const uint64_t*)s.d_mask, s.g, s.d_counts, s.d_trims, s.d_sums, s.scan.shift, d_owned);
+        }
         HIPCALL(hipGetLastError());
         return MISO_OK;
     }
 
-    int launch_count(RowState& s)
+    /* pass 3 with this order's offsets */
+    int launch_scan(RowState& s)
     {
-        if (order == MISO_MC_ORDER_EDGE) return MISO_OK;   // no first-visit offsets needed
-        if (!fused_count(s)) {
-            hipLaunchKernelGGL(k_mc_count, dim3(s.row_blocks()), dim3(256), 0, s.stream, (const uint64_t*)s.d_mask,
-                               s.g, (const RowCounts*)s.d_counts, d_owned, d_scan, (int64_t)(1 + ntiles));
-            HIPCALL(hipGetLastError());
+        ScanMore more;
+        if (order == MISO_MC_ORDER_EDGE) {
+            more.xyz = d_xyz;
+        } else {
+            more.owned = d_owned;
+            more.moff = d_moff;
         }
-        hipLaunchKernelGGL(k_scan_u32, dim3((unsigned)ntiles), dim3(256), 0, s.stream, (const uint32_t*)d_owned,
-                           s.g.ny * s.g.nz, d_moff, d_scan, ntiles, d_total);
-        HIPCALL(hipGetLastError());
-        return MISO_OK;
+        return s.launch_scan(more);
     }
 
     template <typename Index>
@@ -321,18 +313,12 @@ struct McState {
             map_bytes = need;
         }
         if (order == MISO_MC_ORDER_EDGE) {
-            // vertices sorted by global edge id: the permutation from the three axis scans,
+            // vertices sorted by global edge id: the permutation from pass 3's axis scans,
             // then owners write at perm[FE id]; triangles through the same permutation
             const int64_t R = s.g.ny * s.g.nz;
-            const int64_t sw = 1 + ntiles;
-            hipLaunchKernelGGL(k_batch_zero, dim3(64), dim3(256), 0, s.stream, d_axstate, 3 * sw + 3);
-            for (int a = 0; a < 3; ++a)
-                hipLaunchKernelGGL(k_scan_u32, dim3((unsigned)ntiles), dim3(256), 0, s.stream,
-                                   (const uint32_t*)s.d_counts + a, R, d_xyz + a * R, d_axstate + a * sw, ntiles,
-                                   d_axstate + 3 * sw + a, (int64_t)4);
             hipLaunchKernelGGL(k_edge_order_perm<Index>, dim3((unsigned)((R + 15) / 16)), dim3(256), 0, s.stream,
                                (const RowCounts*)s.d_counts, (const uint64_t*)s.d_voff, (const uint64_t*)d_xyz,
-                               (const uint64_t*)(d_axstate + 3 * sw), R, (Index*)d_map);
+                               (const uint64_t*)(s.d_totals + 2), R, (Index*)d_map);
             const uint64_t* no_moff = nullptr;
             if (s.lane_rows() && s.unit_geometry()) {
                 // Flying Edges pass 4 through the permutation
@@ -824,18 +810,6 @@ struct miso_fe_slabs {
 
 namespace {
 
-/* Rows below lo belong to the previous slab: zeroed, so the slab's offsets start at 0. Rows from
- * hi on keep their vertex counts (the slab's last cell row names those vertices) but their cells
- * belong to the next slab: their triangle counts are zeroed. */
-__global__ __launch_bounds__(256) void k_slab_trim_counts(RowCounts* __restrict__ counts, int64_t R, int64_t lo,
-                                                          int64_t hi)
-{
-    for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < R; r += (int64_t)gridDim.x * 256) {
-        if (r < lo) counts[r] = RowCounts{0u, 0u, 0u, 0u};
-        else if (r >= hi) counts[r].t = 0u;
-    }
-}
-
 int64_t slab_data_lo(int64_t k0) { return k0 > 0 ? k0 - 1 : 0; }
 int64_t slab_data_hi(const miso_fe_slabs* h, int64_t k1) { return std::min<int64_t>(k1 + 2, h->full.nz); }
 
@@ -866,12 +840,9 @@ int slab_launch_counts(miso_fe_slabs* h, int p, int64_t k0)
     g.bo = plan_block_order(g.ny, g.nz, g.W);
     s.g = g;
     const int64_t R = g.ny * g.nz;
-    s.ntiles = (R + kScanTile - 1) / kScanTile;
+    s.scan = plan_scan(R);
     if (int rc = s.launch_classify(h->iso)) return rc;
-    if (int rc = s.launch_count()) return rc;
-    hipLaunchKernelGGL(k_slab_trim_counts, dim3((unsigned)std::min<int64_t>((R + 255) / 256, 4096)), dim3(256), 0,
-                       s.stream, s.d_counts, R, g.emit_lo, g.emit_hi);
-    HIPCALL(hipGetLastError());
+    if (int rc = s.launch_count()) return rc;   // the slab's own rows (fe_count_rows_block)
     if (int rc = s.launch_scan()) return rc;
     if (g.emit_hi < R)
         HIPCALL(hipMemcpyAsync(h->h_vown + p, s.d_voff + g.emit_hi, sizeof(uint64_t), hipMemcpyDeviceToHost, s.stream));
@@ -1126,8 +1097,7 @@ extern "C" int miso_mc_run(miso_mc* h)
     HIPCALL(hipEventRecord(h->ev[0], s.stream));
     if (int rc = s.launch_classify(h->iso)) return rc;
     if (int rc = h->mc.launch_fe_count(s)) return rc;
-    if (int rc = s.launch_scan()) return rc;  // FE row offsets: the rank -> id map layout
-    if (int rc = h->mc.launch_count(s)) return rc;
+    if (int rc = h->mc.launch_scan(s)) return rc;   // FE row offsets too: the rank -> id map layout
     HIPCALL(hipStreamSynchronize(s.stream));
     if (int rc = h->out.reserve(s.h_totals[0], s.h_totals[1])) return rc;
     if (h->out.nverts || h->out.ntris)
@@ -1202,7 +1172,7 @@ extern "C" void miso_mc_destroy(miso_mc* h)
 /* ====================================================================== Flying Edges without allocation */
 
 /* miso_fe_run_noalloc keeps all of its per-extraction device state -- the sign mask, the row counts
- * and trims, the row offsets, the scan state and the two totals -- in this file-scope array instead
+ * and trims, the row offsets, the scan's tile sums and the totals -- in this file-scope array instead
  * of memory allocated per call. Each GPU holds its own copy from the library's load to the end of
  * the process. In host code `scratch` names no device address; the device address is taken per
  * device with hipGetSymbolAddress (scratch_ptr) and only that is passed to kernels. */
@@ -1236,19 +1206,18 @@ size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
 /* Byte offsets of the row state inside the scratch array for geometry g; the total in `end`. */
 struct ScratchLayout {
-    size_t mask, counts, trims, voff, toff, scan, totals, end;
+    size_t mask, counts, trims, voff, toff, sums, totals, end;
     explicit ScratchLayout(const Geom& g)
     {
         const size_t R = (size_t)(g.ny * g.nz);
-        const size_t ntiles = (R + kScanTile - 1) / kScanTile;
         mask = 0;
         counts = align256(mask + R * (size_t)g.W * sizeof(uint64_t));
         trims = align256(counts + R * sizeof(RowCounts));
         voff = align256(trims + R * sizeof(RowTrim));
         toff = align256(voff + R * sizeof(uint64_t));
-        scan = align256(toff + R * sizeof(uint64_t));
-        totals = align256(scan + (1 + 2 * ntiles) * sizeof(uint64_t));
-        end = totals + 2 * sizeof(uint64_t);
+        sums = align256(toff + R * sizeof(uint64_t));
+        totals = align256(sums + (size_t)(kTileSums * plan_scan((int64_t)R).ntiles) * sizeof(uint64_t));
+        end = totals + 5 * sizeof(uint64_t);
     }
 };
 
@@ -1285,16 +1254,14 @@ extern "C" int miso_fe_run_noalloc(const miso_volume* vol, float isoval, void* s
     s.d_trims = (RowTrim*)(sp + lay.trims);
     s.d_voff = (uint64_t*)(sp + lay.voff);
     s.d_toff = (uint64_t*)(sp + lay.toff);
-    s.d_scan = (uint64_t*)(sp + lay.scan);
+    s.d_sums = (uint64_t*)(sp + lay.sums);
     s.d_totals = (uint64_t*)(sp + lay.totals);
-    s.ntiles = (g.ny * g.nz + kScanTile - 1) / kScanTile;
-    // passes 1-3 (pass 2 clears the scan state that pass 3 starts from); pass 4 checks the totals
-    // against the caller's capacities on the device and writes nothing unless they fit
+    s.scan = plan_scan(g.ny * g.nz);
+    // passes 1-3; pass 4 checks the totals against the caller's capacities on the device and writes
+    // nothing unless they fit
     if (int rc = s.launch_classify(isoval)) return rc;
     if (int rc = s.launch_count()) return rc;
-    hipLaunchKernelGGL(k_fe_scan, dim3((unsigned)s.ntiles), dim3(256), 0, s.stream, (const RowCounts*)s.d_counts,
-                       g.ny * g.nz, s.d_voff, s.d_toff, s.d_scan, s.ntiles, s.d_totals);
-    HIPCALL(hipGetLastError());
+    if (int rc = s.launch_scan()) return rc;
     {
         const uint64_t* need = s.d_totals;
         if (s.unit_geometry())

@@ -89,7 +89,53 @@ __device__ __forceinline__ void run_queue(uint64_t* __restrict__ ticket, const i
     }
 }
 
-/* clears the queue tickets and the scan's tile status (a kernel, so it can sit in a graph) */
+/* Pass 2 of the batch's row blocks into the scan's tile sums: a wavefront keeps the sums of the items it
+ * takes one after the other, as long as they lie in one tile, and adds them at once. */
+struct BatchSums {
+    uint64_t* __restrict__ sums;
+    int shift;
+    int64_t tile = -1;
+    uint64_t v[4] = {0, 0, 0, 0};
+
+    __device__ __forceinline__ void flush()
+    {
+        const int l = lane_id();
+        const uint64_t mine = l == 0 ? v[0] : (l == 1 ? v[1] : (l == 2 ? v[2] : v[3]));
+        if (l < 4 && mine) add_sum(&sums[tile * kTileSums + l], mine);
+        v[0] = v[1] = v[2] = v[3] = 0;
+    }
+    __device__ __forceinline__ void add(int64_t t, uint32_t xy, uint32_t zt)
+    {
+        if ((xy | zt) == 0) return;
+        if (t != tile) {
+            if (tile >= 0) flush();
+            tile = t;
+        }
+        v[0] += xy & 0xFFFFu;
+        v[1] += xy >> 16;
+        v[2] += zt & 0xFFFFu;
+        v[3] += zt >> 16;
+    }
+    __device__ __forceinline__ void count(const BatchJob& J, const uint64_t* __restrict__ mask,
+                                          RowCounts* __restrict__ counts, RowTrim* __restrict__ trims, int64_t blk)
+    {
+        // a job's rows start anywhere in a tile, so a wavefront's may lie in two
+        const WaveSums w = fe_count_rows_block(
+            mask + J.mask_base, J.g, counts + J.row_base, trims + J.row_base, blk, NoRowExtra(),
+            [&](uint32_t xy, uint32_t zt, int64_t r0, int64_t r, int nrows) {
+                const int64_t first = (J.row_base + r0) >> shift, last = (J.row_base + r0 + nrows - 1) >> shift;
+                if (first == last) return false;
+                for (int64_t t = first; t <= last; ++t) {
+                    const bool mine = (J.row_base + r) >> shift == t;
+                    add(t, wave_sum_u32(mine ? xy : 0u), wave_sum_u32(mine ? zt : 0u));
+                }
+                return true;
+            });
+        add((J.row_base + (blk * 4 + wave_in_block()) * row_lanes(J.g.W).rpw) >> shift, w.xy, w.zt);
+    }
+};
+
+/* clears the queue tickets and the scan's tile sums (a kernel, so it can sit in a graph) */
 __global__ __launch_bounds__(256) void k_batch_zero(uint64_t* __restrict__ words, int64_t n)
 {
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x)
@@ -131,12 +177,13 @@ __global__ __launch_bounds__(256) void k_batch_count(const BatchJob* __restrict_
                                                      const int64_t* __restrict__ prefix, int njobs, int64_t nitems,
                                                      int chunk, const uint64_t* __restrict__ mask,
                                                      RowCounts* __restrict__ counts, RowTrim* __restrict__ trims,
+                                                     uint64_t* __restrict__ sums, int shift,
                                                      uint64_t* __restrict__ ticket)
 {
-    run_queue(ticket, prefix, njobs, nitems, chunk, [&](int j, int64_t blk) {
-        const BatchJob& J = jobs[j];
-        fe_count_rows_block(mask + J.mask_base, J.g, counts + J.row_base, trims + J.row_base, blk);
-    });
+    BatchSums acc{sums, shift};
+    run_queue(ticket, prefix, njobs, nitems, chunk,
+              [&](int j, int64_t blk) { acc.count(jobs[j], mask, counts, trims, blk); });
+    acc.flush();
 }
 
 /* Job j's first vertex, first triangle, vertex and triangle counts (from the scan). */
@@ -236,13 +283,11 @@ __global__ __launch_bounds__(256) void k_batch_emit(const BatchJob* __restrict__
 
 /* Everything batch_run does on the device after clearing the tickets and the scan state, in one
  * cooperative launch: the grid (every block resident at once) runs pass 1 over the classify
- * groups, pass 2, the scan (tiles taken in order from its ticket) and pass 4 (when the totals
- * fit the output), with a grid-wide barrier between the phases, which also orders every block's
+ * groups, pass 2, the scan and pass 4 (when the totals fit the output), with a grid-wide barrier between the phases, which also orders every block's
  * writes before the next phase's reads; the per-job counts for the host are written beside
  * pass 4, which does not read them. The queues and block functions are those of the separate
  * kernels, so the output is theirs. state: [0..2] tickets, [3..4] totals, [5..12] the XCD
- * tickets, [13..] the scan state (its ticket, then ntiles vertex and ntiles triangle tile
- * status words). */
+ * tickets, [13..] the scan's tile sums. */
 __global__ __launch_bounds__(256) void k_batch_fused(const BatchJob* __restrict__ jobs,
                                                      const int* __restrict__ group_job,
                                                      const int64_t* __restrict__ cls_prefix, int ngroups, int64_t ncls,
@@ -250,8 +295,8 @@ __global__ __launch_bounds__(256) void k_batch_fused(const BatchJob* __restrict_
                                                      int64_t nlane, int chunk, uint64_t* __restrict__ mask,
                                                      RowCounts* __restrict__ counts, RowTrim* __restrict__ trims,
                                                      uint64_t* __restrict__ voff, uint64_t* __restrict__ toff,
-                                                     uint64_t* __restrict__ state, int64_t R, int64_t ntiles,
-                                                     uint64_t* __restrict__ jobout, uint64_t cap_v, uint64_t cap_t,
+                                                     uint64_t* __restrict__ state, int64_t R, int shift,
+                                                     int64_t ntiles, uint64_t* __restrict__ jobout, uint64_t cap_v, uint64_t cap_t,
                                                      float* __restrict__ pts, float* __restrict__ nrm,
                                                      uint32_t* __restrict__ tris, const int64_t* __restrict__ xprefix)
 {
@@ -263,18 +308,14 @@ __global__ __launch_bounds__(256) void k_batch_fused(const BatchJob* __restrict_
     run_queue(state + 0, cls_prefix, ngroups, ncls, chunk,
               [&](int q, int64_t blk) { batch_classify_item(jobs, group_job, mask, q, blk); });
     grid.sync();
-    run_queue(state + 1, lane_prefix, njobs, nlane, chunk, [&](int j, int64_t blk) {
-        const BatchJob& J = jobs[j];
-        fe_count_rows_block(mask + J.mask_base, J.g, counts + J.row_base, trims + J.row_base, blk);
-    });
+    BatchSums acc{state + 13, shift};
+    run_queue(state + 1, lane_prefix, njobs, nlane, chunk,
+              [&](int j, int64_t blk) { acc.count(jobs[j], mask, counts, trims, blk); });
+    acc.flush();
     grid.sync();
-    uint64_t* scan = state + 13;
     uint64_t* totals = state + 3;
-    for (;;) {
-        const int64_t tile = fe_scan_ticket(scan);
-        if (tile >= ntiles) break;
-        fe_scan_tile(counts, R, voff, toff, scan, ntiles, totals, tile);
-    }
+    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x)
+        fe_scan_tile(counts, R, voff, toff, state + 13, shift, ntiles, totals, nullptr, ScanMore(), tile);
     grid.sync();
     for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < njobs; j += (int64_t)gridDim.x * blockDim.x)
         batch_job_counts_one(jobs, njobs, R, voff, toff, totals, jobout, (int)j);

@@ -151,6 +151,9 @@ __device__ __forceinline__ uint64_t wave_incl_scan_u64(uint64_t v)
     return v;
 }
 
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) { return wave_incl_scan_u32(v); }
+__device__ __forceinline__ uint64_t wave_incl_scan(uint64_t v) { return wave_incl_scan_u64(v); }
+
 /* Coordinate of grid index idx along one axis as the reference writes it. A cell computes its
  * lower corner as origin + float(index) * spacing and its upper corner as that plus spacing
  * (flyingEdges/util/Image3D.cpp:45-87), and the vertex on the last index n-1 is only ever written

@@ -6,8 +6,8 @@
  *   k_fe_count     pass 1b + pass 2: from the masks of rows (j,k), (j+1,k), (j,k+1), (j+1,k+1):
  *                  xl/xr trims (cpp:47-65 with isCutEdge :515-554), cut-edge counts per grid
  *                  row and triangle counts per cell row (cpp:72-190) with popcounts.
- *   k_fe_scan      pass 3: single-pass decoupled look-back exclusive scan of the per-row vertex
- *                  and triangle counts into 64-bit offsets (cpp:196-269).
+ *   k_fe_scan      pass 3: exclusive scan of the per-row vertex and triangle counts into 64-bit
+ *                  offsets (cpp:196-269), tile by tile on the tile sums that pass 2 adds up.
  *   k_fe_emit      pass 4: per grid row, the cut edges are compacted into an LDS list already in
  *                  output order, so lanes write consecutive vertices; per cell row, the active
  *                  cells are compacted, a wave prefix sum of numTris gives triangle slots, and
@@ -22,11 +22,45 @@ namespace miso {
 
 constexpr int kRowsPerBlock = 4;        // one wavefront per grid row, 4 waves per block
 constexpr int kSegWords = 16;           // pass 4 processes a row in segments of 16 words (1024 voxels)
-constexpr int kScanItems = 16;
-constexpr int kScanTile = 256 * kScanItems;
-constexpr uint64_t kFlagAgg = 1ull << 62;
-constexpr uint64_t kFlagPre = 2ull << 62;
-constexpr uint64_t kValMask = (1ull << 62) - 1;
+
+/* Pass 3 works on tiles of 2^shift rows: at least 1024 (256 threads, four rows each), and so many that
+ * a scan has at most 1024 tiles as long as tiles of 2^22 rows do: each tile's block adds up the sums of
+ * the tiles before it. Per tile, the sums of the rows' x, y, z, triangle and (first-visit Marching
+ * Cubes) owned-edge counts. */
+constexpr int kTileSums = 5;
+constexpr int kScanStep = 1024;      // rows per block and step
+struct ScanPlan {
+    int shift;
+    int64_t ntiles;
+    // words for the tile sums of up to this many rows: fewer rows may have up to 1024 tiles all the same
+    int64_t sum_words() const { return kTileSums * (ntiles > 1024 ? ntiles : 1024); }
+};
+inline ScanPlan plan_scan(int64_t R)
+{
+    ScanPlan p{10, 0};
+    while (p.shift < 22 && (R >> p.shift) >= 1024) ++p.shift;
+    p.ntiles = (R + (int64_t(1) << p.shift) - 1) >> p.shift;
+    return p;
+}
+
+/* adds v to a tile sum (pass 1 or the batch's first kernel has cleared them) */
+__device__ __forceinline__ void add_sum(uint64_t* __restrict__ sum, uint64_t v)
+{
+    (void)__hip_atomic_fetch_add((unsigned long long*)sum, (unsigned long long)v, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+}
+
+/* A wavefront's counts, the same in every lane: xy = x | y << 16, zt = z | t << 16 (a wavefront's totals stay
+ * below 2^16), and its owned edges. */
+struct WaveSums {
+    uint32_t xy, zt, own;
+};
+
+/* kind a of a wavefront's sums: x, y, z, t, owned */
+__device__ __forceinline__ uint32_t sum_of_kind(const WaveSums& w, int a)
+{
+    return a == 4 ? w.own : ((a & 2) ? w.zt : w.xy) >> ((a & 1) * 16) & 0xFFFFu;
+}
 
 /* ------------------------------------------------------------------ pass 1a: sign mask */
 /* Voxels at the end of a volume that pass 1 leaves in the 256 MB cache beside the HBM, where pass 4,
@@ -180,8 +214,12 @@ __device__ __forceinline__ void fe_classify_block(const float* __restrict__ vol,
 }
 
 __global__ __launch_bounds__(256) void k_fe_classify(const float* __restrict__ vol, Geom g, float iso,
-                                                     uint64_t* __restrict__ mask, int64_t keep_row)
+                                                     uint64_t* __restrict__ mask, int64_t keep_row,
+                                                     uint64_t* __restrict__ sums, int64_t nsums)
 {
+    // pass 2 adds up the tile sums of pass 3: clear them here
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < nsums; t += (int64_t)gridDim.x * blockDim.x)
+        sums[t] = 0;
     fe_classify_block(vol, g, iso, mask, blockIdx.x, keep_row);
 }
 
@@ -189,15 +227,10 @@ __global__ __launch_bounds__(256) void k_fe_classify(const float* __restrict__ v
 __global__ __launch_bounds__(256) void k_fe_count(const uint64_t* __restrict__ mask, Geom g,
                                                   RowCounts* __restrict__ counts,
                                                   RowTrim* __restrict__ trims,
-                                                  uint64_t* __restrict__ scan_state,
-                                                  int64_t scan_state_words)
+                                                  uint64_t* __restrict__ sums, int shift)
 {
     __shared__ uint8_t s_ntri[256];
     for (int c = threadIdx.x; c < 256; c += blockDim.x) s_ntri[c] = (uint8_t)case_tri_count(kCaseEdges[c]);
-    // The scan of pass 3 runs next on the same stream; clear its tickets and tile status here.
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < scan_state_words;
-         t += (int64_t)gridDim.x * blockDim.x)
-        scan_state[t] = 0;
     __syncthreads();
 
     const int lane = lane_id();
@@ -263,6 +296,10 @@ __global__ __launch_bounds__(256) void k_fe_count(const uint64_t* __restrict__ m
         first = min(first, (int64_t)__shfl_xor((long long)first, o));
         last = max(last, (int64_t)__shfl_xor((long long)last, o));
     }
+    if (r < g.emit_lo) xc = yc = zc = tc = 0u;   // a slab's ghost rows, as in fe_count_rows_block
+    if (r >= g.emit_hi) tc = 0u;
+    const uint32_t c4 = lane == 0 ? xc : (lane == 1 ? yc : (lane == 2 ? zc : tc));
+    if (lane < 4 && c4) add_sum(&sums[(r >> shift) * kTileSums + lane], c4);
     if (lane == 0) {
         counts[r] = RowCounts{xc, yc, zc, tc};
         trims[r] = RowTrim{last < 0 ? (uint32_t)g.nx : (uint32_t)first, last < 0 ? 0u : (uint32_t)(last + 1)};
@@ -270,141 +307,119 @@ __global__ __launch_bounds__(256) void k_fe_count(const uint64_t* __restrict__ m
 }
 
 /* ------------------------------------------------------------------ pass 3: scan */
+/* What a scan writes beside the vertex and triangle offsets: for first-visit Marching Cubes the offsets
+ * of the owned edges (owned -> moff), for its edge order those of the x, y and z counts (xyz, R each). */
+struct ScanMore {
+    const uint32_t* owned = nullptr;
+    uint64_t* moff = nullptr;
+    uint64_t* xyz = nullptr;
+};
 
-/* Decoupled look-back (Merrill & Garland): one wavefront inspects 64 predecessors at a time,
- * waiting until each has published an aggregate or an inclusive prefix. Returns the exclusive
- * prefix of `tile`. */
-__device__ uint64_t lookback(uint64_t* __restrict__ status, int64_t tile)
-{
-    const int lane = lane_id();
-    uint64_t excl = 0;
-    int64_t p = tile - 1;
-    for (;;) {
-        const int64_t q = p - lane;
-        uint64_t s = kFlagPre;          // "before the first tile": an inclusive prefix of 0
-        if (q >= 0) {
-            do {
-                s = __hip_atomic_load(&status[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            } while ((s >> 62) == 0);
-        }
-        const uint64_t pre = __ballot((s >> 62) == 2);
-        if (pre) {
-            const int stop = __ffsll((unsigned long long)pre) - 1;
-            excl += wave_sum_u64(lane <= stop ? (s & kValMask) : 0);
-            return excl;
-        }
-        excl += wave_sum_u64(s & kValMask);
-        p -= 64;
-    }
-}
-
-/* One 4096-row tile of the scan (tile numbers are taken from state[0] in launch order, so that a
- * tile's predecessors have started: the look-back waits for them). */
+/* Tile `tile` of the scan: first the sums of the tiles before it (wavefront a takes every fourth kind),
+ * then its own rows, kScanStep at a time, four per thread. The last tile's block writes totals: V, T,
+ * and with xyz the totals of x, y and z after them; V and T also to host (pinned memory), if given.
+ * Latency-bound: no tile waits for another one. By event pairs, 8 us at 512^3 and 14.4 us at 1024^3,
+ * against 17 and 28 with look-back over tiles of 4096 rows; pass 2, which adds up the sums, takes 2 and
+ * 15 us more (27 and 176). A step's sums are of type
+ * S, 64 bits where 1024 rows of 5 nx triangles may pass 2^32. */
+template <typename S = uint32_t>
 __device__ __forceinline__ void fe_scan_tile(const RowCounts* __restrict__ counts, int64_t R,
                                              uint64_t* __restrict__ voff, uint64_t* __restrict__ toff,
-                                             uint64_t* __restrict__ state, int64_t ntiles,
-                                             uint64_t* __restrict__ totals, int64_t tile)
+                                             const uint64_t* __restrict__ sums, int shift, int64_t ntiles,
+                                             uint64_t* __restrict__ totals, uint64_t* __restrict__ host,
+                                             const ScanMore& more, int64_t tile)
 {
-    __shared__ uint64_t s_wv[4], s_wt[4];
-    __shared__ uint64_t s_ev, s_et;
-    uint64_t* stv = state + 1;
-    uint64_t* stt = state + 1 + ntiles;
+    __shared__ uint64_t s_base[8];
+    __shared__ S s_w[kTileSums][4];
     const int lane = lane_id(), wave = threadIdx.x >> 6;
-    const int64_t r0 = tile * kScanTile + (int64_t)threadIdx.x * kScanItems;
-    uint64_t v[kScanItems], t[kScanItems];
-    uint64_t sv = 0, st = 0;
-#pragma unroll
-    for (int u = 0; u < kScanItems; ++u) {
-        const int64_t r = r0 + u;
-        if (r < R) {
-            const RowCounts c = counts[r];
-            v[u] = (uint64_t)c.x + c.y + c.z;
-            t[u] = c.t;
-        } else {
-            v[u] = 0;
-            t[u] = 0;
-        }
-        sv += v[u];
-        st += t[u];
-    }
-    const uint64_t iv = wave_incl_scan_u64(sv), it = wave_incl_scan_u64(st);
-    if (lane == 63) {
-        s_wv[wave] = iv;
-        s_wt[wave] = it;
+    __syncthreads();   // the block's previous tile is done with the LDS
+    for (int a = wave; a < kTileSums; a += 4) {
+        uint64_t b = 0;
+        if (a < 4 || more.owned)
+            for (int64_t t = lane; t < tile; t += 64) b += sums[t * kTileSums + a];
+        b = wave_sum_u64(b);
+        if (lane == 0) s_base[a] = b;
     }
     __syncthreads();
-    uint64_t wbv = 0, wbt = 0, aggv = 0, aggt = 0;
+    uint64_t base[kTileSums];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        if (q < wave) {
-            wbv += s_wv[q];
-            wbt += s_wt[q];
-        }
-        aggv += s_wv[q];
-        aggt += s_wt[q];
-    }
-    if (wave == 0) {
-        uint64_t ev = 0, et = 0;
-        if (tile == 0) {
-            if (lane == 0) {
-                __hip_atomic_store(&stv[0], kFlagPre | aggv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&stt[0], kFlagPre | aggt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        } else {
-            if (lane == 0) {
-                __hip_atomic_store(&stv[tile], kFlagAgg | aggv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&stt[tile], kFlagAgg | aggt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-            ev = lookback(stv, tile);
-            et = lookback(stt, tile);
-            if (lane == 0) {
-                __hip_atomic_store(&stv[tile], kFlagPre | (ev + aggv), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&stt[tile], kFlagPre | (et + aggt), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-        if (lane == 0) {
-            s_ev = ev;
-            s_et = et;
-            if (tile == ntiles - 1) {
-                totals[0] = ev + aggv;
-                totals[1] = et + aggt;
-            }
-        }
-    }
-    __syncthreads();
-    uint64_t pv = s_ev + wbv + iv - sv, pt = s_et + wbt + it - st;
+    for (int a = 0; a < kTileSums; ++a) base[a] = s_base[a];
+    const int64_t r_lo = tile << shift, r_hi = min(R, (tile + 1) << shift);
+    for (int64_t r0 = r_lo; r0 < r_hi; r0 += kScanStep) {
+        const int64_t r = r0 + 4 * (int64_t)threadIdx.x;
+        uint32_t v[4][kTileSums];
+        S own[kTileSums] = {0, 0, 0, 0, 0};
 #pragma unroll
-    for (int u = 0; u < kScanItems; ++u) {
-        const int64_t r = r0 + u;
-        if (r < R) {
-            voff[r] = pv;
-            toff[r] = pt;
+        for (int u = 0; u < 4; ++u) {
+            RowCounts c{0u, 0u, 0u, 0u};
+            if (r + u < r_hi) c = counts[r + u];
+            v[u][0] = c.x;
+            v[u][1] = c.y;
+            v[u][2] = c.z;
+            v[u][3] = c.t;
+            v[u][4] = more.owned && r + u < r_hi ? more.owned[r + u] : 0u;
+#pragma unroll
+            for (int a = 0; a < kTileSums; ++a) own[a] += v[u][a];
         }
-        pv += v[u];
-        pt += t[u];
+        uint64_t ex[kTileSums];
+        S incl[kTileSums];
+#pragma unroll
+        for (int a = 0; a < kTileSums; ++a) {
+            incl[a] = wave_incl_scan(own[a]);
+            if (lane == 63) s_w[a][wave] = incl[a];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int a = 0; a < kTileSums; ++a) {
+            uint64_t before = 0, all = 0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                before += q < wave ? s_w[a][q] : 0u;
+                all += s_w[a][q];
+            }
+            ex[a] = base[a] + before + (incl[a] - own[a]);
+            base[a] += all;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (r + u < r_hi) {
+                voff[r + u] = ex[0] + ex[1] + ex[2];
+                toff[r + u] = ex[3];
+                if (more.owned) more.moff[r + u] = ex[4];
+                if (more.xyz) {
+                    more.xyz[r + u] = ex[0];
+                    more.xyz[R + r + u] = ex[1];
+                    more.xyz[2 * R + r + u] = ex[2];
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < kTileSums; ++a) ex[a] += v[u][a];
+        }
+    }
+    if (tile == ntiles - 1 && threadIdx.x == 0) {
+        totals[0] = base[0] + base[1] + base[2];
+        totals[1] = base[3];
+        if (more.xyz)
+            for (int a = 0; a < 3; ++a) totals[2 + a] = base[a];
+        if (host) {
+            host[0] = base[0] + base[1] + base[2];
+            host[1] = base[3];
+        }
     }
 }
 
-/* The next tile number of the scan, for every thread of the block. */
-__device__ __forceinline__ int64_t fe_scan_ticket(uint64_t* __restrict__ state)
-{
-    __shared__ int64_t s_tile;
-    __syncthreads();   // every thread has read the previous tile number
-    if (threadIdx.x == 0)
-        s_tile = (int64_t)__hip_atomic_fetch_add((unsigned long long*)&state[0], 1ull, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    return s_tile;
-}
-
+template <typename S>
 __global__ __launch_bounds__(256) void k_fe_scan(const RowCounts* __restrict__ counts, int64_t R,
                                                  uint64_t* __restrict__ voff, uint64_t* __restrict__ toff,
-                                                 uint64_t* __restrict__ state, int64_t ntiles,
-                                                 uint64_t* __restrict__ totals)
+                                                 const uint64_t* __restrict__ sums, int shift, int64_t ntiles,
+                                                 uint64_t* __restrict__ totals, uint64_t* __restrict__ host,
+                                                 ScanMore more)
 {
-    // state[0]: ticket, state[1 .. ntiles]: vertex status, state[1+ntiles ..]: triangle status
-    fe_scan_tile(counts, R, voff, toff, state, ntiles, totals, fe_scan_ticket(state));
+    fe_scan_tile<S>(counts, R, voff, toff, sums, shift, ntiles, totals, host, more, blockIdx.x);
 }
+
+inline bool scan_is_wide(int64_t nx) { return nx > (int64_t(1) << 19); }   // 1024 rows of 5 nx triangles
 
 /* ------------------------------------------------------------------ pass 4: emit */
 

@@ -39,6 +39,9 @@ __device__ __forceinline__ RowLanes row_lanes(int64_t W)
     return L;
 }
 
+/* the first row of lane-row block blk */
+__device__ __forceinline__ int64_t block_row(int64_t W, int64_t blk) { return blk * 4 * row_lanes(W).rpw; }
+
 /* This wavefront's index within its 256-thread block, in a scalar register. */
 __device__ __forceinline__ int wave_in_block() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
@@ -213,22 +216,32 @@ __device__ __forceinline__ uint32_t word_tri_count(const CornerWords& C, uint64_
 }
 
 /* ------------------------------------------------------------------ pass 1b + 2 */
-/* per-row work beside the counts (none here; first-visit Marching Cubes adds its owned-edge
- * counts, k_fe_mc_count_rows): called by every lane with the lane's words, row and flags, and
- * `empty` when every word the wavefront loaded is zero */
+/* per-row count beside these (none here; first-visit Marching Cubes adds its owned-edge counts,
+ * k_fe_mc_count_rows): called by every lane with the lane's words, row and flags, and `empty` when
+ * every word the wavefront loaded is zero; the row's count, in every lane of the row */
 struct NoRowExtra {
-    __device__ void operator()(const LaneWords&, const RowLanes&, int64_t, bool, bool, bool, int64_t, int64_t,
-                               bool) const
+    __device__ uint32_t operator()(const LaneWords&, const RowLanes&, int64_t, bool, bool, bool, int64_t, int64_t,
+                                   bool) const
     {
+        return 0u;
     }
 };
 
-/* the 4 wavefronts of lane-row block blk (rows 4 rpw blk ..) */
-template <class Extra = NoRowExtra>
-__device__ __forceinline__ void fe_count_rows_block(const uint64_t* __restrict__ mask, const Geom& g,
-                                                    RowCounts* __restrict__ counts, RowTrim* __restrict__ trims,
-                                                    int64_t blk, Extra extra = Extra())
+/* The 4 wavefronts of lane-row block blk (rows 4 rpw blk ..); the wavefront's sums for pass 3. In a slab,
+ * rows below emit_lo belong to the slab before it (counts 0, so that the slab's offsets start at 0),
+ * and cells from row emit_hi on to the next (triangle counts 0); the vertices of those rows keep their
+ * counts, the slab's last cell row names them. split: shown the
+ * per-row counts (in one lane per row); true where it has taken them itself (the sums are then 0). */
+struct NoSplit {
+    __device__ bool operator()(uint32_t, uint32_t, int64_t, int64_t, int) const { return false; }
+};
+
+template <class Extra = NoRowExtra, class Split = NoSplit>
+__device__ __forceinline__ WaveSums fe_count_rows_block(const uint64_t* __restrict__ mask, const Geom& g,
+                                                        RowCounts* __restrict__ counts, RowTrim* __restrict__ trims,
+                                                        int64_t blk, Extra extra = Extra(), Split split = Split())
 {
+    WaveSums sums{0u, 0u, 0u};
     const RowLanes rl = row_lanes(g.W);
     const int64_t r0 = (blk * 4 + wave_in_block()) * rl.rpw;
     const int64_t r = r0 + rl.q;
@@ -248,7 +261,7 @@ __device__ __forceinline__ void fe_count_rows_block(const uint64_t* __restrict__
             trims[r] = RowTrim{(uint32_t)g.nx, 0u};
         }
         extra(L, rl, r, ok, has_y, has_z, j, k, true);
-        return;
+        return sums;
     }
     const uint64_t vb = low_bits(g.nx - 64 * rl.w), eb = low_bits(g.nx - 1 - 64 * rl.w);
     const uint64_t xcut = (L.m[0] ^ shifted(L.m[0], L.n[0])) & eb;
@@ -264,30 +277,49 @@ __device__ __forceinline__ void fe_count_rows_block(const uint64_t* __restrict__
     uint32_t tc = 0u;
     if (__ballot(live) != 0ull) tc = (has_y && has_z) ? word_tri_count(corner_words(L), eb) : 0u;
     // two counts per 32-bit scan: row totals stay below 2^16 (nx <= 4096, <= 5 triangles a cell)
-    const uint32_t xy = seg_sum((uint32_t)__popcll(xcut) | (uint32_t)__popcll(ycut) << 16, rl.Wp);
-    const uint32_t zt = seg_sum((uint32_t)__popcll(zcut) | tc << 16, rl.Wp);
-    const uint32_t xc = xy & 0xFFFFu, yc = xy >> 16, zc = zt & 0xFFFFu;
-    tc = zt >> 16;
+    uint32_t xy = seg_sum((uint32_t)__popcll(xcut) | (uint32_t)__popcll(ycut) << 16, rl.Wp);
+    uint32_t zt = seg_sum((uint32_t)__popcll(zcut) | tc << 16, rl.Wp);
+    if (r < g.emit_lo) xy = zt = 0u;
+    if (r >= g.emit_hi) zt &= 0xFFFFu;
     first = seg_reduce<OpMin>(first, rl.Wp);
     lastp1 = seg_reduce<OpMax>(lastp1, rl.Wp);
-    if (r < R && rl.w == 0) {
-        counts[r] = RowCounts{xc, yc, zc, tc};
+    const bool head = r < R && rl.w == 0;
+    if (head) {
+        counts[r] = RowCounts{xy & 0xFFFFu, xy >> 16, zt & 0xFFFFu, zt >> 16};
         trims[r] = RowTrim{lastp1 == 0 ? (uint32_t)g.nx : first, lastp1};
     }
-    extra(L, rl, r, ok, has_y, has_z, j, k, false);
+    const uint32_t own = extra(L, rl, r, ok, has_y, has_z, j, k, false);
+    if (!head) xy = zt = 0u;
+    if (split(xy, zt, r0, r, rl.rpw)) return sums;
+    sums.xy = wave_sum_u32(xy);
+    sums.zt = wave_sum_u32(zt);
+    sums.own = wave_sum_u32(head ? own : 0u);
+    return sums;
+}
+
+/* The sums of a block's four wavefronts into those of the block's tile (2^shift rows hold whole
+ * blocks). One atomic per block and kind: with one per wavefront, pass 2 took 215 us at 1024^3 and
+ * 34 us at 512^3 against 162 and 25 without (atomics on one tile's line follow one another). */
+__device__ __forceinline__ void add_block_sums(const WaveSums& w, uint64_t* __restrict__ tile_sums)
+{
+    __shared__ WaveSums s_sums[4];
+    if (lane_id() == 0) s_sums[threadIdx.x >> 6] = w;
+    __syncthreads();
+    const int a = (int)threadIdx.x;
+    if (a >= kTileSums) return;
+    uint32_t v = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v += sum_of_kind(s_sums[q], a);
+    if (v) add_sum(&tile_sums[a], v);
 }
 
 __global__ __launch_bounds__(256) void k_fe_count_rows(const uint64_t* __restrict__ mask, Geom g,
                                                        RowCounts* __restrict__ counts,
                                                        RowTrim* __restrict__ trims,
-                                                       uint64_t* __restrict__ scan_state,
-                                                       int64_t scan_state_words)
+                                                       uint64_t* __restrict__ sums, int shift)
 {
-    // the scan of pass 3 runs next on the same stream; clear its tickets and tile status here
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < scan_state_words;
-         t += (int64_t)gridDim.x * blockDim.x)
-        scan_state[t] = 0;
-    fe_count_rows_block(mask, g, counts, trims, blockIdx.x);
+    const WaveSums w = fe_count_rows_block(mask, g, counts, trims, blockIdx.x);
+    add_block_sums(w, sums + (block_row(g.W, blockIdx.x) >> shift) * kTileSums);
 }
 
 /* ------------------------------------------------------------------ pass 4: edge points */

@@ -10,7 +10,7 @@
  * linear order, first slot of the edge in the owner's case triangle list) -- no hash map needed.
  *
  *   k_mc_count      owned cut edges per cell row
- *   k_scan_u32      decoupled look-back scan of those counts (vertex offsets per cell row)
+ *   k_fe_scan       scans those counts too (vertex offsets per cell row)
  *   k_mc_vertices   owners write point and normal (with the owner's corner coordinates,
  *                   marchingCubes/util/Image3D.cpp:22-65) and record, at the edge's Flying Edges
  *                   rank, the Marching Cubes id
@@ -47,15 +47,11 @@ __device__ __forceinline__ uint32_t owned_edges(bool i0, bool j0, bool k0)
 
 __global__ __launch_bounds__(256) void k_mc_count(const uint64_t* __restrict__ mask, Geom g,
                                                   const RowCounts* __restrict__ counts,
-                                                  uint32_t* __restrict__ owned,
-                                                  uint64_t* __restrict__ scan_state, int64_t scan_state_words)
+                                                  uint32_t* __restrict__ owned, uint64_t* __restrict__ sums, int shift)
 {
     __shared__ EmitLds lds_all[kRowsPerBlock];
     __shared__ uint16_t s_cut[256];
     for (int c = threadIdx.x; c < 256; c += blockDim.x) s_cut[c] = (uint16_t)case_cut_mask(kCaseEdges[c]);
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < scan_state_words;
-         t += (int64_t)gridDim.x * blockDim.x)
-        scan_state[t] = 0;
     __syncthreads();
     const int lane = lane_id();
     const int wave = threadIdx.x >> 6;
@@ -82,63 +78,9 @@ __global__ __launch_bounds__(256) void k_mc_count(const uint64_t* __restrict__ m
         wave_sync();
     }
     total = wave_sum_u32(total);
-    if (lane == 0) owned[r] = total;
-}
-
-/* Exclusive scan of a uint32 per grid row (vals[r * stride]) into uint64 offsets (same look-back
- * as pass 3). */
-__global__ __launch_bounds__(256) void k_scan_u32(const uint32_t* __restrict__ vals, int64_t R,
-                                                  uint64_t* __restrict__ out, uint64_t* __restrict__ state,
-                                                  int64_t ntiles, uint64_t* __restrict__ total, int64_t stride = 1)
-{
-    __shared__ int64_t s_tile;
-    __shared__ uint64_t s_w[4];
-    __shared__ uint64_t s_e;
-    if (threadIdx.x == 0)
-        s_tile = (int64_t)__hip_atomic_fetch_add((unsigned long long*)&state[0], 1ull, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    const int64_t tile = s_tile;
-    uint64_t* st = state + 1;
-    const int lane = lane_id(), wave = threadIdx.x >> 6;
-    const int64_t r0 = tile * kScanTile + (int64_t)threadIdx.x * kScanItems;
-    uint64_t v[kScanItems], sv = 0;
-#pragma unroll
-    for (int u = 0; u < kScanItems; ++u) {
-        const int64_t r = r0 + u;
-        v[u] = r < R ? vals[r * stride] : 0;
-        sv += v[u];
-    }
-    const uint64_t iv = wave_incl_scan_u64(sv);
-    if (lane == 63) s_w[wave] = iv;
-    __syncthreads();
-    uint64_t wb = 0, agg = 0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        if (q < wave) wb += s_w[q];
-        agg += s_w[q];
-    }
-    if (wave == 0) {
-        uint64_t ev = 0;
-        if (tile == 0) {
-            if (lane == 0) __hip_atomic_store(&st[0], kFlagPre | agg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            if (lane == 0) __hip_atomic_store(&st[tile], kFlagAgg | agg, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            ev = lookback(st, tile);
-            if (lane == 0) __hip_atomic_store(&st[tile], kFlagPre | (ev + agg), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (lane == 0) {
-            s_e = ev;
-            if (tile == ntiles - 1) total[0] = ev + agg;
-        }
-    }
-    __syncthreads();
-    uint64_t p = s_e + wb + iv - sv;
-#pragma unroll
-    for (int u = 0; u < kScanItems; ++u) {
-        const int64_t r = r0 + u;
-        if (r < R) out[r] = p;
-        p += v[u];
+    if (lane == 0) {
+        owned[r] = total;
+        if (total) add_sum(&sums[(r >> shift) * kTileSums + 4], total);
     }
 }
 

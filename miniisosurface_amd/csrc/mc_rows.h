@@ -79,25 +79,19 @@ __device__ __forceinline__ uint32_t mc_owned_row_count(const LaneWords& L, const
 __global__ __launch_bounds__(256) void k_fe_mc_count_rows(const uint64_t* __restrict__ mask, Geom g,
                                                           RowCounts* __restrict__ counts,
                                                           RowTrim* __restrict__ trims,
-                                                          uint64_t* __restrict__ scan_state,
-                                                          int64_t scan_state_words, uint32_t* __restrict__ owned,
-                                                          uint64_t* __restrict__ mc_scan_state,
-                                                          int64_t mc_scan_state_words)
+                                                          uint64_t* __restrict__ sums, int shift,
+                                                          uint32_t* __restrict__ owned)
 {
-    // the scans of both numberings run next on the same stream; clear their tickets and status
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < scan_state_words;
-         t += (int64_t)gridDim.x * blockDim.x)
-        scan_state[t] = 0;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < mc_scan_state_words;
-         t += (int64_t)gridDim.x * blockDim.x)
-        mc_scan_state[t] = 0;
     const int64_t R = g.ny * g.nz;
-    fe_count_rows_block(mask, g, counts, trims, blockIdx.x,
-                        [&](const LaneWords& L, const RowLanes& rl, int64_t r, bool ok, bool has_y, bool has_z,
-                            int64_t j, int64_t k, bool empty) {
-                            const uint32_t cnt = empty ? 0u : mc_owned_row_count(L, g, rl, ok, has_y, has_z, j, k);
-                            if (r < R && rl.w == 0) owned[r] = cnt;
-                        });
+    const WaveSums w = fe_count_rows_block(
+        mask, g, counts, trims, blockIdx.x,
+        [&](const LaneWords& L, const RowLanes& rl, int64_t r, bool ok, bool has_y, bool has_z, int64_t j, int64_t k,
+            bool empty) {
+            const uint32_t cnt = empty ? 0u : mc_owned_row_count(L, g, rl, ok, has_y, has_z, j, k);
+            if (r < R && rl.w == 0) owned[r] = cnt;
+            return cnt;
+        });
+    add_block_sums(w, sums + (block_row(g.W, blockIdx.x) >> shift) * kTileSums);
 }
 
 constexpr int kMcCellCap = 512;
