@@ -70,53 +70,111 @@ __host__ __device__ __forceinline__ RowJK split_row(int64_t r0, int q, int64_t n
     return p;
 }
 
-/* Prefix scans and reductions over the Wp lanes of one row segment (Wp a power of two, the
- * segments aligned), with DPP row shifts and broadcasts. */
-struct OpAdd {
-    __device__ static uint32_t f(uint32_t a, uint32_t b) { return a + b; }
-};
-struct OpMin {
-    __device__ static uint32_t f(uint32_t a, uint32_t b) { return a < b ? a : b; }
-};
-struct OpMax {
-    __device__ static uint32_t f(uint32_t a, uint32_t b) { return a > b ? a : b; }
+/* Where a wavefront's rows lie, the same in every lane, so that what a lane works out from it is 32-bit:
+ * the wavefront's first row r0 = (j0, k0), how many of its rows are there, and how many planes lie
+ * above plane k0 (at most 128; the rows span fewer than 66). */
+struct WaveRows {
+    int64_t r0, k0;
+    int j0, ny, n, above;
 };
 
-template <typename Op>
-__device__ __forceinline__ uint32_t seg_incl(uint32_t v, int Wp, int w)
+__device__ __forceinline__ WaveRows wave_rows(const Geom& g, int64_t r0, int rpw)
 {
-    uint32_t n;
-    n = dpp_u32<kDppRowShr1>(v);
-    if (Wp > 1 && w >= 1) v = Op::f(v, n);
-    n = dpp_u32<kDppRowShr2>(v);
-    if (Wp > 2 && w >= 2) v = Op::f(v, n);
-    n = dpp_u32<kDppRowShr4>(v);
-    if (Wp > 4 && w >= 4) v = Op::f(v, n);
-    n = dpp_u32<kDppRowShr8>(v);
-    if (Wp > 8 && w >= 8) v = Op::f(v, n);
-    if (Wp > 16) {
-        n = dpp_u32<kDppRowBcast15, 0xA>(v);
-        if (w & 16) v = Op::f(v, n);
-    }
-    if (Wp > 32) {
-        n = dpp_u32<kDppRowBcast31, 0xC>(v);
-        if (w & 32) v = Op::f(v, n);
-    }
-    return v;
+    WaveRows A;
+    A.r0 = r0;
+    const RowJK first = split_row(r0, 0, g.ny);
+    A.k0 = first.k;
+    A.j0 = (int)first.j;
+    A.ny = (int)g.ny;
+    const int64_t left = g.ny * g.nz - r0, up = g.nz - 1 - A.k0;
+    A.n = (int)(left < rpw ? left : rpw);
+    A.above = (int)(up < 128 ? up : 128);
+    return A;
 }
 
-__device__ __forceinline__ uint32_t seg_excl_scan(uint32_t v, int Wp, int w) { return seg_incl<OpAdd>(v, Wp, w) - v; }
+/* Row r0 + q: its j, and the planes from k0 on */
+struct LaneRow {
+    int j, dk;
+    bool has_y, has_z;
+};
 
-/* segment total (or min / max), valid in every lane of the segment */
-template <typename Op>
-__device__ __forceinline__ uint32_t seg_reduce(uint32_t v, int Wp)
+__device__ __forceinline__ LaneRow lane_row(const WaveRows& A, int q)
 {
-    const int lane = lane_id();
-    const uint32_t inc = seg_incl<Op>(v, Wp, lane & (Wp - 1));
-    return (uint32_t)__shfl(inc, (lane & ~(Wp - 1)) + Wp - 1);
+    LaneRow p;
+    p.j = A.j0 + q;
+    p.dk = 0;
+    if (A.ny >= 64) {
+        const bool wrap = p.j >= A.ny;
+        p.j -= wrap ? A.ny : 0;
+        p.dk = wrap ? 1 : 0;
+    } else {
+        while (p.j >= A.ny) {
+            p.j -= A.ny;
+            ++p.dk;
+        }
+    }
+    p.has_y = p.j < A.ny - 1;
+    p.has_z = p.dk < A.above;
+    return p;
 }
 
-__device__ __forceinline__ uint32_t seg_sum(uint32_t v, int Wp) { return seg_reduce<OpAdd>(v, Wp); }
+/* A lane's entry of a per-row array: row r0 + q + `ahead`, r0 the same in every lane */
+template <typename T>
+__device__ __forceinline__ T& row_entry(T* __restrict__ rows, const WaveRows& A, int q, int64_t ahead = 0)
+{
+    return *reinterpret_cast<T*>(const_cast<char*>(reinterpret_cast<const char*>(rows + (A.r0 + ahead)) +
+                                                   (uint32_t)q * (uint32_t)sizeof(T)));
+}
+
+/* Bits of a lane's word that are voxels (vb), and x-edges or cells (eb): all but in the row's last word */
+struct WordBits {
+    uint64_t vb, eb;
+};
+
+__device__ __forceinline__ WordBits word_bits(const Geom& g, int w)
+{
+    const int last = (int)g.W - 1, in_last = (int)(g.nx - 64 * (int64_t)last);   // 1 .. 64 voxels in the last word
+    const uint64_t vb = ~0ull >> (64 - in_last);
+    return w == last ? WordBits{vb, vb >> 1} : WordBits{~0ull, ~0ull};
+}
+
+/* Prefix sums over the lanes of a row: a scan of the whole wavefront (six DPP adds, no lane masks) less
+ * what comes before the row's first lane. Two counts may share a value, 16 bits each, as long as the
+ * wavefront's totals fit 16 bits (its 4096 voxels have at most 4096 cut edges along an axis and
+ * 20480 triangles). */
+__device__ __forceinline__ uint32_t seg_before(uint32_t incl, const RowLanes& rl)
+{
+    const int head = lane_id() - rl.w;
+    const uint32_t before = (uint32_t)__shfl((int)incl, (head - 1) & 63);
+    return head ? before : 0u;
+}
+
+__device__ __forceinline__ uint32_t seg_excl_scan(uint32_t v, const RowLanes& rl)
+{
+    const uint32_t incl = wave_incl_scan_u32(v);
+    return incl - v - seg_before(incl, rl);
+}
+
+/* the row's total, in every lane of the row */
+__device__ __forceinline__ uint32_t seg_sum(uint32_t v, const RowLanes& rl)
+{
+    const uint32_t incl = wave_incl_scan_u32(v);
+    return (uint32_t)__shfl((int)incl, lane_id() - rl.w + rl.Wp - 1) - seg_before(incl, rl);
+}
+
+/* The row's xl and xr of pass 1, in every lane of the row, from the lanes' trim words: the row's first and
+ * last lanes with a bit are found in the ballot. nx and 0 for a row without one. */
+__device__ __forceinline__ RowTrim seg_trim(uint64_t trim, const RowLanes& rl, int64_t nx)
+{
+    const int head = lane_id() - rl.w;
+    const uint64_t all = __ballot(trim != 0ull) >> head;
+    const uint64_t lanes = rl.Wp == 64 ? all : all & ((1ull << rl.Wp) - 1ull);
+    const uint32_t lo = trim ? (uint32_t)(64 * rl.w + __builtin_ctzll(trim)) : 0u;
+    const uint32_t hi = trim ? (uint32_t)(64 * rl.w + 64 - __builtin_clzll(trim)) : 0u;
+    const uint32_t first = (uint32_t)__shfl((int)lo, head + (lanes ? __builtin_ctzll(lanes) : 0));
+    const uint32_t last = (uint32_t)__shfl((int)hi, head + (lanes ? 63 - __builtin_clzll(lanes) : 0));
+    return lanes ? RowTrim{first, last} : RowTrim{(uint32_t)nx, 0u};
+}
 
 /* Sign-mask words around lane (row r, word w): rows (j,k) (j+1,k) (j,k+1) (j+1,k+1). n holds the
  * lowest bit of each row's next word (the +1 neighbour of bit 63), taken from the next lane, which
@@ -126,20 +184,26 @@ struct LaneWords {
     uint32_t n[4];
 };
 
-__device__ __forceinline__ LaneWords load_lane_words(const uint64_t* __restrict__ mask, const Geom& g, int64_t r,
-                                                     int64_t w, bool ok, bool has_y, bool has_z)
+__device__ __forceinline__ LaneWords load_lane_words(const uint64_t* __restrict__ mask, const Geom& g,
+                                                     const WaveRows& A, const RowLanes& rl, bool ok, bool has_y,
+                                                     bool has_z)
 {
     LaneWords L;
-    const int64_t W = g.W;
-    const int64_t rows[4] = {r, r + 1, r + g.ny, r + g.ny + 1};
+    // scalar bases for the four rows, one 32-bit offset per lane (below 2^15)
+    const uint64_t* __restrict__ base = mask + A.r0 * g.W;
+    const uint32_t off = 8u * ((uint32_t)rl.q * (uint32_t)g.W + (uint32_t)rl.w);
+    const uint64_t* __restrict__ rows[4] = {base, base + g.W, base + g.ny * g.W, base + (g.ny + 1) * g.W};
     const bool rok[4] = {ok, ok && has_y, ok && has_z, ok && has_y && has_z};
     uint32_t low = 0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) L.m[q] = rok[q] ? mask[rows[q] * W + w] : 0ull;
+    for (int q = 0; q < 4; ++q) {
+        L.m[q] = 0ull;
+        if (rok[q]) __builtin_memcpy(&L.m[q], reinterpret_cast<const char*>(rows[q]) + off, 8);
+    }
 #pragma unroll
     for (int q = 0; q < 4; ++q) low |= ((uint32_t)L.m[q] & 1u) << q;
     const uint32_t of_next = dpp_u32<kDppWaveShl1>(low);   // every lane takes part
-    low = w + 1 < W ? of_next : 0u;
+    low = rl.w + 1 < (int)g.W ? of_next : 0u;
 #pragma unroll
     for (int q = 0; q < 4; ++q) L.n[q] = __builtin_amdgcn_ubfe(low, q, 1);
     return L;
@@ -185,43 +249,50 @@ __device__ __forceinline__ uint64_t active_cells(const LaneWords& L, uint64_t eb
     return active_cells(corner_words(L), eb);
 }
 
-/* Triangles of the marching-cubes cases of a word's 64 cells, bit-sliced over the cells. For a
- * cell with corners on both sides of the isovalue, the case table's triangle count
- * (numTris, flyingEdges/util/MarchingCubesTables.h:23-41) equals V - 2F - 4S: V the corners
- * >= iso, F the faces whose four corners are >= iso, S = 1 for the six-corner rings (both ends
- * of a body diagonal below iso, the other six corners >= iso). Cells with all corners >= iso are
- * masked out; cells with none contribute 0. */
-__device__ __forceinline__ uint32_t word_tri_count(const CornerWords& C, uint64_t eb)
+/* Triangles of the marching-cubes cases of a cell row, bit-sliced over the 64 cells of a lane's word: the
+ * lane's share, modulo 2^32, of a count that only the row's sum makes. For a cell with corners on both
+ * sides of the isovalue, the case table's triangle count (numTris,
+ * flyingEdges/util/MarchingCubesTables.h:23-41) equals V - 2F - 4S: V the corners >= iso, F the faces
+ * whose four corners are >= iso, S = 1 for the six-corner rings (both ends of a body diagonal below
+ * iso, the other six corners >= iso); a cell with all corners >= iso has 8 - 12, so each adds 4 back.
+ * Corners and x-faces at x = i + 1 are those at x = i of the next cell, so that over the row they count
+ * twice but at its two ends: V = sum over the four rows of 2 P - (first voxel) - (last voxel), and the
+ * x-faces likewise, which takes one popcount for two. Bits past the row are 0, and no x-pair, ring or
+ * inner face has one there. Pass 2 is bound by its vector instructions; at 1024^3 176 -> 160 us with
+ * this in the place of every corner and face masked and counted, and with 32-bit lane arithmetic. */
+__device__ __forceinline__ uint32_t word_tri_count(const CornerWords& C, const Geom& g, int w)
 {
-    // corners v0..v7 of the cells (the case's bit order)
-    const uint64_t v0 = C.m[0], v1 = C.s[0], v2 = C.s[1], v3 = C.m[1];
-    const uint64_t v4 = C.m[2], v5 = C.s[2], v6 = C.s[3], v7 = C.m[3];
-    const uint64_t a01 = v0 & v1, a23 = v2 & v3, a45 = v4 & v5, a67 = v6 & v7;
-    const uint64_t a03 = v0 & v3, a12 = v1 & v2, a56 = v5 & v6, a47 = v4 & v7;
-    const uint64_t M = eb & ~(a01 & a23 & a45 & a67);
-    uint32_t V = 0;
-    V += (uint32_t)__popcll(v0 & M) + (uint32_t)__popcll(v1 & M) + (uint32_t)__popcll(v2 & M) +
-         (uint32_t)__popcll(v3 & M);
-    V += (uint32_t)__popcll(v4 & M) + (uint32_t)__popcll(v5 & M) + (uint32_t)__popcll(v6 & M) +
-         (uint32_t)__popcll(v7 & M);
-    const uint32_t F = (uint32_t)__popcll(a01 & a23 & M) + (uint32_t)__popcll(a45 & a67 & M) +
-                       (uint32_t)__popcll(a01 & a45 & M) + (uint32_t)__popcll(a23 & a67 & M) +
-                       (uint32_t)__popcll(a03 & a47 & M) + (uint32_t)__popcll(a12 & a56 & M);
-    // body diagonals (0,6) (1,7) (2,4) (3,5): both ends set, and both ends clear
-    const uint64_t pd0 = v0 & v6, pd1 = v1 & v7, pd2 = v2 & v4, pd3 = v3 & v5;
-    const uint64_t p01 = pd0 & pd1, p23 = pd2 & pd3;
-    const uint32_t S = (uint32_t)__popcll(~(v0 | v6) & pd1 & p23 & eb) + (uint32_t)__popcll(~(v1 | v7) & pd0 & p23 & eb) +
-                       (uint32_t)__popcll(~(v2 | v4) & p01 & pd3 & eb) + (uint32_t)__popcll(~(v3 | v5) & p01 & pd2 & eb);
-    return V - 2 * F - 4 * S;
+    const uint64_t p0 = C.m[0] & C.s[0], p1 = C.m[1] & C.s[1], p2 = C.m[2] & C.s[2], p3 = C.m[3] & C.s[3];
+    const uint64_t f01 = p0 & p1, f23 = p2 & p3;
+    const uint64_t xface = C.m[0] & C.m[1] & C.m[2] & C.m[3];
+    const uint32_t P = (uint32_t)__popcll(C.m[0]) + (uint32_t)__popcll(C.m[1]) + (uint32_t)__popcll(C.m[2]) +
+                       (uint32_t)__popcll(C.m[3]);
+    const uint32_t F = (uint32_t)__popcll(f01) + (uint32_t)__popcll(f23) + (uint32_t)__popcll(p0 & p2) +
+                       (uint32_t)__popcll(p1 & p3);
+    // body diagonals: both ends of v0-v6, v1-v7, v2-v4, v3-v5 (rows 0 and 3, 1 and 2)
+    const uint64_t d0 = C.m[0] & C.s[3], d1 = C.s[0] & C.m[3], d2 = C.s[1] & C.m[2], d3 = C.m[1] & C.s[2];
+    const uint64_t ring = (((~(C.m[0] | C.s[3]) & d1) | (~(C.s[0] | C.m[3]) & d0)) & (d2 & d3)) |
+                          (((~(C.s[1] | C.m[2]) & d3) | (~(C.m[1] | C.s[2]) & d2)) & (d0 & d1));
+    // the row's first and last voxels, one bit per row
+    const int last = (int)g.W - 1, top = (int)(g.nx - 64 * (int64_t)last) - 1;
+    uint32_t lo = 0, hi = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        lo |= ((uint32_t)C.m[q] & 1u) << q;
+        hi |= ((uint32_t)(C.m[q] >> top) & 1u) << q;
+    }
+    lo = w == 0 ? lo : 0u;
+    hi = w == last ? hi : 0u;
+    const uint32_t ends = (uint32_t)__popc(lo) + (uint32_t)__popc(hi), xends = (lo == 15u) + (hi == 15u);
+    return 2 * (P - F + xends) - ends -
+           4 * ((uint32_t)__popcll(xface) - (uint32_t)__popcll(f01 & f23) + (uint32_t)__popcll(ring));
 }
 
 /* ------------------------------------------------------------------ pass 1b + 2 */
 /* per-row count beside these (none here; first-visit Marching Cubes adds its owned-edge counts,
- * k_fe_mc_count_rows): called by every lane with the lane's words, row and flags, and `empty` when
- * every word the wavefront loaded is zero; the row's count, in every lane of the row */
+ * k_fe_mc_count_rows): called by every lane with its words and row, and `empty` when every word the wavefront loaded is zero; the row's count, in every lane of the row */
 struct NoRowExtra {
-    __device__ uint32_t operator()(const LaneWords&, const RowLanes&, int64_t, bool, bool, bool, int64_t, int64_t,
-                                   bool) const
+    __device__ uint32_t operator()(const LaneWords&, const RowLanes&, const WaveRows&, bool, const LaneRow&, bool) const
     {
         return 0u;
     }
@@ -244,53 +315,46 @@ __device__ __forceinline__ WaveSums fe_count_rows_block(const uint64_t* __restri
     WaveSums sums{0u, 0u, 0u};
     const RowLanes rl = row_lanes(g.W);
     const int64_t r0 = (blk * 4 + wave_in_block()) * rl.rpw;
-    const int64_t r = r0 + rl.q;
-    const int64_t R = g.ny * g.nz;
-    const bool ok = r < R && rl.w < g.W;
-    const RowJK jk = split_row(r0, rl.q, g.ny);
-    const int64_t j = jk.j, k = jk.k;
-    const bool has_y = j < g.ny - 1, has_z = k < g.nz - 1;
-    const LaneWords L = load_lane_words(mask, g, r, rl.w, ok, has_y, has_z);
+    if (r0 >= g.ny * g.nz) return sums;
+    const WaveRows A = wave_rows(g, r0, rl.rpw);
+    const bool there = rl.q < A.n, ok = there && rl.w < (int)g.W, head = there && rl.w == 0;
+    const LaneRow at = lane_row(A, rl.q);
+    const bool has_y = at.has_y, has_z = at.has_z;
+    const LaneWords L = load_lane_words(mask, g, A, rl, ok, has_y, has_z);
     // the words and bit 0 of the next words (corner i + 1 of bit 63)
     const uint64_t any = L.m[0] | L.m[1] | L.m[2] | L.m[3] | (uint64_t)(L.n[0] | L.n[1] | L.n[2] | L.n[3]);
     if (__ballot(any != 0ull) == 0ull) {
         // every voxel the wavefront's rows see is below the isovalue (most wavefronts at a
         // sparse, high isovalue): no cut edge, no triangle, an empty trim
-        if (r < R && rl.w == 0) {
-            counts[r] = RowCounts{0u, 0u, 0u, 0u};
-            trims[r] = RowTrim{(uint32_t)g.nx, 0u};
+        if (head) {
+            row_entry(counts, A, rl.q) = RowCounts{0u, 0u, 0u, 0u};
+            row_entry(trims, A, rl.q) = RowTrim{(uint32_t)g.nx, 0u};
         }
-        extra(L, rl, r, ok, has_y, has_z, j, k, true);
+        extra(L, rl, A, ok, at, true);
         return sums;
     }
-    const uint64_t vb = low_bits(g.nx - 64 * rl.w), eb = low_bits(g.nx - 1 - 64 * rl.w);
+    const auto [vb, eb] = word_bits(g, rl.w);
     const uint64_t xcut = (L.m[0] ^ shifted(L.m[0], L.n[0])) & eb;
     const uint64_t ycut = has_y ? ((L.m[0] ^ L.m[1]) & vb) : 0;
     const uint64_t zcut = has_z ? ((L.m[0] ^ L.m[2]) & vb) : 0;
     const uint64_t trim = (xcut | ycut | zcut) & eb;
-    // positions as unsigned: "none" is 0xFFFFFFFF for the minimum and 0 (= last + 1) for the maximum
-    uint32_t first = trim ? (uint32_t)(64 * rl.w + __builtin_ctzll(trim)) : 0xFFFFFFFFu;
-    uint32_t lastp1 = trim ? (uint32_t)(64 * rl.w + 64 - __builtin_clzll(trim)) : 0u;
     // word_tri_count is 0 where every corner of the lane's cells is below the isovalue (`any`
     // zero); a wavefront with only such lanes skips it
     const bool live = has_y && has_z && any != 0ull;
     uint32_t tc = 0u;
-    if (__ballot(live) != 0ull) tc = (has_y && has_z) ? word_tri_count(corner_words(L), eb) : 0u;
-    // two counts per 32-bit scan: row totals stay below 2^16 (nx <= 4096, <= 5 triangles a cell)
-    uint32_t xy = seg_sum((uint32_t)__popcll(xcut) | (uint32_t)__popcll(ycut) << 16, rl.Wp);
-    uint32_t zt = seg_sum((uint32_t)__popcll(zcut) | tc << 16, rl.Wp);
-    if (r < g.emit_lo) xy = zt = 0u;
-    if (r >= g.emit_hi) zt &= 0xFFFFu;
-    first = seg_reduce<OpMin>(first, rl.Wp);
-    lastp1 = seg_reduce<OpMax>(lastp1, rl.Wp);
-    const bool head = r < R && rl.w == 0;
+    if (__ballot(live) != 0ull) tc = (has_y && has_z) ? word_tri_count(corner_words(L), g, rl.w) : 0u;
+    uint32_t xy = seg_sum((uint32_t)__popcll(xcut) | (uint32_t)__popcll(ycut) << 16, rl);
+    uint32_t zt = seg_sum((uint32_t)__popcll(zcut) | tc << 16, rl);
+    if (r0 + rl.q < g.emit_lo) xy = zt = 0u;
+    if (r0 + rl.q >= g.emit_hi) zt &= 0xFFFFu;
+    const RowTrim tr = seg_trim(trim, rl, g.nx);
     if (head) {
-        counts[r] = RowCounts{xy & 0xFFFFu, xy >> 16, zt & 0xFFFFu, zt >> 16};
-        trims[r] = RowTrim{lastp1 == 0 ? (uint32_t)g.nx : first, lastp1};
+        row_entry(counts, A, rl.q) = RowCounts{xy & 0xFFFFu, xy >> 16, zt & 0xFFFFu, zt >> 16};
+        row_entry(trims, A, rl.q) = tr;
     }
-    const uint32_t own = extra(L, rl, r, ok, has_y, has_z, j, k, false);
+    const uint32_t own = extra(L, rl, A, ok, at, false);
     if (!head) xy = zt = 0u;
-    if (split(xy, zt, r0, r, rl.rpw)) return sums;
+    if (split(xy, zt, r0, r0 + rl.q, rl.rpw)) return sums;
     sums.xy = wave_sum_u32(xy);
     sums.zt = wave_sum_u32(zt);
     sums.own = wave_sum_u32(head ? own : 0u);
@@ -566,31 +630,31 @@ __device__ __forceinline__ bool emit_rows_setup(EmitRows& E, EmitRowsLds* s_w, c
     const int64_t R = g.ny * g.nz;
     E.r0 = (blk * 4 + E.wv) * rl.rpw;
     if (E.r0 >= R) return false;
-    const int64_t r = E.r0 + rl.q;
-    const bool ok = r < R && rl.w < g.W;
-    const bool first = ok && rl.w == 0;        // the lane that holds the row's state
-    // a wavefront whose rows have no vertex and no triangle leaves before reading mask words
-    // (most of them at a sparse isovalue)
+    // a wavefront whose rows have no vertex and no triangle leaves before anything else (most of
+    // them at a sparse isovalue)
     RowCounts c{0u, 0u, 0u, 0u};
-    if (first) c = counts[r];
+    const bool ok = E.r0 + rl.q < R && rl.w < (int)g.W;
+    const bool first = ok && rl.w == 0;        // the lane that holds the row's state
+    if (first) c = counts[E.r0 + rl.q];
     if (__ballot((c.x | c.y | c.z | c.t) != 0u) == 0ull) return false;
-    const RowJK jk = split_row(E.r0, rl.q, g.ny);
-    const bool has_y = jk.j < g.ny - 1, has_z = jk.k < g.nz - 1;
-    const LaneWords L = load_lane_words(mask, g, r, rl.w, ok, has_y, has_z);
+    const WaveRows A = wave_rows(g, E.r0, rl.rpw);
+    const LaneRow at = lane_row(A, rl.q);
+    const bool has_y = at.has_y, has_z = at.has_z;
+    const LaneWords L = load_lane_words(mask, g, A, rl, ok, has_y, has_z);
     E.v0 = voff[E.r0];
     E.t0 = toff[E.r0];
-    E.k0 = uniform_div(E.r0, g.ny);
-    E.j0 = (int)(E.r0 - E.k0 * g.ny);
+    E.k0 = A.k0;
+    E.j0 = A.j0;
     // the row's vertex offset and, in the plane above, that row's, from v0 and v2 (below 2^16: at
     // most 65 rows of 64 words in all hold 3 * 64 * 65 voxels' edges)
-    const bool up = E.r0 + g.ny < R;
-    E.v2 = up ? voff[E.r0 + g.ny] : 0ull;
+    const int64_t left_above = R - E.r0 - g.ny;             // rows from the one above the wavefront's first
+    E.v2 = left_above > 0 ? voff[E.r0 + g.ny] : 0ull;
     uint32_t own = 0, above = 0, above_x = 0;
     if (first) {
-        own = (uint32_t)(voff[r] - E.v0);
-        if (r + g.ny < R) {
-            above = (uint32_t)(voff[r + g.ny] - E.v2);
-            above_x = counts[r + g.ny].x;
+        own = (uint32_t)(row_entry(voff, A, rl.q) - E.v0);
+        if (rl.q < left_above) {
+            above = (uint32_t)(row_entry(voff, A, rl.q, g.ny) - E.v2);
+            above_x = row_entry(counts, A, rl.q, g.ny).x;
         }
     }
     // first ids of the row's x-edges (a, low), z-edges (a, high), y-edges (b); x- and y-edges above (c)
@@ -613,7 +677,7 @@ __device__ __forceinline__ bool emit_rows_setup(EmitRows& E, EmitRowsLds* s_w, c
     cc = (uint32_t)__shfl((int)cc, head);
     E.wp_log2 = 6 - __builtin_ctz((unsigned)rl.rpw);
 
-    const uint64_t vb = low_bits(g.nx - 64 * rl.w), eb = low_bits(g.nx - 1 - 64 * rl.w);
+    const auto [vb, eb] = word_bits(g, rl.w);
     const uint64_t cw[8] = {(L.m[0] ^ shifted(L.m[0], L.n[0])) & eb, (L.m[1] ^ shifted(L.m[1], L.n[1])) & eb,
                             (L.m[2] ^ shifted(L.m[2], L.n[2])) & eb, (L.m[3] ^ shifted(L.m[3], L.n[3])) & eb,
                             (L.m[0] ^ L.m[1]) & vb, (L.m[2] ^ L.m[3]) & vb,
@@ -624,8 +688,7 @@ __device__ __forceinline__ bool emit_rows_setup(EmitRows& E, EmitRowsLds* s_w, c
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         // two combinations per segmented scan and per dword
-        lo[q] = base[q] + seg_excl_scan((uint32_t)__popcll(cw[2 * q]) | (uint32_t)__popcll(cw[2 * q + 1]) << 16, rl.Wp,
-                                        rl.w);
+        lo[q] = base[q] + seg_excl_scan((uint32_t)__popcll(cw[2 * q]) | (uint32_t)__popcll(cw[2 * q + 1]) << 16, rl);
         hi[q] = lo[q] + ((uint32_t)__popc((uint32_t)cw[2 * q]) | (uint32_t)__popc((uint32_t)cw[2 * q + 1]) << 16);
     }
     EmitRowsLds& S = s_w[E.wv];
@@ -637,7 +700,7 @@ __device__ __forceinline__ bool emit_rows_setup(EmitRows& E, EmitRowsLds* s_w, c
         S.words[q][2 * E.lane] = (uint32_t)m[q];
         S.words[q][2 * E.lane + 1] = (uint32_t)(m[q] >> 32);
     }
-    const bool emit = ok && r >= g.emit_lo && r < g.emit_hi;
+    const bool emit = ok && E.r0 + rl.q >= g.emit_lo && E.r0 + rl.q < g.emit_hi;
     E.origins = emit ? cw[0] | (m[0] ^ m[1]) | (m[0] ^ m[2]) : 0ull;
     E.act = emit && has_y && has_z ? active_cells(L, eb) : 0ull;
     wave_sync();

@@ -50,14 +50,16 @@ __device__ __forceinline__ uint64_t corner_plane(const CornerWords& C, int q)
     }
 }
 
-/* Owned cut edges of the cell row of lane words L (row r = (j, k)), summed over the row's lanes
- * (valid in every lane of the row): bit-sliced over the 64 cells of a word. Lanes without cells
- * (the last row or plane, or past the row) count nothing, whatever their words. */
-__device__ __forceinline__ uint32_t mc_owned_row_count(const LaneWords& L, const Geom& g, const RowLanes& rl, bool ok,
-                                                       bool has_y, bool has_z, int64_t j, int64_t k)
+/* Owned cut edges of the cell row of lane words L (row `at` from (j0, k0)), summed over the row's lanes
+ * (valid in every lane of the row): bit-sliced over the 64 cells of a word. Lanes without cells (the
+ * last row or plane, or past the row) count nothing, whatever their words. */
+__device__ __forceinline__ uint32_t mc_owned_row_count(const LaneWords& L, const Geom& g, const RowLanes& rl,
+                                                       const WaveRows& A, bool ok, const LaneRow& at)
 {
+    const int j = at.j;
+    const bool k_first = A.k0 == 0 && at.dk == 0;
     const CornerWords C = corner_words(L);
-    const uint64_t eb = (ok && has_y && has_z) ? low_bits(g.nx - 1 - 64 * rl.w) : 0ull;
+    const uint64_t eb = (ok && at.has_y && at.has_z) ? word_bits(g, rl.w).eb : 0ull;
     const uint64_t first_cell = rl.w == 0 ? 1ull : 0ull;
     uint32_t cnt = 0;
 #pragma unroll
@@ -67,11 +69,11 @@ __device__ __forceinline__ uint32_t mc_owned_row_count(const LaneWords& L, const
         // e: 0(j,k) 1(k) 2(k) 3(i,k) 4(j) 7(i) 8(i,j) 9(j) 10(i); always 5 6 11
         uint64_t own = eb;
         if (need_j && j != 0) own = 0;
-        if (need_k && k != 0) own = 0;
+        if (need_k && !k_first) own = 0;
         if (need_i) own &= first_cell;
         cnt += (uint32_t)__popcll(cut & own);
     }
-    return seg_sum(cnt, rl.Wp);
+    return seg_sum(cnt, rl);
 }
 
 /* Flying Edges pass 2 (k_fe_count_rows) and the first-visit owned-edge counts per cell row in
@@ -82,13 +84,11 @@ __global__ __launch_bounds__(256) void k_fe_mc_count_rows(const uint64_t* __rest
                                                           uint64_t* __restrict__ sums, int shift,
                                                           uint32_t* __restrict__ owned)
 {
-    const int64_t R = g.ny * g.nz;
     const WaveSums w = fe_count_rows_block(
         mask, g, counts, trims, blockIdx.x,
-        [&](const LaneWords& L, const RowLanes& rl, int64_t r, bool ok, bool has_y, bool has_z, int64_t j, int64_t k,
-            bool empty) {
-            const uint32_t cnt = empty ? 0u : mc_owned_row_count(L, g, rl, ok, has_y, has_z, j, k);
-            if (r < R && rl.w == 0) owned[r] = cnt;
+        [&](const LaneWords& L, const RowLanes& rl, const WaveRows& A, bool ok, const LaneRow& at, bool empty) {
+            const uint32_t cnt = empty ? 0u : mc_owned_row_count(L, g, rl, A, ok, at);
+            if (rl.q < A.n && rl.w == 0) row_entry(owned, A, rl.q) = cnt;
             return cnt;
         });
     add_block_sums(w, sums + (block_row(g.W, blockIdx.x) >> shift) * kTileSums);
@@ -190,12 +190,11 @@ __global__ __launch_bounds__(256) void k_mc_vertices_rows(const float* __restric
     const int64_t r0 = (emit_block(blockIdx.x, gridDim.x, g) * 4 + wv) * rl.rpw;   // Flying Edges pass 4's order
     if (r0 >= R) return;
     const int64_t r = r0 + rl.q;
-    const bool ok = r < R && rl.w < g.W;
-    const RowJK jk = split_row(r0, rl.q, g.ny);
-    const int64_t j = jk.j, k = jk.k;
-    const bool cells = ok && j < g.ny - 1 && k < g.nz - 1;
-    const LaneWords L = load_lane_words(mask, g, r, rl.w, cells, true, true);
-    const uint64_t vb = low_bits(g.nx - 64 * rl.w), eb = low_bits(g.nx - 1 - 64 * rl.w);
+    const WaveRows A = wave_rows(g, r0, rl.rpw);
+    const LaneRow at = lane_row(A, rl.q);
+    const bool cells = rl.q < A.n && rl.w < (int)g.W && at.has_y && at.has_z;
+    const LaneWords L = load_lane_words(mask, g, A, rl, cells, true, true);
+    const auto [vb, eb] = word_bits(g, rl.w);
     const CornerWords C = corner_words(L);
     const uint64_t act = cells ? active_cells(C, eb) : 0ull;
     const uint32_t ncell = (uint32_t)__popcll(act);
@@ -218,8 +217,7 @@ __global__ __launch_bounds__(256) void k_mc_vertices_rows(const float* __restric
         }
 #pragma unroll
         for (int q = 0; q < 8; q += 2) {
-            const uint32_t ex = seg_excl_scan((uint32_t)__popcll(cw[q]) | (uint32_t)__popcll(cw[q + 1]) << 16, rl.Wp,
-                                              rl.w);
+            const uint32_t ex = seg_excl_scan((uint32_t)__popcll(cw[q]) | (uint32_t)__popcll(cw[q + 1]) << 16, rl);
             S.cut[q][lane] = cw[q];
             S.cut[q + 1][lane] = cw[q + 1];
             S.base[q][lane] = (uint32_t)(cb[q] - v0) + (ex & 0xFFFFu);
@@ -237,7 +235,7 @@ __global__ __launch_bounds__(256) void k_mc_vertices_rows(const float* __restric
     const uint32_t clo[8] = {lo[0], lo[1], lo[3], lo[2], lo[4], lo[5], lo[7], lo[6]};
     const uint32_t chi[8] = {hi[0], hi[1], hi[3], hi[2], hi[4], hi[5], hi[7], hi[6]};
     const uint32_t cfirst = cincl - ncell;
-    const int64_t k0 = uniform_div(r0, g.ny), j0 = r0 - k0 * g.ny;
+    const int64_t k0 = A.k0, j0 = A.j0;
     uint64_t mid = EdgeOrder ? 0 : moff[r0];   // the wavefront's first Marching Cubes vertex
     for (uint32_t win = 0; win < ctotal; win += kMcCellCap) {
         const uint32_t wend = win + kMcCellCap;
