@@ -514,7 +514,7 @@ def bench_batched(reps, cpu_threads=None):
             return round((time.perf_counter() - t0) / reps * 1e3, 3)
 
         # at the tuned shape: pass 4's queue order (one queue, or one per XCD), then the launch
-        # (six kernels from one graph, or one cooperative kernel)
+        # (five kernels from one graph, or one cooperative kernel)
         chosen, by_order = b.queue_order(), {}
         for order in ("dispatch", "xcd"):
             b.set_queue_order(order)

@@ -184,19 +184,20 @@ int miso_batch_job_output(const miso_batch* b, int64_t job, const float** points
                           const uint32_t** triangles);
 /* host copy of one job's mesh, triangles widened to 64-bit (util::TriangleMesh's size_t) */
 int miso_batch_copy_out(miso_batch* b, int64_t job, float* points, float* normals, uint64_t* triangles);
-/* launch shape of the persistent kernels: resident blocks per CU and work items per ticket */
+/* launch shape of the persistent kernels, passes 1 and 2 (and all of a fused launch): pairs of blocks per CU
+ * (blocks, in a fused launch), and the consecutive work items a block takes at a time */
 int miso_batch_set_tuning(miso_batch* b, int blocks_per_cu, int chunk);
 int miso_batch_get_tuning(const miso_batch* b, int* blocks_per_cu, int* chunk);
-/* Pass 4's work queue. DISPATCH (the default): one queue, row blocks in job order. XCD: one
- * queue per XCD of the MI355X (a persistent block serves the queue of the XCD it runs on, block
- * b on XCD b mod 8); each XCD owns every eighth row block of a job, in the tile order of the
- * single-volume pass 4, so that neighbouring rows meet in one XCD's L2. Same output. */
+/* The order of pass 4's work, a row block of one job per workgroup. DISPATCH (the default): the jobs'
+ * row blocks in order, from the last one. XCD: workgroup b runs on XCD b mod 8 of the MI355X; each XCD
+ * owns every eighth row block of a job, in the tile order of the single-volume pass 4, so that
+ * neighbouring rows meet in one XCD's L2. Same output. */
 #define MISO_BATCH_QUEUE_DISPATCH 0
 #define MISO_BATCH_QUEUE_XCD 1
 int miso_batch_set_queue_order(miso_batch* b, int order);
 int miso_batch_get_queue_order(const miso_batch* b, int* order);
 /* How miso_batch_run launches once the output capacity is known from an earlier run. GRAPHS (the
- * default): one captured graph of six kernels (clear, passes 1, 2, 3, per-job counts, 4). FUSED:
+ * default): one captured graph of five kernels (passes 1, 2, 3, per-job counts, 4). FUSED:
  * one cooperative kernel whose resident blocks run the same phases with a grid-wide barrier
  * between them (at most the blocks per CU that fit at once; MISO_ERR_ARG where the device has no
  * cooperative launch). Same output; a run whose output outgrows the buffers ends with pass 4
@@ -205,8 +206,8 @@ int miso_batch_get_queue_order(const miso_batch* b, int* order);
 #define MISO_BATCH_LAUNCH_FUSED 1
 int miso_batch_set_launch(miso_batch* b, int mode);
 int miso_batch_get_launch(const miso_batch* b, int* mode);
-/* times every setting of a small grid on this batch (reps runs each) -- resident blocks per CU,
- * items per ticket, pass 4's queue order, launch mode -- and keeps the fastest */
+/* times every setting of a small grid on this batch (reps runs each) -- blocks per CU, items
+ * at a time, pass 4's order, launch mode -- and keeps the fastest */
 int miso_batch_autotune(miso_batch* b, int reps, float* best_ms);
 /* device time of the last run, passes 1-4 */
 int miso_batch_time_ms(const miso_batch* b, float* ms);

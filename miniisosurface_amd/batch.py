@@ -79,7 +79,7 @@ class BatchExtraction:
         return b.value, c.value
 
     def set_queue_order(self, order):
-        """Pass 4's work queue: "dispatch" (one queue) or "xcd" (one per XCD, tiled rows)."""
+        """Order of pass 4's row blocks: "dispatch" (the jobs' order) or "xcd" (tiled rows per XCD)."""
         check(lib().miso_batch_set_queue_order(self._h, {"dispatch": 0, "xcd": 1}[order]), "set_queue_order")
 
     def queue_order(self):
@@ -88,7 +88,7 @@ class BatchExtraction:
         return ("dispatch", "xcd")[o.value]
 
     def set_launch(self, mode):
-        """How run() launches once the output size is known: "graphs" (six kernels replayed from
+        """How run() launches once the output size is known: "graphs" (five kernels replayed from
         one HIP graph) or "fused" (one cooperative kernel, a grid barrier between the passes)."""
         check(lib().miso_batch_set_launch(self._h, {"graphs": 0, "fused": 1}[mode]), "set_launch")
 

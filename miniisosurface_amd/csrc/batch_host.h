@@ -27,8 +27,7 @@ struct miso_batch {
     RowTrim* d_trims = nullptr;
     uint64_t* d_voff = nullptr;
     uint64_t* d_toff = nullptr;
-    uint64_t* d_state = nullptr;      // [0..2] queue tickets, [3] totals V, [4] totals T, [5..12] the XCD
-                                      // queues' tickets of pass 4, [13..] scan tile sums
+    uint64_t* d_state = nullptr;      // [0..1] totals V, T, [2..] the scan's tile sums
     int64_t state_words = 0;
     uint64_t* d_jobout = nullptr;     // 4 per job: first vertex, first triangle, vertices, triangles
     uint64_t* h_jobout = nullptr;     // pinned copy, then the two totals
@@ -37,8 +36,8 @@ struct miso_batch {
     uint32_t* d_tris = nullptr;
     uint64_t cap_v = 0, cap_t = 0;
     int blocks_per_cu = 4, chunk = 4, num_cus = 256;
-    int queue_order = MISO_BATCH_QUEUE_DISPATCH;     // pass 4's work queue: one, or one per XCD
-    int launch = MISO_BATCH_LAUNCH_GRAPHS;           // graph of six kernels, or k_batch_fused
+    int queue_order = MISO_BATCH_QUEUE_DISPATCH;     // pass 4's block order: the jobs', or per XCD
+    int launch = MISO_BATCH_LAUNCH_GRAPHS;           // graph of five kernels, or k_batch_fused
     int fused_per_cu = 0;                            // k_batch_fused blocks resident per CU (0: none)
     std::vector<int64_t> xcd_prefix;                 // 8 x (njobs + 1): XCD x's pass 4 items before job j
     int64_t* d_xcd_prefix = nullptr;
@@ -51,10 +50,10 @@ struct miso_batch {
     float last_ms = 0.0f;
     bool ran = false;
 
-    uint64_t* tickets() { return d_state; }
-    uint64_t* totals() { return d_state + 3; }
-    uint64_t* xcd_tickets() { return d_state + 5; }
-    uint64_t* scan_sums() { return d_state + 13; }
+    BatchUnits units = kSomeUnit;
+
+    uint64_t* totals() { return d_state; }
+    uint64_t* scan_sums() { return d_state + 2; }
 };
 
 namespace {
@@ -86,9 +85,11 @@ void destroy_graphs(miso_batch* b)
     b->g_scan = b->g_emit = b->g_all = nullptr;
 }
 
+/* blocks of a persistent kernel (pass 1 or 2): two per tuned block per CU, so that the default of 4 fills
+ * the 32 wavefronts a CU holds (256 mixed volumes: 668 us for the batch, 700 with half of them) */
 unsigned batch_grid(const miso_batch* b, int64_t nitems)
 {
-    const int64_t want = (int64_t)b->num_cus * b->blocks_per_cu;
+    const int64_t want = (int64_t)b->num_cus * b->blocks_per_cu * 2;
     const int64_t need = (nitems + b->chunk - 1) / b->chunk;
     return (unsigned)std::max<int64_t>(1, std::min(want, need));
 }
@@ -96,26 +97,29 @@ unsigned batch_grid(const miso_batch* b, int64_t nitems)
 int enqueue_scan(miso_batch* b)
 {
     const int64_t ncls = b->cls_prefix.back(), nlane = b->lane_prefix.back();
-    hipLaunchKernelGGL(k_batch_zero, dim3((unsigned)std::min<int64_t>(1024, (b->state_words + 255) / 256)), dim3(256),
-                       0, b->stream, b->d_state, b->state_words);
     hipLaunchKernelGGL(k_batch_classify, dim3(batch_grid(b, ncls)), dim3(256), 0, b->stream,
                        (const BatchJob*)b->d_jobs, (const int*)b->d_group_job, (const int64_t*)b->d_cls_prefix,
-                       b->ngroups, ncls, b->chunk, b->d_mask, b->tickets() + 0);
+                       b->ngroups, ncls, b->chunk, b->d_mask, b->scan_sums(), kTileSums * b->scan.ntiles);
     hipLaunchKernelGGL(k_batch_count, dim3(batch_grid(b, nlane)), dim3(256), 0, b->stream, (const BatchJob*)b->d_jobs,
                        (const int64_t*)b->d_lane_prefix, b->njobs, nlane, b->chunk, (const uint64_t*)b->d_mask,
-                       b->d_counts, b->d_trims, b->scan_sums(), b->scan.shift, b->tickets() + 1);
+                       b->d_counts, b->d_trims, b->scan_sums(), b->scan.shift);
     hipLaunchKernelGGL(k_fe_scan<uint32_t>, dim3((unsigned)b->scan.ntiles), dim3(256), 0, b->stream,
                        (const RowCounts*)b->d_counts, b->R, b->d_voff, b->d_toff, (const uint64_t*)b->scan_sums(),
-                       b->scan.shift, b->scan.ntiles, b->totals(), (uint64_t*)nullptr, ScanMore());
+                       b->scan.shift, b->scan.ntiles, b->totals(), b->h_jobout + 4 * b->njobs, ScanMore());
     hipLaunchKernelGGL(k_batch_job_counts, dim3((unsigned)((b->njobs + 255) / 256)), dim3(256), 0, b->stream,
                        (const BatchJob*)b->d_jobs, b->njobs, b->R, (const uint64_t*)b->d_voff,
-                       (const uint64_t*)b->d_toff, (const uint64_t*)b->totals(), b->d_jobout);
+                       (const uint64_t*)b->d_toff, (const uint64_t*)b->totals(), b->d_jobout, b->h_jobout);
     HIPCALL(hipGetLastError());
-    HIPCALL(hipMemcpyAsync(b->h_jobout, b->d_jobout, 4 * (size_t)b->njobs * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                           b->stream));
-    HIPCALL(hipMemcpyAsync(b->h_jobout + 4 * b->njobs, b->totals(), 2 * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                           b->stream));
     return MISO_OK;
+}
+
+/* blocks of pass 4 for jobs [0, nemit): their items, in XCD order eight times the longest XCD's */
+int64_t emit_items(const miso_batch* b, int64_t nemit)
+{
+    if (b->queue_order != MISO_BATCH_QUEUE_XCD) return b->lane_prefix[nemit];
+    int64_t most = 0;
+    for (int x = 0; x < 8; ++x) most = std::max(most, b->xcd_prefix[x * (b->njobs + 1) + nemit]);
+    return 8 * most;
 }
 
 /* pass 4 for jobs [0, nemit) into the given buffers */
@@ -125,18 +129,19 @@ int enqueue_emit_into(miso_batch* b, int64_t nemit, float* pts, float* nrm, uint
     const int64_t nlane = b->lane_prefix[nemit];
     if (nlane == 0) return MISO_OK;
     const uint64_t* need = nemit < b->njobs ? b->d_jobout + 4 * nemit : b->totals();
-    // the emit queue's tickets start at zero on every emit, also a second emit after one count
-    // (a fill kernel, not a memset node, so that the enqueue can be captured)
     const bool xcd = b->queue_order == MISO_BATCH_QUEUE_XCD;
-    uint64_t* tk = xcd ? b->xcd_tickets() : b->tickets() + 2;
-    hipLaunchKernelGGL(k_batch_zero, dim3(1), dim3(64), 0, b->stream, tk, (int64_t)(xcd ? 8 : 1));
-    unsigned grid = batch_grid(b, nlane);
-    if (xcd) grid = std::max(8u, (grid + 7u) / 8u * 8u);     // every XCD queue has blocks
-    hipLaunchKernelGGL(k_batch_emit, dim3(grid), dim3(256), 0, b->stream, (const BatchJob*)b->d_jobs,
-                       (const int64_t*)b->d_lane_prefix, b->njobs, nlane, b->chunk, (const uint64_t*)b->d_mask,
-                       (const RowCounts*)b->d_counts, (const uint64_t*)b->d_voff, (const uint64_t*)b->d_toff,
-                       need, cap_v, cap_t, pts, nrm, tris, tk,
-                       xcd ? (const int64_t*)b->d_xcd_prefix : (const int64_t*)nullptr, (int)nemit);
+    const int64_t items = emit_items(b, nemit), most = int64_t(1) << 23;   // a launch has fewer than 2^32 threads
+    auto launch = [&](auto kernel) {
+        for (int64_t first = 0; first < items; first += most)
+            hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(most, items - first)), dim3(256), 0, b->stream,
+                               (const BatchJob*)b->d_jobs, (const int64_t*)b->d_lane_prefix, b->njobs, nlane,
+                               (const uint64_t*)b->d_mask, (const RowCounts*)b->d_counts, (const uint64_t*)b->d_voff,
+                               (const uint64_t*)b->d_toff, need, cap_v, cap_t, pts, nrm, tris,
+                               xcd ? (const int64_t*)b->d_xcd_prefix : (const int64_t*)nullptr, (int)nemit, first);
+    };
+    if (b->units == kAllUnit) launch(k_batch_emit<kAllUnit>);
+    else if (b->units == kNoneUnit) launch(k_batch_emit<kNoneUnit>);
+    else launch(k_batch_emit<kSomeUnit>);
     HIPCALL(hipGetLastError());
     return MISO_OK;
 }
@@ -310,8 +315,11 @@ int batch_set_jobs(miso_batch* b, const miso_volume* vols, const float* isovals,
     b->R = R;
     b->mask_words = mw;
     b->scan = plan_scan(R);
-    b->state_words = 13 + kTileSums * b->scan.ntiles;
-    // pass 4's XCD queues: XCD x owns the dispatch indices 8 t + x of each job's row blocks
+    b->state_words = 2 + kTileSums * b->scan.ntiles;
+    int64_t nunit = 0;
+    for (const BatchJob& J : b->jobs) nunit += J.unit;
+    b->units = nunit == njobs ? kAllUnit : (nunit == 0 ? kNoneUnit : kSomeUnit);
+    // pass 4's XCD order: XCD x owns the dispatch indices 8 t + x of each job's row blocks
     b->xcd_prefix.assign(8 * (size_t)(njobs + 1), 0);
     for (int x = 0; x < 8; ++x)
         for (int64_t j = 0; j < njobs; ++j) {
@@ -359,7 +367,7 @@ int batch_init(miso_batch* b, const miso_volume* vols, const float* isovals, int
 }
 
 /* Passes 1-4 as one cooperative launch of k_batch_fused (all blocks resident at once) after a
- * small kernel clears its tickets and scan state (cheaper there than before a grid barrier that
+ * small kernel clears the scan's tile sums (cheaper there than before a grid barrier that
  * every block reaches at once), then the per-job counts and totals to the host. */
 int enqueue_fused(miso_batch* b)
 {
@@ -376,19 +384,16 @@ int enqueue_fused(miso_batch* b)
     int64_t ncls = b->cls_prefix.back(), nlane = b->lane_prefix.back();
     int64_t R = b->R, ntiles = b->scan.ntiles;
     int shift = b->scan.shift;
+    int64_t nitems = emit_items(b, b->njobs);
     uint64_t cap_v = b->cap_v, cap_t = b->cap_t;
     void* args[] = {&jobs,      &group_job, &cls_prefix, &ngroups,     &ncls,  &lane_prefix, &njobs,
                     &nlane,     &chunk,     &b->d_mask,  &b->d_counts, &b->d_trims, &b->d_voff, &b->d_toff,
-                    &b->d_state, &R,        &shift,      &ntiles,      &b->d_jobout, &cap_v, &cap_t,
-                    &b->d_pts,  &b->d_nrm,  &b->d_tris,  &xprefix};
+                    &b->d_state, &R,        &shift,      &ntiles,      &b->d_jobout, &b->h_jobout, &cap_v,
+                    &cap_t,     &b->d_pts,  &b->d_nrm,  &b->d_tris,   &xprefix,  &nitems};
     hipLaunchKernelGGL(k_batch_zero, dim3((unsigned)std::min<int64_t>(1024, (b->state_words + 255) / 256)), dim3(256),
                        0, b->stream, b->d_state, b->state_words);
     HIPCALL(hipLaunchCooperativeKernel((const void*)k_batch_fused, dim3((unsigned)grid), dim3(256), args, 0,
                                        b->stream));
-    HIPCALL(hipMemcpyAsync(b->h_jobout, b->d_jobout, 4 * (size_t)b->njobs * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                           b->stream));
-    HIPCALL(hipMemcpyAsync(b->h_jobout + 4 * b->njobs, b->totals(), 2 * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                           b->stream));
     return MISO_OK;
 }
 

@@ -76,8 +76,7 @@ inline int64_t keep_from_row(const Geom& g) { return g.ny * g.nz - (kKeepVoxels 
  * non-temporal load, so a wavefront step covers 256 voxels = 4 mask words); its 4 sign bits are placed at
  * bit 4 * (lane % 16) and OR-reduced over each 16-lane row with DPP, so lane 16 t + 15 ends up
  * holding mask word t of the step. Rows from keep_row on are read with plain loads instead, so that
- * they stay in the caches for pass 4 (kKeepVoxels). Voxels past nx read as below the isovalue. Rows
- * of at most 256 voxels take one voxel per lane and __ballot instead (fewer instructions per short row).
+ * they stay in the caches for pass 4 (kKeepVoxels). Voxels past nx read as below the isovalue.
  * The voxels are loaded once and classified against n isovalues of the same volume:
  * sink(t, iso, mask) names isovalue t and the mask array it writes (n = 1 for one extraction). */
 template <class Sink>
@@ -88,29 +87,6 @@ __device__ __forceinline__ void fe_classify_block_n(const float* __restrict__ vo
     const int64_t r = blk * kRowsPerBlock + (threadIdx.x >> 6);
     if (r >= g.ny * g.nz) return;
     const float* __restrict__ row = vol + r * g.nx;
-    if (g.W <= 4) {
-        // short rows: one 4-byte voxel per lane and word, the sign bits straight from __ballot
-        float v[4];
-        bool in[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int64_t i = 64 * u + lane;
-            in[u] = u < g.W && i < g.nx;
-            v[u] = in[u] ? row[i] : 0.0f;
-        }
-        for (int t = 0; t < n; ++t) {
-            float iso;
-            uint64_t* mask;
-            sink(t, iso, mask);
-            uint64_t* __restrict__ mrow = mask + r * g.W;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const uint64_t b = __ballot(in[u] && v[u] >= iso);
-                if (lane == 0 && u < g.W) mrow[u] = b;
-            }
-        }
-        return;
-    }
     const int sub = lane & 15;
     constexpr int kSteps = 4;                      // 1024 voxels in flight per wavefront
     for (int64_t c0 = 0; c0 < g.nx; c0 += 256 * kSteps) {
@@ -165,53 +141,82 @@ __device__ __forceinline__ void fe_classify_block_n(const float* __restrict__ vo
     }
 }
 
-/* Rows of at most 256 voxels (W <= 4) in blocks of 4 kShortRows rows: each wavefront loads
- * kShortRows consecutive rows (one voxel per lane and word, as the short-row path above) before
- * classifying them, one memory round trip for all of them. The batch's pass 1 takes this for
- * its short-row jobs, where a work item otherwise moves one short row per wavefront. */
-constexpr int kShortRows = 4;
+/* Rows of at most 256 voxels (W <= 4): a wavefront takes `per` whole rows, at most 16 mask words, all their
+ * voxels in flight at once, one per lane and word; each word's bits come from __ballot, are gathered in
+ * one lane each, and leave in one store. With all 16 words a wavefront moves 4 KB per round trip,
+ * whatever the rows' length, where a row each moved 256 B to 1 KB. */
+constexpr int kShortWords = 16;
+__host__ __device__ __forceinline__ int short_rows_per_wave(int64_t W) { return kShortWords / (int)W; }
+
+/* For one volume: as many of them as leave 4096 wavefronts, four on each of the chip's 1024 SIMDs. Less than
+ * two: a row per wavefront (fe_classify_block_n); a volume so small takes one round trip either way, and
+ * the 16 words' steps cost more than they save (64^3: 2.6 us at a row each, 4.2 at 16, and the whole
+ * call 46.3 us against 49 with one row in these steps). */
+__host__ __device__ __forceinline__ int short_rows_per_wave(const Geom& g)
+{
+    const int64_t spread = g.ny * g.nz / 4096, most = g.W <= 4 ? short_rows_per_wave(g.W) : 1;
+    return (int)(spread < most ? spread : most);
+}
 
 template <class Sink>
 __device__ __forceinline__ void fe_classify_short_rows_n(const float* __restrict__ vol, const Geom& g, int n,
-                                                         Sink sink, int64_t blk)
+                                                         Sink sink, int64_t blk, int per)
 {
     const int lane = lane_id();
-    const int64_t R = g.ny * g.nz;
-    const int64_t r0 = (blk * 4 + (threadIdx.x >> 6)) * kShortRows;
-    if (r0 >= R) return;
-    float v[kShortRows][4];
-    bool in[kShortRows][4];
+    const int W = (int)g.W;
+    const int64_t r0 = (blk * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) * per;
+    const int64_t left = g.ny * g.nz - r0;
+    if (left <= 0) return;
+    const int words = (left < per ? (int)left : per) * W;
+    const int in_last = (int)(g.nx - 64 * (int64_t)(W - 1));          // voxels in a row's last word
+    const uint64_t last_bits = ~0ull >> (64 - in_last);
+    const float* __restrict__ base = vol + r0 * g.nx;
+    float v[kShortWords];
+    int u = 0;                       // word d is word u of its row
 #pragma unroll
-    for (int q = 0; q < kShortRows; ++q) {
-        const int64_t r = r0 + q;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int64_t i = 64 * u + lane;
-            in[q][u] = r < R && u < g.W && i < g.nx;
-            v[q][u] = in[q][u] ? vol[r * g.nx + i] : 0.0f;
-        }
+    for (int d = 0; d < kShortWords; ++d) {
+        v[d] = 0.0f;
+        if (d < words && (u + 1 < W || lane < in_last)) v[d] = base[lane];
+        const bool end = ++u == W;
+        base += end ? g.nx - 64 * (int64_t)(W - 1) : 64;
+        u = end ? 0 : u;
     }
     for (int t = 0; t < n; ++t) {
         float iso;
         uint64_t* mask;
         sink(t, iso, mask);
+        uint64_t word = 0;
+        u = 0;
 #pragma unroll
-        for (int q = 0; q < kShortRows; ++q) {
-            const int64_t r = r0 + q;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const uint64_t b = __ballot(in[q][u] && v[q][u] >= iso);
-                if (lane == 0 && u < g.W && r < R) mask[r * g.W + u] = b;
-            }
+        for (int d = 0; d < kShortWords; ++d) {
+            const bool end = ++u == W;
+            uint64_t b = __ballot(v[d] >= iso);
+            b &= end ? last_bits : ~0ull;
+            word = lane == d ? b : word;
+            u = end ? 0 : u;
         }
+        if (lane < words) mask[r0 * W + lane] = word;
     }
 }
 
 __device__ __forceinline__ void fe_classify_block(const float* __restrict__ vol, const Geom& g, float iso,
                                                   uint64_t* __restrict__ mask, int64_t blk, int64_t keep_row)
 {
-    fe_classify_block_n(vol, g, 1, [&](int, float& is, uint64_t*& m) { is = iso; m = mask; }, blk, keep_row);
+    auto sink = [&](int, float& is, uint64_t*& m) { is = iso; m = mask; };
+    const int per = short_rows_per_wave(g);
+    if (per > 1)
+        fe_classify_short_rows_n(vol, g, 1, sink, blk, per);
+    else
+        fe_classify_block_n(vol, g, 1, sink, blk, keep_row);
 }
+
+/* rows of a pass 1 block: of one volume, and of a batch's job */
+inline int64_t classify_rows(const Geom& g)
+{
+    const int per = short_rows_per_wave(g);
+    return per > 1 ? 4 * per : kRowsPerBlock;
+}
+inline int64_t batch_classify_rows(const Geom& g) { return g.W <= 4 ? 4 * short_rows_per_wave(g.W) : kRowsPerBlock; }
 
 __global__ __launch_bounds__(256) void k_fe_classify(const float* __restrict__ vol, Geom g, float iso,
                                                      uint64_t* __restrict__ mask, int64_t keep_row,

@@ -301,18 +301,15 @@ struct NoRowExtra {
 /* The 4 wavefronts of lane-row block blk (rows 4 rpw blk ..); the wavefront's sums for pass 3. In a slab,
  * rows below emit_lo belong to the slab before it (counts 0, so that the slab's offsets start at 0),
  * and cells from row emit_hi on to the next (triangle counts 0); the vertices of those rows keep their
- * counts, the slab's last cell row names them. split: shown the
- * per-row counts (in one lane per row); true where it has taken them itself (the sums are then 0). */
-struct NoSplit {
-    __device__ bool operator()(uint32_t, uint32_t, int64_t, int64_t, int) const { return false; }
-};
-
-template <class Extra = NoRowExtra, class Split = NoSplit>
+ * counts, the slab's last cell row names them. xy, zt: the row's counts, packed, in the row's first
+ * lane (0 in the others). */
+template <class Extra>
 __device__ __forceinline__ WaveSums fe_count_rows_block(const uint64_t* __restrict__ mask, const Geom& g,
                                                         RowCounts* __restrict__ counts, RowTrim* __restrict__ trims,
-                                                        int64_t blk, Extra extra = Extra(), Split split = Split())
+                                                        int64_t blk, Extra extra, uint32_t& xy, uint32_t& zt)
 {
     WaveSums sums{0u, 0u, 0u};
+    xy = zt = 0u;
     const RowLanes rl = row_lanes(g.W);
     const int64_t r0 = (blk * 4 + wave_in_block()) * rl.rpw;
     if (r0 >= g.ny * g.nz) return sums;
@@ -343,8 +340,8 @@ __device__ __forceinline__ WaveSums fe_count_rows_block(const uint64_t* __restri
     const bool live = has_y && has_z && any != 0ull;
     uint32_t tc = 0u;
     if (__ballot(live) != 0ull) tc = (has_y && has_z) ? word_tri_count(corner_words(L), g, rl.w) : 0u;
-    uint32_t xy = seg_sum((uint32_t)__popcll(xcut) | (uint32_t)__popcll(ycut) << 16, rl);
-    uint32_t zt = seg_sum((uint32_t)__popcll(zcut) | tc << 16, rl);
+    xy = seg_sum((uint32_t)__popcll(xcut) | (uint32_t)__popcll(ycut) << 16, rl);
+    zt = seg_sum((uint32_t)__popcll(zcut) | tc << 16, rl);
     if (r0 + rl.q < g.emit_lo) xy = zt = 0u;
     if (r0 + rl.q >= g.emit_hi) zt &= 0xFFFFu;
     const RowTrim tr = seg_trim(trim, rl, g.nx);
@@ -354,7 +351,6 @@ __device__ __forceinline__ WaveSums fe_count_rows_block(const uint64_t* __restri
     }
     const uint32_t own = extra(L, rl, A, ok, at, false);
     if (!head) xy = zt = 0u;
-    if (split(xy, zt, r0, r0 + rl.q, rl.rpw)) return sums;
     sums.xy = wave_sum_u32(xy);
     sums.zt = wave_sum_u32(zt);
     sums.own = wave_sum_u32(head ? own : 0u);
@@ -382,7 +378,8 @@ __global__ __launch_bounds__(256) void k_fe_count_rows(const uint64_t* __restric
                                                        RowTrim* __restrict__ trims,
                                                        uint64_t* __restrict__ sums, int shift)
 {
-    const WaveSums w = fe_count_rows_block(mask, g, counts, trims, blockIdx.x);
+    uint32_t xy, zt;
+    const WaveSums w = fe_count_rows_block(mask, g, counts, trims, blockIdx.x, NoRowExtra(), xy, zt);
     add_block_sums(w, sums + (block_row(g.W, blockIdx.x) >> shift) * kTileSums);
 }
 

@@ -84,13 +84,15 @@ __global__ __launch_bounds__(256) void k_fe_mc_count_rows(const uint64_t* __rest
                                                           uint64_t* __restrict__ sums, int shift,
                                                           uint32_t* __restrict__ owned)
 {
+    uint32_t xy, zt;
     const WaveSums w = fe_count_rows_block(
         mask, g, counts, trims, blockIdx.x,
         [&](const LaneWords& L, const RowLanes& rl, const WaveRows& A, bool ok, const LaneRow& at, bool empty) {
             const uint32_t cnt = empty ? 0u : mc_owned_row_count(L, g, rl, A, ok, at);
             if (rl.q < A.n && rl.w == 0) row_entry(owned, A, rl.q) = cnt;
             return cnt;
-        });
+        },
+        xy, zt);
     add_block_sums(w, sums + (block_row(g.W, blockIdx.x) >> shift) * kTileSums);
 }
 
