@@ -302,6 +302,23 @@ struct McState {
         return s.launch_scan(more);
     }
 
+    /* Flying Edges pass 4 through the map */
+    template <typename Index>
+    int emit_rows(RowState& s, float iso, float* pts, float* nrm, Index* tris)
+    {
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(s.lane_row_blocks()), dim3(256), 0, s.stream, s.d_vol,
+                               (const uint64_t*)s.d_mask, s.g, iso, (const RowCounts*)s.d_counts,
+                               (const uint64_t*)s.d_voff, (const uint64_t*)s.d_toff, (const Index*)d_map, pts, nrm, tris);
+        };
+        if (s.unit_geometry())
+            launch(k_mc_emit_rows<Index, true>);
+        else
+            launch(k_mc_emit_rows<Index, false>);
+        HIPCALL(hipGetLastError());
+        return MISO_OK;
+    }
+
     template <typename Index>
     int emit(RowState& s, float iso, float* pts, float* nrm, Index* tris, uint64_t nverts)
     {
@@ -321,61 +338,25 @@ struct McState {
             hipLaunchKernelGGL(k_edge_order_perm<Index>, dim3((unsigned)((R + 15) / 16)), dim3(256), 0, s.stream,
                                (const RowCounts*)s.d_counts, (const uint64_t*)s.d_voff, (const uint64_t*)d_xyz,
                                (const uint64_t*)(s.d_totals + 2), R, (Index*)d_map);
-            const uint64_t* no_moff = nullptr;
-            if (s.lane_rows() && s.unit_geometry()) {
-                // Flying Edges pass 4 through the permutation
-                hipLaunchKernelGGL(k_mc_emit_rows<Index>, dim3(s.lane_row_blocks()), dim3(256), 0, s.stream, s.d_vol,
-                                   (const uint64_t*)s.d_mask, s.g, iso, (const RowCounts*)s.d_counts,
-                                   (const uint64_t*)s.d_voff, (const uint64_t*)s.d_toff, (const Index*)d_map, pts,
-                                   nrm, tris);
-                HIPCALL(hipGetLastError());
-                return MISO_OK;
-            }
-            if (!s.lane_rows()) {
-                hipLaunchKernelGGL((k_mc_vertices<Index, true>), dim3(s.row_blocks()), dim3(256), 0, s.stream,
-                                   s.d_vol, (const uint64_t*)s.d_mask, s.g, iso, (const RowCounts*)s.d_counts,
-                                   (const uint64_t*)s.d_voff, no_moff, pts, nrm, (Index*)d_map);
-                HIPCALL(hipGetLastError());
-                hipLaunchKernelGGL(k_mc_triangles<Index>, dim3(s.row_blocks()), dim3(256), 0, s.stream,
-                                   (const uint64_t*)s.d_mask, s.g, (const RowCounts*)s.d_counts,
-                                   (const uint64_t*)s.d_voff, (const uint64_t*)s.d_toff, (const Index*)d_map, tris);
-                HIPCALL(hipGetLastError());
-                return MISO_OK;
-            }
-            if (s.unit_geometry())
-                hipLaunchKernelGGL((k_mc_vertices_rows<Index, true, true>), dim3(s.lane_row_blocks()), dim3(256), 0,
-                                   s.stream, s.d_vol, (const uint64_t*)s.d_mask, s.g, iso,
-                                   (const RowCounts*)s.d_counts, (const uint64_t*)s.d_voff, no_moff, pts, nrm,
-                                   (Index*)d_map);
-            else
-                hipLaunchKernelGGL((k_mc_vertices_rows<Index, false, true>), dim3(s.lane_row_blocks()), dim3(256), 0,
-                                   s.stream, s.d_vol, (const uint64_t*)s.d_mask, s.g, iso,
-                                   (const RowCounts*)s.d_counts, (const uint64_t*)s.d_voff, no_moff, pts, nrm,
-                                   (Index*)d_map);
             HIPCALL(hipGetLastError());
-            hipLaunchKernelGGL(k_mc_triangles_rows<Index>, dim3(s.lane_row_blocks()), dim3(256), 0, s.stream,
+            if (s.lane_rows()) return emit_rows(s, iso, pts, nrm, tris);
+            const uint64_t* no_moff = nullptr;
+            hipLaunchKernelGGL((k_mc_vertices<Index, true>), dim3(s.row_blocks()), dim3(256), 0, s.stream,
+                               s.d_vol, (const uint64_t*)s.d_mask, s.g, iso, (const RowCounts*)s.d_counts,
+                               (const uint64_t*)s.d_voff, no_moff, pts, nrm, (Index*)d_map);
+            HIPCALL(hipGetLastError());
+            hipLaunchKernelGGL(k_mc_triangles<Index>, dim3(s.row_blocks()), dim3(256), 0, s.stream,
                                (const uint64_t*)s.d_mask, s.g, (const RowCounts*)s.d_counts,
                                (const uint64_t*)s.d_voff, (const uint64_t*)s.d_toff, (const Index*)d_map, tris);
             HIPCALL(hipGetLastError());
             return MISO_OK;
         }
         if (s.lane_rows()) {
-            // (the map alone followed by k_mc_emit_rows, as edge order runs, measures the same here:
-            // first-visit ids scatter the Flying Edges emit's vertex writes)
-            if (s.unit_geometry())
-                hipLaunchKernelGGL((k_mc_vertices_rows<Index, true>), dim3(s.lane_row_blocks()), dim3(256), 0, s.stream,
-                                   s.d_vol, (const uint64_t*)s.d_mask, s.g, iso, (const RowCounts*)s.d_counts,
-                                   (const uint64_t*)s.d_voff, (const uint64_t*)d_moff, pts, nrm, (Index*)d_map);
-            else
-                hipLaunchKernelGGL((k_mc_vertices_rows<Index, false>), dim3(s.lane_row_blocks()), dim3(256), 0,
-                                   s.stream, s.d_vol, (const uint64_t*)s.d_mask, s.g, iso, (const RowCounts*)s.d_counts,
-                                   (const uint64_t*)s.d_voff, (const uint64_t*)d_moff, pts, nrm, (Index*)d_map);
+            hipLaunchKernelGGL(k_mc_ids_rows<Index>, dim3(s.lane_row_blocks()), dim3(256), 0, s.stream,
+                               (const uint64_t*)s.d_mask, s.g, (const RowCounts*)s.d_counts, (const uint64_t*)s.d_voff,
+                               (const uint64_t*)s.d_toff, (const uint64_t*)d_moff, (Index*)d_map);
             HIPCALL(hipGetLastError());
-            hipLaunchKernelGGL(k_mc_triangles_rows<Index>, dim3(s.lane_row_blocks()), dim3(256), 0, s.stream,
-                               (const uint64_t*)s.d_mask, s.g, (const RowCounts*)s.d_counts,
-                               (const uint64_t*)s.d_voff, (const uint64_t*)s.d_toff, (const Index*)d_map, tris);
-            HIPCALL(hipGetLastError());
-            return MISO_OK;
+            return emit_rows(s, iso, pts, nrm, tris);
         }
         hipLaunchKernelGGL(k_mc_vertices<Index>, dim3(s.row_blocks()), dim3(256), 0, s.stream, s.d_vol,
                            (const uint64_t*)s.d_mask, s.g, iso, (const RowCounts*)s.d_counts,

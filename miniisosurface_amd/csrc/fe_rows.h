@@ -532,12 +532,14 @@ __device__ __forceinline__ void vertex_yz(const float* __restrict__ v, const Geo
     edge_finish<Unit>(g, axis, i, j, k, w, ga, gb, p, nrm);
 }
 
-/* Flying Edges corner coordinates of the edges from an origin (i,j,k) below the last index of each
- * axis (fe_edge_corners), and the end of edge_point with them: p = a + w (b - a), where b - a is 1 or
- * spacing along the edge and a - a (0, or NaN) across it. */
-template <bool Unit>
+/* Corner coordinates of the edges from an origin (i,j,k) below the last index of each axis, and the end
+ * of edge_point with them: p = a + w (b - a), where b - a is 1 or spacing along the edge and a - a (0, or
+ * NaN) across it. Flying Edges' are fe_edge_corners; Marching Cubes' (Mc) those of the cell that first
+ * visits the edge, one back across it where there is one: that cell's corner plus one spacing
+ * (marchingCubes/util/Image3D.cpp:22-65). With unit spacing and zero origin both are the indices. */
+template <bool Unit, bool Mc = false>
 struct CornerCoords {
-    float A[3];
+    float A[3], P[3];   // along the edge, and (Mc) across it
     __device__ __forceinline__ CornerCoords(const Geom& g, int i, int j, int k)
     {
         if (Unit) {
@@ -546,8 +548,14 @@ struct CornerCoords {
             A[0] = g.org[0] + (float)i * g.sp[0];
             A[1] = g.org[1] + (float)j * g.sp[1];
             A[2] = g.org[2] + (float)(k + (int)g.kofs) * g.sp[2];
+            if (Mc) {
+                P[0] = i > 0 ? g.org[0] + (float)(i - 1) * g.sp[0] + g.sp[0] : A[0];
+                P[1] = j > 0 ? g.org[1] + (float)(j - 1) * g.sp[1] + g.sp[1] : A[1];
+                P[2] = k > 0 ? g.org[2] + (float)(k - 1) * g.sp[2] + g.sp[2] : A[2];
+            }
         }
     }
+    __device__ __forceinline__ float across(int c) const { return Mc && !Unit ? P[c] : A[c]; }
     __device__ __forceinline__ void finish(const Geom& g, int axis, float w, const float ga[3], const float gb[3],
                                            float p[3], float nrm[3]) const
     {
@@ -555,8 +563,10 @@ struct CornerCoords {
         for (int c = 0; c < 3; ++c) {
             if (Unit)
                 p[c] = A[c] + (c == axis ? w : w * 0.0f);
+            else if (c == axis)
+                p[c] = A[c] + w * (A[c] + g.sp[c] - A[c]);
             else
-                p[c] = A[c] + w * ((c == axis ? A[c] + g.sp[c] : A[c]) - A[c]);
+                p[c] = across(c) + w * (across(c) - across(c));
             nrm[c] = ga[c] + w * (gb[c] - ga[c]);
         }
     }
@@ -758,6 +768,7 @@ struct VertexStep {
  * vertices leave in runs of neighbouring ids (1024^3: 1.405 ms against 1.445 ms with word w of all rows
  * before word w + 1, whose gathers share more lines). */
 struct VertexRows {
+    const float* __restrict__ vol;
     const float* __restrict__ row0;   // voxel (0, j0, k0)
     bool rows_inner;                  // every row at least one row from a near face, two from a far one
     uint32_t n, first;                // the wavefront's origins; this lane's first in their order
@@ -766,6 +777,7 @@ struct VertexRows {
 __device__ __forceinline__ VertexRows vertex_rows(const EmitRows& E, const float* __restrict__ vol, const Geom& g)
 {
     VertexRows R;
+    R.vol = vol;
     R.row0 = vol + E.r0 * g.nx;
     R.rows_inner = E.j0 >= 1 && E.j0 + E.rl.rpw <= (int)g.ny - 2 && E.k0 >= 1 && E.k0 <= (int)g.nz - 3;
     const uint32_t cnt = (uint32_t)__popcll(E.origins);
@@ -858,7 +870,7 @@ __device__ __forceinline__ void vertex_store(const VertexStep& V, const EmitRows
         const Around& a = V.a;
         const float ga[3] = {central<Unit>(a.r.x, a.r.z, g.sp[0]), central<Unit>(a.ym.x, a.yp.y, g.sp[1]),
                              central<Unit>(a.zm.x, a.zp.y, g.sp[2])};
-        const CornerCoords<Unit> cc(g, i, V.j, V.k);
+        const CornerCoords<Unit, Map> cc(g, i, V.j, V.k);
         const float num = iso - a.r.y;
         float p[3], nn[3];
         if (V.cut[0]) {
@@ -885,7 +897,17 @@ __device__ __forceinline__ void vertex_store(const VertexStep& V, const EmitRows
         for (int ax = 0; ax < 3; ++ax) {
             if (!V.cut[ax]) continue;
             float p[3], nn[3];
-            fe_edge_point<Unit>(v, g, iso, ax, i, V.j, V.k, p, nn);
+            if (Map && !Unit) {
+                // Marching Cubes' corner coordinates, the general edge_point
+                const CornerCoords<Unit, Map> cc(g, i, V.j, V.k);
+                float A[3] = {cc.across(0), cc.across(1), cc.across(2)};
+                A[ax] = cc.A[ax];
+                float B[3] = {A[0], A[1], A[2]};
+                B[ax] = A[ax] + g.sp[ax];
+                edge_point(R.vol, g, iso, ax, i, V.j, V.k, A, B, p, nn);
+            } else {
+                fe_edge_point<Unit>(v, g, iso, ax, i, V.j, V.k, p, nn);
+            }
             put(V.at[ax], p, nn);
         }
     }
@@ -1011,24 +1033,19 @@ __device__ __forceinline__ void emit_rows_both(const EmitRows& E, EmitRowsLds& S
 }
 
 /* Lane-row block blk. s_case holds kCaseSlots; vertex ids are written less vbias (the first
- * vertex of this volume's output when several volumes share one buffer). With Remap, only the
- * triangles are written, each Flying Edges vertex id replaced by remap[id]. */
-template <typename Index, bool Unit, bool Remap = false>
+ * vertex of this volume's output when several volumes share one buffer). */
+template <typename Index, bool Unit>
 __device__ __forceinline__ void fe_emit_rows_block(const uint64_t* __restrict__ s_case, EmitRowsLds* s_w,
                                                    const float* __restrict__ vol, const uint64_t* __restrict__ mask,
                                                    const Geom& g, float iso, const RowCounts* __restrict__ counts,
                                                    const uint64_t* __restrict__ voff,
                                                    const uint64_t* __restrict__ toff, float* __restrict__ pts,
                                                    float* __restrict__ nrm, Index* __restrict__ tris,
-                                                   uint64_t vbias, int64_t blk, const Index* __restrict__ remap = nullptr)
+                                                   uint64_t vbias, int64_t blk)
 {
     EmitRows E;
     if (!emit_rows_setup(E, s_w, mask, g, counts, voff, toff, blk)) return;
-    EmitRowsLds& S = s_w[E.wv];
-    if (Remap)
-        emit_rows_triangles<Index, true>(E, S, s_case, tris, vbias, remap);
-    else
-        emit_rows_both<Index, Unit, false>(E, S, s_case, vol, g, iso, pts, nrm, tris, vbias, remap);
+    emit_rows_both<Index, Unit, false>(E, s_w[E.wv], s_case, vol, g, iso, pts, nrm, tris, vbias, (const Index*)nullptr);
 }
 
 /* The order in which pass 4's blocks take the rows, across the 8 XCDs. The hardware hands blocks
@@ -1112,10 +1129,9 @@ __global__ __launch_bounds__(256) void k_fe_emit_rows(const float* __restrict__ 
     fe_emit_rows_block<Index, Unit>(s_case, s_w, vol, mask, g, iso, counts, voff, toff, pts, nrm, tris, vbias, blk);
 }
 
-/* Marching Cubes for unit spacing and zero origin, where a Marching Cubes vertex has the bits of
- * the Flying Edges vertex on the same edge: the Flying Edges pass 4 with every vertex written at
- * fe_to_mc[its id] and every triangle's ids read through the same map. */
-template <typename Index>
+/* Marching Cubes: the Flying Edges pass 4 with Marching Cubes' corner coordinates, every vertex written at
+ * fe_to_mc[its Flying Edges id] and every triangle's ids read through the same map. */
+template <typename Index, bool Unit>
 __global__ __launch_bounds__(256) void k_mc_emit_rows(const float* __restrict__ vol,
                                                       const uint64_t* __restrict__ mask, Geom g, float iso,
                                                       const RowCounts* __restrict__ counts,
@@ -1131,25 +1147,7 @@ __global__ __launch_bounds__(256) void k_mc_emit_rows(const float* __restrict__ 
     const int64_t blk = emit_block(blockIdx.x, gridDim.x, g);
     EmitRows E;
     if (!emit_rows_setup(E, s_w, mask, g, counts, voff, toff, blk)) return;
-    emit_rows_both<Index, true, true>(E, s_w[E.wv], s_case, vol, g, iso, pts, nrm, tris, 0, fe_to_mc);
-}
-
-/* Marching Cubes triangles: the Flying Edges triangle stream through the id map. */
-template <typename Index>
-__global__ __launch_bounds__(256) void k_mc_triangles_rows(const uint64_t* __restrict__ mask, Geom g,
-                                                           const RowCounts* __restrict__ counts,
-                                                           const uint64_t* __restrict__ voff,
-                                                           const uint64_t* __restrict__ toff,
-                                                           const Index* __restrict__ fe_to_mc,
-                                                           Index* __restrict__ tris)
-{
-    __shared__ uint64_t s_case[256];
-    __shared__ EmitRowsLds s_w[4];
-    s_case[threadIdx.x] = kCaseSlots.v[threadIdx.x];
-    __syncthreads();
-    const int64_t blk = emit_block(blockIdx.x, gridDim.x, g);
-    fe_emit_rows_block<Index, true, true>(s_case, s_w, nullptr, mask, g, 0.0f, counts, voff, toff, nullptr, nullptr,
-                                          tris, 0, blk, fe_to_mc);
+    emit_rows_both<Index, Unit, true>(E, s_w[E.wv], s_case, vol, g, iso, pts, nrm, tris, 0, fe_to_mc);
 }
 
 }  // namespace miso

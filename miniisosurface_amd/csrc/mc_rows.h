@@ -10,9 +10,8 @@
  *
  *   k_fe_mc_count_rows Flying Edges pass 2 and the owned cut edges per cell row, bit-sliced over
  *                      the 64 cells of a word, in one pass over the mask words
- *   k_mc_vertices_rows owners' points and normals at their Marching Cubes ids, and the map
- *                      from Flying Edges vertex id to Marching Cubes id
- *   k_fe_emit_rows with a map (fe_rows.h) writes the triangles
+ *   k_mc_ids_rows      the map from Flying Edges vertex id to Marching Cubes id
+ *   k_mc_emit_rows     (fe_rows.h) Flying Edges pass 4 through that map
  */
 #ifndef MINIISO_MC_ROWS_H
 #define MINIISO_MC_ROWS_H
@@ -96,16 +95,6 @@ __global__ __launch_bounds__(256) void k_fe_mc_count_rows(const uint64_t* __rest
     add_block_sums(w, sums + (block_row(g.W, blockIdx.x) >> shift) * kTileSums);
 }
 
-constexpr int kMcCellCap = 512;
-constexpr int kMcVertCap = 64 * 12;
-
-struct McRowsLds {
-    uint64_t cut[8][64];
-    uint32_t base[8][64];
-    uint32_t cells[kMcCellCap];
-    uint32_t verts[kMcVertCap];
-};
-
 /* Per case: for each cut edge e, its rank in order of first appearance in the case's triangle
  * list (nibble e, bits 4e .. 4e + 3), and the 12-bit mask of cut edges (bits 48 .. 59). */
 __device__ __forceinline__ uint64_t first_appearance(uint64_t packed)
@@ -122,23 +111,6 @@ __device__ __forceinline__ uint64_t first_appearance(uint64_t packed)
         ++n;
     }
     return pos | (uint64_t)seen << 48;
-}
-
-/* Marching Cubes corner coordinates of the owner cell (marchingCubes/util/Image3D.cpp:22-65):
- * origin + index * spacing, plus one spacing on the far side. */
-__device__ __forceinline__ void mc_corners(const Geom& g, int64_t i, int64_t j, int64_t k, int e, float A[3],
-                                           float B[3])
-{
-    const float X = g.org[0] + (float)i * g.sp[0], Y = g.org[1] + (float)j * g.sp[1];
-    const float Z = g.org[2] + (float)k * g.sp[2];
-    A[0] = edge_dx(e) ? X + g.sp[0] : X;
-    A[1] = edge_dy(e) ? Y + g.sp[1] : Y;
-    A[2] = edge_dz(e) ? Z + g.sp[2] : Z;
-    B[0] = A[0];
-    B[1] = A[1];
-    B[2] = A[2];
-    const int a = edge_axis(e);
-    B[a] = A[a] + g.sp[a];
 }
 
 /* Edge order (the order of util::duplicateRemover, marchingCubes/util/DuplicateRemover.h:34-70:
@@ -169,198 +141,90 @@ __global__ __launch_bounds__(256) void k_edge_order_perm(const RowCounts* __rest
     }
 }
 
-/* EdgeOrder: each owned edge's point goes to fe_to_mc[its Flying Edges id] (an edge-order
- * permutation made beforehand), which this kernel then only reads. */
-template <typename Index, bool Unit, bool EdgeOrder = false>
-__global__ __launch_bounds__(256) void k_mc_vertices_rows(const float* __restrict__ vol,
-                                                          const uint64_t* __restrict__ mask, Geom g, float iso,
-                                                          const RowCounts* __restrict__ counts,
-                                                          const uint64_t* __restrict__ voff,
-                                                          const uint64_t* __restrict__ moff,
-                                                          float* __restrict__ pts, float* __restrict__ nrm,
-                                                          Index* __restrict__ fe_to_mc)
+/* First-visit order: the map from Flying Edges vertex id to Marching Cubes id. Active cells one per lane
+ * in order, as in pass 4's triangles, from the same words and ranks: a scan of the owned edges' counts
+ * gives a cell's first id, the edges' order of first appearance the ids within the cell. Cells off the
+ * near faces own at most the three edges that meet at their far corner (5, 6, 11), whose Flying Edges
+ * ids run on from cell to cell: the stores of 64 lanes are runs. */
+template <typename Index>
+__global__ __launch_bounds__(256) void k_mc_ids_rows(const uint64_t* __restrict__ mask, Geom g,
+                                                     const RowCounts* __restrict__ counts,
+                                                     const uint64_t* __restrict__ voff,
+                                                     const uint64_t* __restrict__ toff,
+                                                     const uint64_t* __restrict__ moff, Index* __restrict__ fe_to_mc)
 {
     __shared__ uint64_t s_first[256];
-    __shared__ McRowsLds s_w[4];
-    s_first[threadIdx.x] = first_appearance(kCaseEdges[threadIdx.x]);
+    __shared__ EmitRowsLds s_w[4];
+    {
+        // by the bits as the mask words give them (make_case_slots)
+        const uint32_t c = threadIdx.x;
+        s_first[c] = first_appearance(kCaseEdges[(c & 0x33) | (c & 0x44) << 1 | (c & 0x88) >> 1]);
+    }
     __syncthreads();
-    const int lane = lane_id();
-    const int wv = wave_in_block();
-    McRowsLds& S = s_w[wv];
-    const RowLanes rl = row_lanes(g.W);
-    const int64_t R = g.ny * g.nz;
-    const int64_t r0 = (emit_block(blockIdx.x, gridDim.x, g) * 4 + wv) * rl.rpw;   // Flying Edges pass 4's order
-    if (r0 >= R) return;
-    const int64_t r = r0 + rl.q;
-    const WaveRows A = wave_rows(g, r0, rl.rpw);
-    const LaneRow at = lane_row(A, rl.q);
-    const bool cells = rl.q < A.n && rl.w < (int)g.W && at.has_y && at.has_z;
-    const LaneWords L = load_lane_words(mask, g, A, rl, cells, true, true);
-    const auto [vb, eb] = word_bits(g, rl.w);
-    const CornerWords C = corner_words(L);
-    const uint64_t act = cells ? active_cells(C, eb) : 0ull;
-    const uint32_t ncell = (uint32_t)__popcll(act);
+    EmitRows E;
+    if (!emit_rows_setup(E, s_w, mask, g, counts, voff, toff, emit_block(blockIdx.x, gridDim.x, g))) return;
+    EmitRowsLds& S = s_w[E.wv];
+    const uint32_t ncell = (uint32_t)__popcll(E.act);
     const uint32_t cincl = wave_incl_scan_u32(ncell);
     const uint32_t ctotal = (uint32_t)__builtin_amdgcn_readlane((int)cincl, 63);
-    if (ctotal == 0) return;
-    const uint64_t v0 = voff[r0];
-    {
-        uint64_t cw[8];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) cw[q] = (L.m[q] ^ shifted(L.m[q], L.n[q])) & eb;
-        cw[4] = (L.m[0] ^ L.m[1]) & vb;
-        cw[5] = (L.m[2] ^ L.m[3]) & vb;
-        cw[6] = (L.m[0] ^ L.m[2]) & vb;
-        cw[7] = (L.m[1] ^ L.m[3]) & vb;
-        uint64_t cb[8] = {v0, v0, v0, v0, v0, v0, v0, v0};
-        if (act) {
-            const int64_t rows[4] = {r, r + 1, r + g.ny, r + g.ny + 1};
-            combo_bases(counts, voff, rows, cb);
-        }
-#pragma unroll
-        for (int q = 0; q < 8; q += 2) {
-            const uint32_t ex = seg_excl_scan((uint32_t)__popcll(cw[q]) | (uint32_t)__popcll(cw[q + 1]) << 16, rl);
-            S.cut[q][lane] = cw[q];
-            S.cut[q + 1][lane] = cw[q + 1];
-            S.base[q][lane] = (uint32_t)(cb[q] - v0) + (ex & 0xFFFFu);
-            S.base[q + 1][lane] = (uint32_t)(cb[q + 1] - v0) + (ex >> 16);
-        }
-    }
-    uint32_t lo[8], hi[8];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        lo[2 * q] = (uint32_t)C.m[q];
-        hi[2 * q] = (uint32_t)(C.m[q] >> 32);
-        lo[2 * q + 1] = (uint32_t)C.s[q];
-        hi[2 * q + 1] = (uint32_t)(C.s[q] >> 32);
-    }
-    const uint32_t clo[8] = {lo[0], lo[1], lo[3], lo[2], lo[4], lo[5], lo[7], lo[6]};
-    const uint32_t chi[8] = {hi[0], hi[1], hi[3], hi[2], hi[4], hi[5], hi[7], hi[6]};
-    const uint32_t cfirst = cincl - ncell;
-    const int64_t k0 = A.k0, j0 = A.j0;
-    uint64_t mid = EdgeOrder ? 0 : moff[r0];   // the wavefront's first Marching Cubes vertex
-    for (uint32_t win = 0; win < ctotal; win += kMcCellCap) {
-        const uint32_t wend = win + kMcCellCap;
-        if (ncell && cfirst < wend && cfirst + ncell > win) {
-            uint32_t p = cfirst;
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                uint32_t a = h ? (uint32_t)(act >> 32) : (uint32_t)act;
-                while (a && p < wend) {
-                    const int b = __builtin_ctz(a);
-                    a &= a - 1;
-                    if (p >= win) {
-                        const uint32_t cs = case_of_half(h ? chi : clo, b);
-                        S.cells[p - win] = (uint32_t)lane | (uint32_t)(b + 32 * h) << 6 | cs << 12;
-                    }
-                    ++p;
-                }
-            }
-        }
+    uint64_t mid = moff[E.r0];
+    for (uint32_t win = 0; win < ctotal; win += kEmitCellCap) {
+        list_bits<kEmitCellCap>(E.act, cincl - ncell, win, E.lane, S.t.cells);
         wave_sync();
-        const uint32_t n = min((uint32_t)kMcCellCap, ctotal - win);
-        // The owned edges of consecutive 64-cell groups collect in S.verts until the next group
-        // might not fit: x-edges from the front, y/z-edges from the back, so that each step of
-        // the flush runs one vertex path on 64 lanes. Entry: window cell | edge << 9 | id << 13,
-        // the id relative to fbase (the first Marching Cubes vertex of the collection).
-        uint32_t fx = 0, fyz = 0;
-        uint64_t fbase = mid;
-        auto vertex_of = [&](uint32_t ve, bool xpath) {
-            const uint32_t cent = S.cells[ve & 511];
-            const int e = (int)((ve >> 9) & 15);
-            const int src = (int)(cent & 63), b = (int)((cent >> 6) & 63);
-            const int q = src >> __builtin_ctz((unsigned)rl.Wp), w = src & (rl.Wp - 1);
-            int64_t jj = j0 + q, kk = k0;
-            while (jj >= g.ny) {
-                jj -= g.ny;
-                ++kk;
-            }
-            const int64_t i = 64 * (int64_t)w + b;
-            float pp[3], nn[3];
-            if (Unit) {
-                // unit spacing, zero origin: the owner's corner coordinates are float(index),
-                // as Flying Edges' are, so the Flying Edges vertex code gives the same bits
-                const int ia = (int)i + edge_dx(e), ja = (int)jj + edge_dy(e), ka = (int)kk + edge_dz(e);
-                const float* __restrict__ v = vol + ((int64_t)ka * g.ny + ja) * g.nx + ia;
-                if (xpath)
-                    vertex_x<true>(v, g, iso, ia, ja, ka, pp, nn);
-                else
-                    vertex_yz<true>(v, g, iso, edge_axis(e), ia, ja, ka, pp, nn);
-            } else {
-                float A[3], B[3];
-                mc_corners(g, i, jj, kk, e, A, B);
-                edge_point(vol, g, iso, edge_axis(e), i + edge_dx(e), jj + edge_dy(e), kk + edge_dz(e), A, B, pp, nn);
-            }
-            // the edge's Flying Edges id, as the triangle pass computes it
-            const int cq = combo_of_edge(e);
-            const int p = b + edge_dx(e);
-            const uint64_t cwq = S.cut[cq][src];
-            const uint64_t below = p == 64 ? cwq : (cwq & ((1ull << p) - 1ull));
-            const uint64_t fe = v0 + S.base[cq][src] + (uint32_t)__popcll(below);
-            const uint64_t id = EdgeOrder ? (uint64_t)fe_to_mc[fe] : fbase + (ve >> 13);
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                pts[3 * id + c] = pp[c];
-                nrm[3 * id + c] = nn[c];
-            }
-            if (!EdgeOrder) fe_to_mc[fe] = (Index)id;
-        };
-        auto flush = [&]() {
-            wave_sync();
-            for (uint32_t v = lane; v < fx; v += 64) vertex_of(S.verts[v], true);
-            for (uint32_t v = lane; v < fyz; v += 64) vertex_of(S.verts[kMcVertCap - 1 - v], false);
-            wave_sync();
-            fx = fyz = 0;
-            fbase = mid;
-        };
-        constexpr uint32_t kXEdges = 0x55u;   // edges 0, 2, 4, 6 run along x
+        const uint32_t n = min((uint32_t)kEmitCellCap, ctotal - win);
         for (uint32_t g0 = 0; g0 < n; g0 += 64) {
-            // one cell per lane: its owned cut edges, in first-appearance order
-            const uint32_t idx = g0 + (uint32_t)lane;
-            uint32_t ent = 0, own = 0;
-            uint64_t order = 0;
-            if (idx < n) {
-                ent = S.cells[idx];
-                const int src = (int)(ent & 63), b = (int)((ent >> 6) & 63);
-                const int q = src >> __builtin_ctz((unsigned)rl.Wp), w = src & (rl.Wp - 1);
-                int64_t jj = j0 + q, kk = k0;
-                while (jj >= g.ny) {
-                    jj -= g.ny;
-                    ++kk;
-                }
-                order = s_first[ent >> 12];
-                own = (uint32_t)(order >> 48) & 0xFFFu & mc_owned_edges(w == 0 && b == 0, jj == 0, kk == 0);
+            const uint32_t idx = g0 + (uint32_t)E.lane;
+            const uint32_t ent = idx < n ? (uint32_t)S.t.cells[idx] : 0u;
+            const uint32_t h2 = ent >> 5, b = ent & 31;
+            uint32_t w[4], t[4], x[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t lo = S.words[q][h2], hi = S.words[q][h2 + 1];
+                w[q] = lo;
+                t[q] = __builtin_amdgcn_alignbit(hi, lo, b);
+                x[q] = lo ^ __builtin_amdgcn_alignbit(hi, lo, 1);
             }
-            const uint32_t no = (uint32_t)__popc(own), nox = (uint32_t)__popc(own & kXEdges);
-            // both counts in one scan (a group has at most 64 * 12 owned edges)
-            const uint32_t inc = wave_incl_scan_u32(no | nox << 16);
-            const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
-            const uint32_t vtot = tot & 0xFFFFu, xtot = tot >> 16;
-            if (fx + fyz + vtot > (uint32_t)kMcVertCap) flush();
-            if (own) {
-                // first-visit rank of an owned edge: owned edges appearing earlier in the cell's
-                // triangles, after the vertices of earlier lanes and groups
-                uint32_t posmask = 0;
-                for (uint32_t o = own; o; o &= o - 1) posmask |= 1u << ((order >> (4 * __builtin_ctz(o))) & 0xF);
-                const uint32_t base = (uint32_t)(mid - fbase) + (inc & 0xFFFFu) - no;
-                uint32_t sx = fx + (inc >> 16) - nox;
-                uint32_t syz = fyz + ((inc & 0xFFFFu) - no) - ((inc >> 16) - nox);
-                for (uint32_t o = own; o; o &= o - 1) {
-                    const int e = __builtin_ctz(o);
-                    const uint32_t p = (uint32_t)(order >> (4 * e)) & 0xF;
-                    const uint32_t rel = base + (uint32_t)__popc(posmask & ((1u << p) - 1u));
-                    const uint32_t ve = idx | (uint32_t)e << 9 | rel << 13;
-                    if ((kXEdges >> e) & 1u)
-                        S.verts[sx++] = ve;
-                    else
-                        S.verts[kMcVertCap - 1 - syz++] = ve;
-                }
+            const uint4 rk = S.rank[h2];
+            const uint32_t cs = (t[0] & 3) | (t[1] & 3) << 2 | (t[2] & 3) << 4 | (t[3] & 3) << 6;
+            const uint64_t order = s_first[cs];
+            const int i = (int)(ent & ((64u << E.wp_log2) - 1u));
+            int j = E.j0 + (int)(ent >> (6 + E.wp_log2));
+            int64_t k = E.k0;
+            while (j >= (int)g.ny) {
+                j -= (int)g.ny;
+                ++k;
             }
-            fx += xtot;
-            fyz += vtot - xtot;
-            mid += vtot;
+            const uint32_t own = idx < n ? (uint32_t)(order >> 48) & 0xFFFu & mc_owned_edges(i == 0, j == 0, k == 0) : 0u;
+            const uint32_t no = (uint32_t)__popc(own);
+            const uint32_t incl = wave_incl_scan_u32(no);
+            uint32_t place = 0;      // bit p: the edge that appears p-th is owned
+            for (uint32_t o = own; o; o &= o - 1) place |= 1u << ((order >> (4 * __builtin_ctz(o))) & 0xF);
+            const uint64_t first = mid + (incl - no);
+            const uint32_t below = bits_below(b);
+            auto cnt = [&](uint32_t bits) { return (uint32_t)__popc(bits & below); };
+            auto put = [&](int e, uint64_t fe) {
+                if (!((own >> e) & 1u)) return;
+                const uint32_t p = (uint32_t)(order >> (4 * e)) & 0xF;
+                fe_to_mc[fe] = (Index)(first + (uint32_t)__popc(place & bits_below(p)));
+            };
+            const uint32_t y0 = (rk.z & 0xFFFFu) + cnt(w[0] ^ w[1]), y1 = (rk.z >> 16) + cnt(w[2] ^ w[3]);
+            const uint32_t z0 = (rk.w & 0xFFFFu) + cnt(w[0] ^ w[2]), z1 = (rk.w >> 16) + cnt(w[1] ^ w[3]);
+            put(6, E.v2 + ((rk.y >> 16) + cnt(x[3])));
+            put(5, E.v2 + (y1 + ((t[2] ^ t[3]) & 1u)));
+            put(11, E.v0 + (z1 + ((t[1] ^ t[3]) & 1u)));
+            if (own & ~((1u << 5) | (1u << 6) | (1u << 11))) {
+                put(0, E.v0 + ((rk.x & 0xFFFFu) + cnt(x[0])));
+                put(2, E.v0 + ((rk.x >> 16) + cnt(x[1])));
+                put(4, E.v2 + ((rk.y & 0xFFFFu) + cnt(x[2])));
+                put(3, E.v0 + y0);
+                put(1, E.v0 + (y0 + ((t[0] ^ t[1]) & 1u)));
+                put(7, E.v2 + y1);
+                put(8, E.v0 + z0);
+                put(9, E.v0 + (z0 + ((t[0] ^ t[2]) & 1u)));
+                put(10, E.v0 + z1);
+            }
+            mid += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
         }
-        flush();
         wave_sync();
     }
 }
