@@ -302,14 +302,16 @@ struct McState {
         return s.launch_scan(more);
     }
 
-    /* Flying Edges pass 4 through the map */
+    /* Flying Edges pass 4 through the map; with need, only if the totals fit */
     template <typename Index>
-    int emit_rows(RowState& s, float iso, float* pts, float* nrm, Index* tris)
+    int emit_rows(RowState& s, float iso, float* pts, float* nrm, Index* tris, const uint64_t* need, uint64_t cap_v,
+                  uint64_t cap_t)
     {
         auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(s.lane_row_blocks()), dim3(256), 0, s.stream, s.d_vol,
                                (const uint64_t*)s.d_mask, s.g, iso, (const RowCounts*)s.d_counts,
-                               (const uint64_t*)s.d_voff, (const uint64_t*)s.d_toff, (const Index*)d_map, pts, nrm, tris);
+                               (const uint64_t*)s.d_voff, (const uint64_t*)s.d_toff, (const Index*)d_map, pts, nrm, tris,
+                               need, cap_v, cap_t);
         };
         if (s.unit_geometry())
             launch(k_mc_emit_rows<Index, true>);
@@ -319,17 +321,21 @@ struct McState {
         return MISO_OK;
     }
 
+    /* need (row kernels only): launched before the totals are known on the host, into buffers and a map for
+     * nverts vertices and cap_t triangles; the kernels write nothing if the totals do not fit */
     template <typename Index>
-    int emit(RowState& s, float iso, float* pts, float* nrm, Index* tris, uint64_t nverts)
+    int emit(RowState& s, float iso, float* pts, float* nrm, Index* tris, uint64_t nverts, const uint64_t* need,
+             uint64_t cap_t)
     {
-        const uint64_t need = (nverts ? nverts : 1) * sizeof(Index);
-        if (need > map_bytes) {
+        const uint64_t bytes = (nverts ? nverts : 1) * sizeof(Index);
+        if (bytes > map_bytes) {
             if (d_map) (void)hipFree(d_map);
             d_map = nullptr;
+            map_bytes = 0;
             uint8_t* p = nullptr;
-            if (int rc = dev_alloc(&p, (size_t)need)) return rc;
+            if (int rc = dev_alloc(&p, (size_t)bytes)) return rc;
             d_map = p;
-            map_bytes = need;
+            map_bytes = bytes;
         }
         if (order == MISO_MC_ORDER_EDGE) {
             // vertices sorted by global edge id: the permutation from pass 3's axis scans,
@@ -337,9 +343,9 @@ struct McState {
             const int64_t R = s.g.ny * s.g.nz;
             hipLaunchKernelGGL(k_edge_order_perm<Index>, dim3((unsigned)((R + 15) / 16)), dim3(256), 0, s.stream,
                                (const RowCounts*)s.d_counts, (const uint64_t*)s.d_voff, (const uint64_t*)d_xyz,
-                               (const uint64_t*)(s.d_totals + 2), R, (Index*)d_map);
+                               (const uint64_t*)(s.d_totals + 2), R, (Index*)d_map, need, nverts, cap_t);
             HIPCALL(hipGetLastError());
-            if (s.lane_rows()) return emit_rows(s, iso, pts, nrm, tris);
+            if (s.lane_rows()) return emit_rows(s, iso, pts, nrm, tris, need, nverts, cap_t);
             const uint64_t* no_moff = nullptr;
             hipLaunchKernelGGL((k_mc_vertices<Index, true>), dim3(s.row_blocks()), dim3(256), 0, s.stream,
                                s.d_vol, (const uint64_t*)s.d_mask, s.g, iso, (const RowCounts*)s.d_counts,
@@ -354,9 +360,9 @@ struct McState {
         if (s.lane_rows()) {
             hipLaunchKernelGGL(k_mc_ids_rows<Index>, dim3(s.lane_row_blocks()), dim3(256), 0, s.stream,
                                (const uint64_t*)s.d_mask, s.g, (const RowCounts*)s.d_counts, (const uint64_t*)s.d_voff,
-                               (const uint64_t*)s.d_toff, (const uint64_t*)d_moff, (Index*)d_map);
+                               (const uint64_t*)s.d_toff, (const uint64_t*)d_moff, (Index*)d_map, need, nverts, cap_t);
             HIPCALL(hipGetLastError());
-            return emit_rows(s, iso, pts, nrm, tris);
+            return emit_rows(s, iso, pts, nrm, tris, need, nverts, cap_t);
         }
         hipLaunchKernelGGL(k_mc_vertices<Index>, dim3(s.row_blocks()), dim3(256), 0, s.stream, s.d_vol,
                            (const uint64_t*)s.d_mask, s.g, iso, (const RowCounts*)s.d_counts,
@@ -369,10 +375,11 @@ struct McState {
         return MISO_OK;
     }
 
-    int launch_emit(RowState& s, float iso, float* pts, float* nrm, void* tris, int index_bits, uint64_t nverts)
+    int launch_emit(RowState& s, float iso, float* pts, float* nrm, void* tris, int index_bits, uint64_t nverts,
+                    const uint64_t* need = nullptr, uint64_t cap_t = 0)
     {
-        if (index_bits == 64) return emit<uint64_t>(s, iso, pts, nrm, (uint64_t*)tris, nverts);
-        return emit<uint32_t>(s, iso, pts, nrm, (uint32_t*)tris, nverts);
+        if (index_bits == 64) return emit<uint64_t>(s, iso, pts, nrm, (uint64_t*)tris, nverts, need, cap_t);
+        return emit<uint32_t>(s, iso, pts, nrm, (uint32_t*)tris, nverts, need, cap_t);
     }
 };
 
@@ -386,6 +393,20 @@ struct MeshBuffers {
     uint64_t nverts = 0, ntris = 0;
     int index_bits = 32;
     bool force64 = false;
+
+    /* triangles that the buffer holds at the current index width */
+    uint64_t cap_t_of() const { return index_bits ? cap_t * (uint64_t)cap_t_bits / (uint64_t)index_bits : 0; }
+
+    /* the totals of a pass 4 launched into the buffers as they are: false, and nothing changed, if they do
+     * not fit them or want the other index width */
+    bool take(uint64_t v, uint64_t t)
+    {
+        const int bits = (force64 || v > 0xFFFFFFFFull) ? 64 : 32;
+        if (v > cap_v || t > cap_t_of() || bits != index_bits) return false;
+        nverts = v;
+        ntris = t;
+        return true;
+    }
 
     int reserve(uint64_t v, uint64_t t)
     {
@@ -511,7 +532,7 @@ int fe_pass_launch(miso_fe* h, int pass, const uint64_t* need = nullptr)
     case 4: {
         const MeshBuffers& o = h->out;
         const bool work = need || o.nverts || o.ntris;
-        const uint64_t cap_t = o.index_bits ? o.cap_t * (uint64_t)o.cap_t_bits / (uint64_t)o.index_bits : 0;
+        const uint64_t cap_t = o.cap_t_of();
         if (work && s.lane_rows()) {
 #define MISO_EMIT_ROWS(IDX, UNIT)                                                                                  \
     hipLaunchKernelGGL((k_fe_emit_rows<IDX, UNIT>), dim3(s.lane_row_blocks()), dim3(256), 0, s.stream, s.d_vol,    \
@@ -632,12 +653,7 @@ extern "C" int miso_fe_run(miso_fe* h)
         // other index width) are the buffers grown and pass 4 run again.
         if (int rc = fe_pass_launch(h, 4, h->st.d_totals)) return rc;
         HIPCALL(hipStreamSynchronize(h->st.stream));
-        const uint64_t v = h->st.h_totals[0], t = h->st.h_totals[1];
-        const int bits = (o.force64 || v > 0xFFFFFFFFull) ? 64 : 32;
-        const uint64_t cap_t = o.cap_t * (uint64_t)o.cap_t_bits / (uint64_t)o.index_bits;
-        if (v <= o.cap_v && t <= cap_t && bits == o.index_bits) {
-            o.nverts = v;
-            o.ntris = t;
+        if (o.take(h->st.h_totals[0], h->st.h_totals[1])) {
             h->done = 4;
             return fe_collect_times(h);
         }
@@ -1081,14 +1097,25 @@ extern "C" int miso_mc_run(miso_mc* h)
     if (int rc = s.launch_classify(h->iso)) return rc;
     if (int rc = h->mc.launch_fe_count(s)) return rc;
     if (int rc = h->mc.launch_scan(s)) return rc;   // FE row offsets too: the rank -> id map layout
-    HIPCALL(hipStreamSynchronize(s.stream));
-    if (int rc = h->out.reserve(s.h_totals[0], s.h_totals[1])) return rc;
-    if (h->out.nverts || h->out.ntris)
-        if (int rc = h->mc.launch_emit(s, h->iso, h->out.d_pts, h->out.d_nrm, h->out.d_tris, h->out.index_bits,
-                                       h->out.nverts))
+    MeshBuffers& o = h->out;
+    bool fits = false;
+    if (s.lane_rows() && o.d_pts && o.d_tris) {
+        // buffers from an earlier run: as miso_fe_run, without a host round trip before pass 4
+        if (int rc = h->mc.launch_emit(s, h->iso, o.d_pts, o.d_nrm, o.d_tris, o.index_bits, o.cap_v, s.d_totals,
+                                       o.cap_t_of()))
             return rc;
-    HIPCALL(hipEventRecord(h->ev[1], s.stream));
-    HIPCALL(hipStreamSynchronize(s.stream));
+        HIPCALL(hipEventRecord(h->ev[1], s.stream));
+        HIPCALL(hipStreamSynchronize(s.stream));
+        fits = o.take(s.h_totals[0], s.h_totals[1]);
+    }
+    if (!fits) {
+        HIPCALL(hipStreamSynchronize(s.stream));
+        if (int rc = o.reserve(s.h_totals[0], s.h_totals[1])) return rc;
+        if (o.nverts || o.ntris)
+            if (int rc = h->mc.launch_emit(s, h->iso, o.d_pts, o.d_nrm, o.d_tris, o.index_bits, o.nverts)) return rc;
+        HIPCALL(hipEventRecord(h->ev[1], s.stream));
+        HIPCALL(hipStreamSynchronize(s.stream));
+    }
     HIPCALL(hipEventElapsedTime(&h->ms, h->ev[0], h->ev[1]));
     h->done = true;
     return MISO_OK;

@@ -625,7 +625,8 @@ struct EmitRows {
  * The row state comes from one lane per row and reaches the others by lane moves: a load that 64
  * lanes make of their row's entry costs the L1 one access per four lanes, 1024^3 about 100 of a
  * wavefront's 1320. */
-__device__ __forceinline__ bool emit_rows_setup(EmitRows& E, EmitRowsLds* s_w, const uint64_t* __restrict__ mask,
+template <class Lds>
+__device__ __forceinline__ bool emit_rows_setup(EmitRows& E, Lds* s_w, const uint64_t* __restrict__ mask,
                                                 const Geom& g, const RowCounts* __restrict__ counts,
                                                 const uint64_t* __restrict__ voff, const uint64_t* __restrict__ toff,
                                                 int64_t blk)
@@ -698,7 +699,7 @@ __device__ __forceinline__ bool emit_rows_setup(EmitRows& E, EmitRowsLds* s_w, c
         lo[q] = base[q] + seg_excl_scan((uint32_t)__popcll(cw[2 * q]) | (uint32_t)__popcll(cw[2 * q + 1]) << 16, rl);
         hi[q] = lo[q] + ((uint32_t)__popc((uint32_t)cw[2 * q]) | (uint32_t)__popc((uint32_t)cw[2 * q + 1]) << 16);
     }
-    EmitRowsLds& S = s_w[E.wv];
+    Lds& S = s_w[E.wv];
     S.rank[2 * E.lane] = uint4{lo[0], lo[1], lo[2], lo[3]};
     S.rank[2 * E.lane + 1] = uint4{hi[0], hi[1], hi[2], hi[3]};
     const uint64_t m[4] = {L.m[0], has_y ? L.m[1] : L.m[0], has_z ? L.m[2] : L.m[0], L.m[3]};
@@ -1138,8 +1139,11 @@ __global__ __launch_bounds__(256) void k_mc_emit_rows(const float* __restrict__ 
                                                       const uint64_t* __restrict__ voff,
                                                       const uint64_t* __restrict__ toff,
                                                       const Index* __restrict__ fe_to_mc, float* __restrict__ pts,
-                                                      float* __restrict__ nrm, Index* __restrict__ tris)
+                                                      float* __restrict__ nrm, Index* __restrict__ tris,
+                                                      const uint64_t* __restrict__ need = nullptr,
+                                                      uint64_t cap_v = 0, uint64_t cap_t = 0)
 {
+    if (need && !output_fits<Index>(need, cap_v, cap_t)) return;   // as k_fe_emit_rows
     __shared__ uint64_t s_case[256];
     __shared__ EmitRowsLds s_w[4];
     s_case[threadIdx.x] = kCaseSlots.v[threadIdx.x];

@@ -124,8 +124,11 @@ __global__ __launch_bounds__(256) void k_edge_order_perm(const RowCounts* __rest
                                                          const uint64_t* __restrict__ voff,
                                                          const uint64_t* __restrict__ xyz,
                                                          const uint64_t* __restrict__ tot, int64_t R,
-                                                         Index* __restrict__ perm)
+                                                         Index* __restrict__ perm,
+                                                         const uint64_t* __restrict__ need = nullptr,
+                                                         uint64_t cap_v = 0, uint64_t cap_t = 0)
 {
+    if (need && !output_fits<Index>(need, cap_v, cap_t)) return;
     const int64_t r = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
     if (r >= R) return;
     const uint32_t l = threadIdx.x & 15;
@@ -141,6 +144,14 @@ __global__ __launch_bounds__(256) void k_edge_order_perm(const RowCounts* __rest
     }
 }
 
+/* LDS of one wavefront of k_mc_ids_rows: as EmitRowsLds. With this alone, not pass 4's whole struct, eight
+ * blocks share a CU. */
+struct McIdsLds {
+    uint4 rank[128];
+    uint32_t words[4][130];
+    uint16_t cells[kEmitCellCap];
+};
+
 /* First-visit order: the map from Flying Edges vertex id to Marching Cubes id. Active cells one per lane
  * in order, as in pass 4's triangles, from the same words and ranks: a scan of the owned edges' counts
  * gives a cell's first id, the edges' order of first appearance the ids within the cell. Cells off the
@@ -151,10 +162,13 @@ __global__ __launch_bounds__(256) void k_mc_ids_rows(const uint64_t* __restrict_
                                                      const RowCounts* __restrict__ counts,
                                                      const uint64_t* __restrict__ voff,
                                                      const uint64_t* __restrict__ toff,
-                                                     const uint64_t* __restrict__ moff, Index* __restrict__ fe_to_mc)
+                                                     const uint64_t* __restrict__ moff, Index* __restrict__ fe_to_mc,
+                                                     const uint64_t* __restrict__ need = nullptr,
+                                                     uint64_t cap_v = 0, uint64_t cap_t = 0)
 {
+    if (need && !output_fits<Index>(need, cap_v, cap_t)) return;
     __shared__ uint64_t s_first[256];
-    __shared__ EmitRowsLds s_w[4];
+    __shared__ McIdsLds s_w[4];
     {
         // by the bits as the mask words give them (make_case_slots)
         const uint32_t c = threadIdx.x;
@@ -163,18 +177,18 @@ __global__ __launch_bounds__(256) void k_mc_ids_rows(const uint64_t* __restrict_
     __syncthreads();
     EmitRows E;
     if (!emit_rows_setup(E, s_w, mask, g, counts, voff, toff, emit_block(blockIdx.x, gridDim.x, g))) return;
-    EmitRowsLds& S = s_w[E.wv];
+    McIdsLds& S = s_w[E.wv];
     const uint32_t ncell = (uint32_t)__popcll(E.act);
     const uint32_t cincl = wave_incl_scan_u32(ncell);
     const uint32_t ctotal = (uint32_t)__builtin_amdgcn_readlane((int)cincl, 63);
     uint64_t mid = moff[E.r0];
     for (uint32_t win = 0; win < ctotal; win += kEmitCellCap) {
-        list_bits<kEmitCellCap>(E.act, cincl - ncell, win, E.lane, S.t.cells);
+        list_bits<kEmitCellCap>(E.act, cincl - ncell, win, E.lane, S.cells);
         wave_sync();
         const uint32_t n = min((uint32_t)kEmitCellCap, ctotal - win);
         for (uint32_t g0 = 0; g0 < n; g0 += 64) {
             const uint32_t idx = g0 + (uint32_t)E.lane;
-            const uint32_t ent = idx < n ? (uint32_t)S.t.cells[idx] : 0u;
+            const uint32_t ent = idx < n ? (uint32_t)S.cells[idx] : 0u;
             const uint32_t h2 = ent >> 5, b = ent & 31;
             uint32_t w[4], t[4], x[4];
 #pragma unroll
