@@ -86,7 +86,7 @@ void destroy_graphs(miso_batch* b)
 }
 
 /* blocks of a persistent kernel (pass 1 or 2): two per tuned block per CU, so that the default of 4 fills
- * the 32 wavefronts a CU holds (256 mixed volumes: 668 us for the batch, 700 with half of them) */
+ * the 32 wavefronts a CU holds (256 mixed volumes, when pass 1 took a third of it more: 668 us for the batch, 700 with half of them) */
 unsigned batch_grid(const miso_batch* b, int64_t nitems)
 {
     const int64_t want = (int64_t)b->num_cus * b->blocks_per_cu * 2;
@@ -298,7 +298,7 @@ int batch_set_jobs(miso_batch* b, const miso_volume* vols, const float* isovals,
         while (e < njobs && e - j < kClassifyGroup && jobs[e].vol == jobs[j].vol && jobs[e].g.nx == g.nx &&
                jobs[e].g.ny == g.ny && jobs[e].g.nz == g.nz)
             ++e;
-        const int64_t per_item = batch_classify_rows(g);
+        const int64_t per_item = classify_rows(g);
         cls.push_back(cls.back() + (g.ny * g.nz + per_item - 1) / per_item);
         grp.push_back((int)e);
         j = e;

@@ -61,8 +61,8 @@ __device__ __forceinline__ int find_job(const int64_t* __restrict__ prefix, int 
 /* The items of block b of nblocks persistent ones: the chunks b, b + nblocks, ... of `chunk` consecutive
  * items each; item i of job j after next(). Every wavefront walks the same items by itself: no barrier,
  * and no queue's counter to wait for. A counter gives out a ticket every 14 ns: pass 1 of 256 mixed volumes
- * (170,000 small items of a row per wavefront, then) took 600 us with tickets and 390 now, and the batch
- * 943 us and 668. */
+ * (170,000 small items of a row per wavefront, then) took 600 us with tickets, 385 without (and several
+ * rows per wavefront), and the batch 943 us and 668. */
 struct ItemWalk {
     const int64_t* __restrict__ prefix;
     int64_t nitems, stride, it, end, i;
@@ -144,8 +144,8 @@ __device__ __forceinline__ void batch_classify_item(const BatchJob* __restrict__
         iso = jobs[j0 + t].iso;
         m = mask + jobs[j0 + t].mask_base;
     };
-    if (J.g.W <= 4)
-        fe_classify_short_rows_n(job_volume(J), J.g, n, sink, blk, short_rows_per_wave(J.g.W));
+    if (J.g.W <= kFlatWords)
+        fe_classify_flat_n(job_volume(J), J.g, n, sink, blk, flat_rows_per_wave(J.g.nx));
     else
         fe_classify_block_n(job_volume(J), J.g, n, sink, blk, INT64_MAX);
 }
@@ -253,7 +253,7 @@ __device__ __forceinline__ void batch_emit_nth(const uint64_t* __restrict__ s_ca
 
 /* Pass 4 for the first nemit jobs, one item per block, from item `first`; writes nothing when their output
  * exceeds the capacity (the host then grows the buffers and runs this pass again). The items' costs
- * differ, and the dispatcher evens them out for nothing: with tickets from a queue, one gyroid 512^3
+ * differ, and the dispatcher evens them out for nothing: with tickets from a queue, one gyroid 256^3
  * volume at 16 isovalues took 1360 us for the batch, now 1080; 12 clients' jobs of one serving step 618, now
  * 505. */
 template <BatchUnits Units>

@@ -1,8 +1,8 @@
 /*
  * fe_kernels.h -- Flying Edges passes 1-4 as HIP kernels for gfx950 (wave64).
  *
- *   k_fe_classify  pass 1a: one wavefront per grid row, coalesced loads, v >= iso through
- *                  __ballot into the 1-bit sign mask (replaces FlyingEdgesAlgorithm.cpp:31-45).
+ *   k_fe_classify  pass 1a: a wavefront per grid row, or for several short ones, coalesced loads,
+ *                  v >= iso into the 1-bit sign mask (replaces FlyingEdgesAlgorithm.cpp:31-45).
  *   k_fe_count     pass 1b + pass 2: from the masks of rows (j,k), (j+1,k), (j,k+1), (j+1,k+1):
  *                  xl/xr trims (cpp:47-65 with isCutEdge :515-554), cut-edge counts per grid
  *                  row and triangle counts per cell row (cpp:72-190) with popcounts.
@@ -141,82 +141,79 @@ __device__ __forceinline__ void fe_classify_block_n(const float* __restrict__ vo
     }
 }
 
-/* Rows of at most 256 voxels (W <= 4): a wavefront takes `per` whole rows, at most 16 mask words, all their
- * voxels in flight at once, one per lane and word; each word's bits come from __ballot, are gathered in
- * one lane each, and leave in one store. With all 16 words a wavefront moves 4 KB per round trip,
- * whatever the rows' length, where a row each moved 256 B to 1 KB. */
-constexpr int kShortWords = 16;
-__host__ __device__ __forceinline__ int short_rows_per_wave(int64_t W) { return kShortWords / (int)W; }
-
-/* For one volume: as many of them as leave 4096 wavefronts, four on each of the chip's 1024 SIMDs. Less than
- * two: a row per wavefront (fe_classify_block_n); a volume so small takes one round trip either way, and
- * the 16 words' steps cost more than they save (64^3: 2.6 us at a row each, 4.2 at 16, and the whole
- * call 46.3 us against 49 with one row in these steps). */
-__host__ __device__ __forceinline__ int short_rows_per_wave(const Geom& g)
-{
-    const int64_t spread = g.ny * g.nz / 4096, most = g.W <= 4 ? short_rows_per_wave(g.W) : 1;
-    return (int)(spread < most ? spread : most);
-}
+/* Short rows (W <= kFlatWords): a wavefront takes `per` whole rows, at most 2048 voxels, which lie one after
+ * the other, and classifies them as one run, eight voxels per lane and step: a byte of sign bits, put in
+ * LDS. A row's words are then cut from the run of bits wherever they start. All steps are in flight at
+ * once, and no lane waits at a row's end: with a row's words loaded one voxel per lane, 16 words a
+ * wavefront, pass 1 of 256 mixed volumes (32 to 256 a side, 1.24 GB) was bound by its instructions and took
+ * 385 us, now 265. 1024 or 4096 voxels a wavefront: the batch 559 and 552 us against 549. Longer rows
+ * (up to 512 or 1024 voxels) gain nothing (400x300x280: 212 us either way), and large volumes of them
+ * lose the streaming loads of the row kernel (512^3: 103 us against 85). */
+constexpr int kFlatWords = 4;
+constexpr int kFlatSteps = 4;
+constexpr int kFlatVoxels = 512 * kFlatSteps;
+__host__ __device__ __forceinline__ int flat_rows_per_wave(int64_t nx) { return kFlatVoxels / (int)nx; }
 
 template <class Sink>
-__device__ __forceinline__ void fe_classify_short_rows_n(const float* __restrict__ vol, const Geom& g, int n,
-                                                         Sink sink, int64_t blk, int per)
+__device__ __forceinline__ void fe_classify_flat_n(const float* __restrict__ vol, const Geom& g, int n, Sink sink,
+                                                   int64_t blk, int per)
 {
-    const int lane = lane_id();
-    const int W = (int)g.W;
-    const int64_t r0 = (blk * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))) * per;
-    const int64_t left = g.ny * g.nz - r0;
+    __shared__ uint32_t s_bits[4][kFlatVoxels / 32 + 4];
+    const int lane = lane_id(), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int64_t r0 = (blk * 4 + wv) * per, left = g.ny * g.nz - r0;
     if (left <= 0) return;
-    const int words = (left < per ? (int)left : per) * W;
-    const int in_last = (int)(g.nx - 64 * (int64_t)(W - 1));          // voxels in a row's last word
-    const uint64_t last_bits = ~0ull >> (64 - in_last);
+    uint32_t* __restrict__ bits = s_bits[wv];
+    const int nx = (int)g.nx, W = (int)g.W, rows = (int)(left < per ? left : per), voxels = rows * nx;
+    const int64_t there = left * g.nx;                  // voxels to the volume's end
     const float* __restrict__ base = vol + r0 * g.nx;
-    float v[kShortWords];
-    int u = 0;                       // word d is word u of its row
+    float v[kFlatSteps][8];
 #pragma unroll
-    for (int d = 0; d < kShortWords; ++d) {
-        v[d] = 0.0f;
-        if (d < words && (u + 1 < W || lane < in_last)) v[d] = base[lane];
-        const bool end = ++u == W;
-        base += end ? g.nx - 64 * (int64_t)(W - 1) : 64;
-        u = end ? 0 : u;
+    for (int u = 0; u < kFlatSteps; ++u) {
+        const int p = 512 * u + 8 * lane;
+        if (512 * u >= voxels) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) v[u][c] = 0.0f;
+        } else if (p + 8 <= there) {
+            const Vox4 a = load_vox<Vox4>(base + p), b = load_vox<Vox4>(base + p + 4);
+            v[u][0] = a.x; v[u][1] = a.y; v[u][2] = a.z; v[u][3] = a.w;
+            v[u][4] = b.x; v[u][5] = b.y; v[u][6] = b.z; v[u][7] = b.w;
+        } else {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) v[u][c] = p + c < there ? base[p + c] : 0.0f;
+        }
     }
     for (int t = 0; t < n; ++t) {
         float iso;
         uint64_t* mask;
         sink(t, iso, mask);
-        uint64_t word = 0;
-        u = 0;
 #pragma unroll
-        for (int d = 0; d < kShortWords; ++d) {
-            const bool end = ++u == W;
-            uint64_t b = __ballot(v[d] >= iso);
-            b &= end ? last_bits : ~0ull;
-            word = lane == d ? b : word;
-            u = end ? 0 : u;
+        for (int u = 0; u < kFlatSteps; ++u) {
+            if (512 * u >= voxels) break;
+            uint32_t byte = 0;
+#pragma unroll
+            for (int c = 7; c >= 0; --c) byte = byte + byte + (uint32_t)(v[u][c] >= iso);
+            reinterpret_cast<uint8_t*>(bits)[64 * u + lane] = (uint8_t)byte;
         }
-        if (lane < words) mask[r0 * W + lane] = word;
+        wave_sync();
+        uint64_t* __restrict__ out = mask + r0 * W;
+        for (int e = lane; e < rows * W; e += 64) {
+            const int q = W == 1 ? e : (W == 2 ? e >> 1 : (W == 3 ? (e * 43691) >> 17 : e >> 2));
+            const int w = e - q * W, at = q * nx + 64 * w, in = nx - 64 * w;      // voxels from the word on
+            const uint32_t* d = bits + (at >> 5);
+            const uint32_t lo = __builtin_amdgcn_alignbit(d[1], d[0], at & 31);
+            const uint32_t hi = __builtin_amdgcn_alignbit(d[2], d[1], at & 31);
+            const uint64_t word = (uint64_t)hi << 32 | lo;
+            out[e] = in < 64 ? word & ((1ull << in) - 1ull) : word;
+        }
+        wave_sync();
     }
 }
 
-__device__ __forceinline__ void fe_classify_block(const float* __restrict__ vol, const Geom& g, float iso,
-                                                  uint64_t* __restrict__ mask, int64_t blk, int64_t keep_row)
-{
-    auto sink = [&](int, float& is, uint64_t*& m) { is = iso; m = mask; };
-    const int per = short_rows_per_wave(g);
-    if (per > 1)
-        fe_classify_short_rows_n(vol, g, 1, sink, blk, per);
-    else
-        fe_classify_block_n(vol, g, 1, sink, blk, keep_row);
-}
-
-/* rows of a pass 1 block: of one volume, and of a batch's job */
+/* rows of a pass 1 block */
 inline int64_t classify_rows(const Geom& g)
 {
-    const int per = short_rows_per_wave(g);
-    return per > 1 ? 4 * per : kRowsPerBlock;
+    return g.W <= kFlatWords ? 4 * flat_rows_per_wave(g.nx) : kRowsPerBlock;
 }
-inline int64_t batch_classify_rows(const Geom& g) { return g.W <= 4 ? 4 * short_rows_per_wave(g.W) : kRowsPerBlock; }
 
 __global__ __launch_bounds__(256) void k_fe_classify(const float* __restrict__ vol, Geom g, float iso,
                                                      uint64_t* __restrict__ mask, int64_t keep_row,
@@ -225,7 +222,11 @@ __global__ __launch_bounds__(256) void k_fe_classify(const float* __restrict__ v
     // pass 2 adds up the tile sums of pass 3: clear them here
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < nsums; t += (int64_t)gridDim.x * blockDim.x)
         sums[t] = 0;
-    fe_classify_block(vol, g, iso, mask, blockIdx.x, keep_row);
+    auto sink = [&](int, float& is, uint64_t*& m) { is = iso; m = mask; };
+    if (g.W <= kFlatWords)
+        fe_classify_flat_n(vol, g, 1, sink, blockIdx.x, flat_rows_per_wave(g.nx));
+    else
+        fe_classify_block_n(vol, g, 1, sink, blockIdx.x, keep_row);
 }
 
 /* ------------------------------------------------------------------ pass 1b + 2: counts */

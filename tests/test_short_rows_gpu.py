@@ -1,6 +1,6 @@
 """GPU: pass 1 where rows are at most 256 voxels and a wavefront takes several -- rows that end on or beside
 a word boundary, one voxel in the last word, row counts that leave the last wavefront some, one or no
-rows, volumes of one row per wavefront and of several -- alone and as jobs of a batch, in every block order
+rows, volumes whose last voxels fill no lane's eight -- alone and as jobs of a batch, in every block order
 and launch, with one geometry or both: bit for bit against the oracle."""
 import numpy as np
 import pytest
