@@ -101,13 +101,96 @@ Geom make_geom(const miso_volume* v)
 
 inline bool has_cells(const Geom& g) { return g.nx >= 2 && g.ny >= 2 && g.nz >= 2; }
 
-/* Shared per-extraction device state: volume, sign masks, row counts, offsets, scan state. */
+/* What a handle without a caller's stream takes from the driver whatever its volume: a stream and a pinned
+ * page for the totals. Making and destroying them took 80 us, as long as everything that a 128^3 volume
+ * needs on the device, so a destroyed handle leaves them, idle, to the next one on its device: at most
+ * kIdleKits per device wait here, the rest are destroyed. Any thread may take or leave one. */
+struct Kit {
+    hipStream_t stream = nullptr;
+    uint64_t* totals = nullptr;
+    int dev = 0;
+};
+constexpr int kIdleKits = 4;
+constexpr size_t kPinnedTotals = 2 * sizeof(uint64_t);
+
+struct IdleKits {
+    std::mutex lock;
+    std::vector<Kit> kits;
+};
+IdleKits& idle_kits()
+{
+    static IdleKits* k = new IdleKits();   // never destroyed: handles may outlive static objects
+    return *k;
+}
+
+void destroy_kit(Kit& k)
+{
+    if (k.totals) (void)hipHostFree(k.totals);
+    if (k.stream) (void)hipStreamDestroy(k.stream);
+    k = Kit();
+}
+
+int take_kit(Kit* out)
+{
+    int dev = 0;
+    HIPCALL(hipGetDevice(&dev));
+    IdleKits& idle = idle_kits();
+    for (;;) {
+        Kit k;
+        {
+            std::lock_guard<std::mutex> hold(idle.lock);
+            for (size_t q = idle.kits.size(); q-- > 0 && !k.stream;)
+                if (idle.kits[q].dev == dev) {
+                    k = idle.kits[q];
+                    idle.kits.erase(idle.kits.begin() + (long)q);
+                }
+        }
+        if (!k.stream) break;
+        if (hipStreamQuery(k.stream) == hipSuccess) {
+            *out = k;
+            return MISO_OK;
+        }
+        (void)hipGetLastError();   // not the stream that was left here (the device was reset): forget it
+    }
+    Kit k;
+    k.dev = dev;
+    // a blocking stream: ordered after work on the null stream (where callers that produce a
+    // device volume without naming a stream usually ran)
+    HIPCALL(hipStreamCreateWithFlags(&k.stream, hipStreamDefault));
+    const hipError_t e = hipHostMalloc((void**)&k.totals, kPinnedTotals, hipHostMallocDefault);
+    if (e != hipSuccess) {
+        k.totals = nullptr;
+        destroy_kit(k);
+        HIPCALL(e);
+    }
+    *out = k;
+    return MISO_OK;
+}
+
+/* the stream's work is done, without an error if `clean` */
+void leave_kit(Kit& k, bool clean)
+{
+    if (clean) {
+        IdleKits& idle = idle_kits();
+        std::lock_guard<std::mutex> hold(idle.lock);
+        int same = 0;
+        for (const Kit& q : idle.kits) same += q.dev == k.dev;
+        if (same < kIdleKits) {
+            idle.kits.push_back(k);
+            k = Kit();
+        }
+    }
+    destroy_kit(k);
+}
+
+/* Shared per-extraction device state: volume, sign masks, row counts, offsets, scan state, in one
+ * allocation (eight took 30 us of a 128^3 call to make and to free). */
 struct RowState {
     Geom g{};
     hipStream_t stream = nullptr;
-    bool own_stream = false;
+    Kit kit;                        // without a caller's stream
     const float* d_vol = nullptr;
-    float* d_vol_own = nullptr;
+    uint8_t* d_all = nullptr;
     uint64_t* d_mask = nullptr;
     RowCounts* d_counts = nullptr;
     RowTrim* d_trims = nullptr;
@@ -123,52 +206,60 @@ struct RowState {
         g = make_geom(v);
         if (user_stream) {
             stream = (hipStream_t)user_stream;
+            HIPCALL(hipHostMalloc((void**)&h_totals, kPinnedTotals, hipHostMallocDefault));
         } else {
-            // a blocking stream: ordered after work on the null stream (where callers that
-            // produce a device volume without naming a stream usually ran)
-            HIPCALL(hipStreamCreateWithFlags(&stream, hipStreamDefault));
-            own_stream = true;
+            if (int rc = take_kit(&kit)) return rc;
+            stream = kit.stream;
+            h_totals = kit.totals;
         }
-        const int64_t N = g.nx * g.ny * g.nz;
-        if (v->on_device || N == 0) {
-            d_vol = v->data;
-        } else {
-            if (int rc = dev_alloc(&d_vol_own, (size_t)N)) return rc;
-            HIPCALL(hipMemcpyAsync(d_vol_own, v->data, (size_t)N * sizeof(float), hipMemcpyHostToDevice, stream));
-            HIPCALL(hipStreamSynchronize(stream));   // the host volume is only borrowed until here
-            d_vol = d_vol_own;
-        }
-        HIPCALL(hipHostMalloc((void**)&h_totals, 2 * sizeof(uint64_t), hipHostMallocDefault));
         h_totals[0] = h_totals[1] = 0;
-        if (!has_cells(g)) return MISO_OK;
+        const int64_t N = g.nx * g.ny * g.nz;
+        const bool copy = !v->on_device && N > 0, cells = has_cells(g);
         const int64_t R = g.ny * g.nz;
-        scan = plan_scan(R);
-        int rc = 0;
-        if ((rc = dev_alloc(&d_mask, (size_t)(R * g.W)))) return rc;
-        if ((rc = dev_alloc(&d_counts, (size_t)R))) return rc;
-        if ((rc = dev_alloc(&d_trims, (size_t)R))) return rc;
-        if ((rc = dev_alloc(&d_voff, (size_t)R))) return rc;
-        if ((rc = dev_alloc(&d_toff, (size_t)R))) return rc;
-        if ((rc = dev_alloc(&d_sums, (size_t)scan.sum_words()))) return rc;
-        if ((rc = dev_alloc(&d_totals, 5))) return rc;
+        scan = cells ? plan_scan(R) : ScanPlan{10, 0};
+        size_t bytes = 0;
+        auto part = [&](size_t count, size_t size) {
+            const size_t at = bytes;
+            bytes += (count * size + 255) & ~size_t(255);
+            return at;
+        };
+        const size_t vol = part(copy ? (size_t)N : 0, sizeof(float));
+        const size_t mask = part(cells ? (size_t)(R * g.W) : 0, sizeof(uint64_t));
+        const size_t counts = part(cells ? (size_t)R : 0, sizeof(RowCounts));
+        const size_t trims = part(cells ? (size_t)R : 0, sizeof(RowTrim));
+        const size_t voff = part(cells ? (size_t)R : 0, sizeof(uint64_t));
+        const size_t toff = part(cells ? (size_t)R : 0, sizeof(uint64_t));
+        const size_t sums = part(cells ? (size_t)scan.sum_words() : 0, sizeof(uint64_t));
+        const size_t totals = part(cells ? 5 : 0, sizeof(uint64_t));
+        if (bytes)
+            if (int rc = dev_alloc(&d_all, bytes)) return rc;
+        d_vol = v->data;
+        if (copy) {
+            HIPCALL(hipMemcpyAsync(d_all + vol, v->data, (size_t)N * sizeof(float), hipMemcpyHostToDevice, stream));
+            HIPCALL(hipStreamSynchronize(stream));   // the host volume is only borrowed until here
+            d_vol = reinterpret_cast<const float*>(d_all + vol);
+        }
+        if (!cells) return MISO_OK;
+        d_mask = reinterpret_cast<uint64_t*>(d_all + mask);
+        d_counts = reinterpret_cast<RowCounts*>(d_all + counts);
+        d_trims = reinterpret_cast<RowTrim*>(d_all + trims);
+        d_voff = reinterpret_cast<uint64_t*>(d_all + voff);
+        d_toff = reinterpret_cast<uint64_t*>(d_all + toff);
+        d_sums = reinterpret_cast<uint64_t*>(d_all + sums);
+        d_totals = reinterpret_cast<uint64_t*>(d_all + totals);
         return MISO_OK;
     }
 
-
     void release()
     {
-        if (stream) (void)hipStreamSynchronize(stream);
-        dev_free(d_vol_own);
-        dev_free(d_mask);
-        dev_free(d_counts);
-        dev_free(d_trims);
-        dev_free(d_voff);
-        dev_free(d_toff);
-        dev_free(d_sums);
-        dev_free(d_totals);
-        if (h_totals) (void)hipHostFree(h_totals);
+        bool clean = true;
+        if (stream) clean = hipStreamSynchronize(stream) == hipSuccess;
+        dev_free(d_all);
+        if (kit.stream)
+            leave_kit(kit, clean);
+        else if (h_totals)
+            (void)hipHostFree(h_totals);
         h_totals = nullptr;
-        if (own_stream && stream) (void)hipStreamDestroy(stream);
         stream = nullptr;
     }
 
@@ -415,9 +506,10 @@ struct MeshBuffers {
         index_bits = (force64 || v > 0xFFFFFFFFull) ? 64 : 32;
         if (v > cap_v || !d_pts) {
             dev_free(d_pts);
-            dev_free(d_nrm);
-            if (int rc = dev_alloc(&d_pts, (size_t)(3 * v))) return rc;
-            if (int rc = dev_alloc(&d_nrm, (size_t)(3 * v))) return rc;
+            d_nrm = nullptr;
+            const size_t n = ((size_t)(3 * v) + 63) & ~size_t(63);   // both in one allocation
+            if (int rc = dev_alloc(&d_pts, 2 * n)) return rc;
+            d_nrm = d_pts + n;
             cap_v = v;
         }
         const uint64_t need = 3 * t * (uint64_t)(index_bits / 8);
@@ -436,7 +528,7 @@ struct MeshBuffers {
     void release()
     {
         dev_free(d_pts);
-        dev_free(d_nrm);
+        d_nrm = nullptr;
         if (d_tris) (void)hipFree(d_tris);
         d_tris = nullptr;
     }
