@@ -118,6 +118,7 @@ __device__ __forceinline__ uint32_t dpp_u32(uint32_t v)
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, Ctrl, RowMask, 0xF, true);
 }
 constexpr int kDppRowShr1 = 0x111, kDppRowShr2 = 0x112, kDppRowShr4 = 0x114, kDppRowShr8 = 0x118;
+constexpr int kDppRowShl1 = 0x101, kDppRowShl2 = 0x102, kDppRowShl4 = 0x104, kDppRowShl8 = 0x108;   // from lane i + o
 constexpr int kDppWaveShl1 = 0x130;   // lane l takes lane l + 1's value, the last lane 0
 constexpr int kDppRowBcast15 = 0x142, kDppRowBcast31 = 0x143;
 

@@ -155,25 +155,38 @@ __device__ __forceinline__ uint32_t seg_excl_scan(uint32_t v, const RowLanes& rl
     return incl - v - seg_before(incl, rl);
 }
 
-/* the row's total, in every lane of the row */
-__device__ __forceinline__ uint32_t seg_sum(uint32_t v, const RowLanes& rl)
+/* the row's total, in every lane of the row; all: the wavefront's */
+__device__ __forceinline__ uint32_t seg_sum(uint32_t v, const RowLanes& rl, uint32_t& all)
 {
     const uint32_t incl = wave_incl_scan_u32(v);
+    all = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
     return (uint32_t)__shfl((int)incl, lane_id() - rl.w + rl.Wp - 1) - seg_before(incl, rl);
 }
 
-/* The row's xl and xr of pass 1, in every lane of the row, from the lanes' trim words: the row's first and
- * last lanes with a bit are found in the ballot. nx and 0 for a row without one. */
-__device__ __forceinline__ RowTrim seg_trim(uint64_t trim, const RowLanes& rl, int64_t nx)
+/* the larger of each 16-bit half */
+__device__ __forceinline__ uint32_t max_halves(uint32_t a, uint32_t b)
 {
-    const int head = lane_id() - rl.w;
-    const uint64_t all = __ballot(trim != 0ull) >> head;
-    const uint64_t lanes = rl.Wp == 64 ? all : all & ((1ull << rl.Wp) - 1ull);
-    const uint32_t lo = trim ? (uint32_t)(64 * rl.w + __builtin_ctzll(trim)) : 0u;
-    const uint32_t hi = trim ? (uint32_t)(64 * rl.w + 64 - __builtin_clzll(trim)) : 0u;
-    const uint32_t first = (uint32_t)__shfl((int)lo, head + (lanes ? __builtin_ctzll(lanes) : 0));
-    const uint32_t last = (uint32_t)__shfl((int)hi, head + (lanes ? 63 - __builtin_clzll(lanes) : 0));
-    return lanes ? RowTrim{first, last} : RowTrim{(uint32_t)nx, 0u};
+    typedef unsigned short Pair __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t,
+                              __builtin_elementwise_max(__builtin_bit_cast(Pair, a), __builtin_bit_cast(Pair, b)));
+}
+
+/* The row's xl and xr of pass 1, in the row's first lane, from the 32-bit halves of the lanes' trim words:
+ * a lane's first bit, counted down from 4096, and its last one, a half each, and the maximum of both over
+ * the row's lanes, to which a lane's window has grown after log2(Wp) moves. nx and 0 for a row without a
+ * bit. */
+__device__ __forceinline__ RowTrim seg_trim(uint32_t lo, uint32_t hi, const RowLanes& rl, int64_t nx)
+{
+    const uint32_t first = lo ? (uint32_t)__builtin_ctz(lo) : 32u + (uint32_t)__builtin_ctz(hi);
+    const uint32_t last = hi ? 64u - (uint32_t)__builtin_clz(hi) : 32u - (uint32_t)__builtin_clz(lo);
+    uint32_t key = (lo | hi) ? (4096u - 64u * (uint32_t)rl.w - first) << 16 | (64u * (uint32_t)rl.w + last) : 0u;
+    if (rl.Wp > 1) key = max_halves(key, dpp_u32<kDppRowShl1>(key));
+    if (rl.Wp > 2) key = max_halves(key, dpp_u32<kDppRowShl2>(key));
+    if (rl.Wp > 4) key = max_halves(key, dpp_u32<kDppRowShl4>(key));
+    if (rl.Wp > 8) key = max_halves(key, dpp_u32<kDppRowShl8>(key));
+    if (rl.Wp > 16) key = max_halves(key, (uint32_t)__shfl((int)key, (lane_id() + 16) & 63));
+    if (rl.Wp > 32) key = max_halves(key, (uint32_t)__shfl((int)key, (lane_id() + 32) & 63));
+    return key ? RowTrim{4096u - (key >> 16), key & 0xFFFFu} : RowTrim{(uint32_t)nx, 0u};
 }
 
 /* Sign-mask words around lane (row r, word w): rows (j,k) (j+1,k) (j,k+1) (j+1,k+1). n holds the
@@ -258,40 +271,53 @@ __device__ __forceinline__ uint64_t active_cells(const LaneWords& L, uint64_t eb
  * Corners and x-faces at x = i + 1 are those at x = i of the next cell, so that over the row they count
  * twice but at its two ends: V = sum over the four rows of 2 P - (first voxel) - (last voxel), and the
  * x-faces likewise, which takes one popcount for two. Bits past the row are 0, and no x-pair, ring or
- * inner face has one there. Pass 2 is bound by its vector instructions; at 1024^3 176 -> 160 us with
- * this in the place of every corner and face masked and counted, and with 32-bit lane arithmetic. */
-__device__ __forceinline__ uint32_t word_tri_count(const CornerWords& C, const Geom& g, int w)
+ * inner face has one there. Word halves, so that three-operand logic takes one instruction. */
+__device__ __forceinline__ uint32_t word_tri_count(const LaneWords& L, const Geom& g, int w)
 {
-    const uint64_t p0 = C.m[0] & C.s[0], p1 = C.m[1] & C.s[1], p2 = C.m[2] & C.s[2], p3 = C.m[3] & C.s[3];
-    const uint64_t f01 = p0 & p1, f23 = p2 & p3;
-    const uint64_t xface = C.m[0] & C.m[1] & C.m[2] & C.m[3];
-    const uint32_t P = (uint32_t)__popcll(C.m[0]) + (uint32_t)__popcll(C.m[1]) + (uint32_t)__popcll(C.m[2]) +
-                       (uint32_t)__popcll(C.m[3]);
-    const uint32_t F = (uint32_t)__popcll(f01) + (uint32_t)__popcll(f23) + (uint32_t)__popcll(p0 & p2) +
-                       (uint32_t)__popcll(p1 & p3);
-    // body diagonals: both ends of v0-v6, v1-v7, v2-v4, v3-v5 (rows 0 and 3, 1 and 2)
-    const uint64_t d0 = C.m[0] & C.s[3], d1 = C.s[0] & C.m[3], d2 = C.s[1] & C.m[2], d3 = C.m[1] & C.s[2];
-    const uint64_t ring = (((~(C.m[0] | C.s[3]) & d1) | (~(C.s[0] | C.m[3]) & d0)) & (d2 & d3)) |
-                          (((~(C.s[1] | C.m[2]) & d3) | (~(C.m[1] | C.s[2]) & d2)) & (d0 & d1));
-    // the row's first and last voxels, one bit per row
+    uint32_t P = 0, F = 0, A = 0, Q = 0;       // corners, faces, x-faces and rings, full cells
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        uint32_t m[4], s[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t lo = (uint32_t)L.m[q], hi = (uint32_t)(L.m[q] >> 32);
+            m[q] = h ? hi : lo;
+            s[q] = h ? __builtin_amdgcn_alignbit(L.n[q], hi, 1) : __builtin_amdgcn_alignbit(hi, lo, 1);
+            P += (uint32_t)__popc(m[q]);
+        }
+        const uint32_t p0 = m[0] & s[0], p1 = m[1] & s[1], p2 = m[2] & s[2], p3 = m[3] & s[3];
+        const uint32_t f01 = p0 & p1, f23 = p2 & p3;
+        F += (uint32_t)__popc(f01);
+        F += (uint32_t)__popc(f23);
+        F += (uint32_t)__popc(p0 & p2);
+        F += (uint32_t)__popc(p1 & p3);
+        A += (uint32_t)__popc(m[0] & m[1] & m[2] & m[3]);
+        Q += (uint32_t)__popc(f01 & f23);
+        // rings about v0-v6 or v1-v7 (rows 0 and 3), about v2-v4 or v3-v5 (rows 1 and 2): the rows' two diagonals
+        // have equal ends each and differ, the other two rows' four corners are set
+        const uint32_t u = ~(m[0] ^ s[3]) & ~(s[0] ^ m[3]) & (m[0] ^ s[0]);
+        const uint32_t v = ~(m[1] ^ s[2]) & ~(s[1] ^ m[2]) & (m[1] ^ s[1]);
+        A += (uint32_t)__popc(p1 & p2 & u);
+        A += (uint32_t)__popc(p0 & p3 & v);
+    }
+    // the row's first voxels (bits 0 .. 3) and last ones (4 .. 7), a bit per row
     const int last = (int)g.W - 1, top = (int)(g.nx - 64 * (int64_t)last) - 1;
     uint32_t lo = 0, hi = 0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        lo |= ((uint32_t)C.m[q] & 1u) << q;
-        hi |= ((uint32_t)(C.m[q] >> top) & 1u) << q;
+        lo |= ((uint32_t)L.m[q] & 1u) << q;
+        hi |= ((top & 32 ? (uint32_t)(L.m[q] >> 32) : (uint32_t)L.m[q]) >> (top & 31)) << (4 + q);
     }
-    lo = w == 0 ? lo : 0u;
-    hi = w == last ? hi : 0u;
-    const uint32_t ends = (uint32_t)__popc(lo) + (uint32_t)__popc(hi), xends = (lo == 15u) + (hi == 15u);
-    return 2 * (P - F + xends) - ends -
-           4 * ((uint32_t)__popcll(xface) - (uint32_t)__popcll(f01 & f23) + (uint32_t)__popcll(ring));
+    const uint32_t e = (w == 0 ? lo : 0u) | (w == last ? hi : 0u);
+    const uint32_t xends = (uint32_t)((e & 15u) == 15u) + (uint32_t)(e >= 0xF0u);
+    return 2 * (P - F + xends) - (uint32_t)__popc(e) - 4 * (A - Q);
 }
 
 /* ------------------------------------------------------------------ pass 1b + 2 */
 /* per-row count beside these (none here; first-visit Marching Cubes adds its owned-edge counts,
  * k_fe_mc_count_rows): called by every lane with its words and row, and `empty` when every word the wavefront loaded is zero; the row's count, in every lane of the row */
 struct NoRowExtra {
+    static constexpr bool kCounts = false;
     __device__ uint32_t operator()(const LaneWords&, const RowLanes&, const WaveRows&, bool, const LaneRow&, bool) const
     {
         return 0u;
@@ -318,9 +344,14 @@ __device__ __forceinline__ WaveSums fe_count_rows_block(const uint64_t* __restri
     const LaneRow at = lane_row(A, rl.q);
     const bool has_y = at.has_y, has_z = at.has_z;
     const LaneWords L = load_lane_words(mask, g, A, rl, ok, has_y, has_z);
-    // the words and bit 0 of the next words (corner i + 1 of bit 63)
-    const uint64_t any = L.m[0] | L.m[1] | L.m[2] | L.m[3] | (uint64_t)(L.n[0] | L.n[1] | L.n[2] | L.n[3]);
-    if (__ballot(any != 0ull) == 0ull) {
+    uint32_t lo[4], hi[4], any = L.n[0] | L.n[1] | L.n[2] | L.n[3];   // bit 0 of the next words: corner i + 1 of bit 63
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        lo[q] = (uint32_t)L.m[q];
+        hi[q] = (uint32_t)(L.m[q] >> 32);
+        any |= lo[q] | hi[q];
+    }
+    if (__ballot(any != 0u) == 0ull) {
         // every voxel the wavefront's rows see is below the isovalue (most wavefronts at a
         // sparse, high isovalue): no cut edge, no triangle, an empty trim
         if (head) {
@@ -330,30 +361,39 @@ __device__ __forceinline__ WaveSums fe_count_rows_block(const uint64_t* __restri
         extra(L, rl, A, ok, at, true);
         return sums;
     }
-    const auto [vb, eb] = word_bits(g, rl.w);
-    const uint64_t xcut = (L.m[0] ^ shifted(L.m[0], L.n[0])) & eb;
-    const uint64_t ycut = has_y ? ((L.m[0] ^ L.m[1]) & vb) : 0;
-    const uint64_t zcut = has_z ? ((L.m[0] ^ L.m[2]) & vb) : 0;
-    const uint64_t trim = (xcut | ycut | zcut) & eb;
-    // word_tri_count is 0 where every corner of the lane's cells is below the isovalue (`any`
-    // zero); a wavefront with only such lanes skips it
-    const bool live = has_y && has_z && any != 0ull;
-    uint32_t tc = 0u;
-    if (__ballot(live) != 0ull) tc = (has_y && has_z) ? word_tri_count(corner_words(L), g, rl.w) : 0u;
-    xy = seg_sum((uint32_t)__popcll(xcut) | (uint32_t)__popcll(ycut) << 16, rl);
-    zt = seg_sum((uint32_t)__popcll(zcut) | tc << 16, rl);
-    if (r0 + rl.q < g.emit_lo) xy = zt = 0u;
-    if (r0 + rl.q >= g.emit_hi) zt &= 0xFFFFu;
-    const RowTrim tr = seg_trim(trim, rl, g.nx);
+    const uint64_t eb = word_bits(g, rl.w).eb;
+    const uint32_t e[2] = {(uint32_t)eb, (uint32_t)(eb >> 32)};
+    const uint32_t ym = has_y ? ~0u : 0u, zm = has_z ? ~0u : 0u;
+    const uint32_t next[2] = {__builtin_amdgcn_alignbit(hi[0], lo[0], 1), __builtin_amdgcn_alignbit(L.n[0], hi[0], 1)};
+    uint32_t nx = 0, ny = 0, nz = 0, trim[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const uint32_t* m = h ? hi : lo;
+        const uint32_t x = (m[0] ^ next[h]) & e[h], y = (m[0] ^ m[1]) & ym, z = (m[0] ^ m[2]) & zm;
+        nx += (uint32_t)__popc(x);
+        ny += (uint32_t)__popc(y);
+        nz += (uint32_t)__popc(z);
+        trim[h] = x | ((y | z) & e[h]);
+    }
+    const uint32_t tc = word_tri_count(L, g, rl.w) & ym & zm;
+    uint32_t all_xy, all_zt;
+    xy = seg_sum(nx | ny << 16, rl, all_xy);
+    zt = seg_sum(nz | tc << 16, rl, all_zt);
+    const bool whole = r0 >= g.emit_lo && r0 + rl.rpw <= g.emit_hi;   // no row of another slab
+    if (!whole) {
+        if (r0 + rl.q < g.emit_lo) xy = zt = 0u;
+        if (r0 + rl.q >= g.emit_hi) zt &= 0xFFFFu;
+    }
+    const RowTrim tr = seg_trim(trim[0], trim[1], rl, g.nx);
     if (head) {
         row_entry(counts, A, rl.q) = RowCounts{xy & 0xFFFFu, xy >> 16, zt & 0xFFFFu, zt >> 16};
         row_entry(trims, A, rl.q) = tr;
     }
     const uint32_t own = extra(L, rl, A, ok, at, false);
     if (!head) xy = zt = 0u;
-    sums.xy = wave_sum_u32(xy);
-    sums.zt = wave_sum_u32(zt);
-    sums.own = wave_sum_u32(head ? own : 0u);
+    sums.xy = whole ? all_xy : wave_sum_u32(xy);
+    sums.zt = whole ? all_zt : wave_sum_u32(zt);
+    if (Extra::kCounts) sums.own = wave_sum_u32(head ? own : 0u);
     return sums;
 }
 

@@ -72,8 +72,23 @@ __device__ __forceinline__ uint32_t mc_owned_row_count(const LaneWords& L, const
         if (need_i) own &= first_cell;
         cnt += (uint32_t)__popcll(cut & own);
     }
-    return seg_sum(cnt, rl);
+    uint32_t all;
+    return seg_sum(cnt, rl, all);
 }
+
+/* the owned-edge counts beside pass 2's (NoRowExtra) */
+struct OwnedEdges {
+    static constexpr bool kCounts = true;
+    const Geom& g;
+    uint32_t* __restrict__ owned;
+    __device__ uint32_t operator()(const LaneWords& L, const RowLanes& rl, const WaveRows& A, bool ok, const LaneRow& at,
+                                   bool empty) const
+    {
+        const uint32_t cnt = empty ? 0u : mc_owned_row_count(L, g, rl, A, ok, at);
+        if (rl.q < A.n && rl.w == 0) row_entry(owned, A, rl.q) = cnt;
+        return cnt;
+    }
+};
 
 /* Flying Edges pass 2 (k_fe_count_rows) and the first-visit owned-edge counts per cell row in
  * one pass over the mask words, each row's words loaded once. */
@@ -84,14 +99,7 @@ __global__ __launch_bounds__(256) void k_fe_mc_count_rows(const uint64_t* __rest
                                                           uint32_t* __restrict__ owned)
 {
     uint32_t xy, zt;
-    const WaveSums w = fe_count_rows_block(
-        mask, g, counts, trims, blockIdx.x,
-        [&](const LaneWords& L, const RowLanes& rl, const WaveRows& A, bool ok, const LaneRow& at, bool empty) {
-            const uint32_t cnt = empty ? 0u : mc_owned_row_count(L, g, rl, A, ok, at);
-            if (rl.q < A.n && rl.w == 0) row_entry(owned, A, rl.q) = cnt;
-            return cnt;
-        },
-        xy, zt);
+    const WaveSums w = fe_count_rows_block(mask, g, counts, trims, blockIdx.x, OwnedEdges{g, owned}, xy, zt);
     add_block_sums(w, sums + (block_row(g.W, blockIdx.x) >> shift) * kTileSums);
 }
 
