@@ -184,8 +184,8 @@ int miso_batch_job_output(const miso_batch* b, int64_t job, const float** points
                           const uint32_t** triangles);
 /* host copy of one job's mesh, triangles widened to 64-bit (util::TriangleMesh's size_t) */
 int miso_batch_copy_out(miso_batch* b, int64_t job, float* points, float* normals, uint64_t* triangles);
-/* launch shape of the persistent kernels, passes 1 and 2 (and all of a fused launch): pairs of blocks per CU
- * (blocks, in a fused launch), and the consecutive work items a block takes at a time */
+/* launch shape: the blocks per CU of a fused launch, and the consecutive work items a block takes at a time
+ * in pass 2 (in passes 1 and 2 of a fused launch) */
 int miso_batch_set_tuning(miso_batch* b, int blocks_per_cu, int chunk);
 int miso_batch_get_tuning(const miso_batch* b, int* blocks_per_cu, int* chunk);
 /* The order of pass 4's work, a row block of one job per workgroup. DISPATCH (the default): the jobs'

@@ -85,24 +85,23 @@ void destroy_graphs(miso_batch* b)
     b->g_scan = b->g_emit = b->g_all = nullptr;
 }
 
-/* blocks of a persistent kernel (pass 1 or 2): two per tuned block per CU, so that the default of 4 fills
- * the 32 wavefronts a CU holds (256 mixed volumes, when pass 1 took a third of it more: 668 us for the batch, 700 with half of them) */
-unsigned batch_grid(const miso_batch* b, int64_t nitems)
-{
-    const int64_t want = (int64_t)b->num_cus * b->blocks_per_cu * 2;
-    const int64_t need = (nitems + b->chunk - 1) / b->chunk;
-    return (unsigned)std::max<int64_t>(1, std::min(want, need));
-}
+/* blocks of 256 threads per launch: a launch has fewer than 2^32 threads */
+constexpr int64_t kMostBlocks = int64_t(1) << 23;
 
 int enqueue_scan(miso_batch* b)
 {
     const int64_t ncls = b->cls_prefix.back(), nlane = b->lane_prefix.back();
-    hipLaunchKernelGGL(k_batch_classify, dim3(batch_grid(b, ncls)), dim3(256), 0, b->stream,
-                       (const BatchJob*)b->d_jobs, (const int*)b->d_group_job, (const int64_t*)b->d_cls_prefix,
-                       b->ngroups, ncls, b->chunk, b->d_mask, b->scan_sums(), kTileSums * b->scan.ntiles);
-    hipLaunchKernelGGL(k_batch_count, dim3(batch_grid(b, nlane)), dim3(256), 0, b->stream, (const BatchJob*)b->d_jobs,
-                       (const int64_t*)b->d_lane_prefix, b->njobs, nlane, b->chunk, (const uint64_t*)b->d_mask,
-                       b->d_counts, b->d_trims, b->scan_sums(), b->scan.shift);
+    const int64_t nchunks = (nlane + b->chunk - 1) / b->chunk;
+    for (int64_t first = 0; first < ncls; first += kMostBlocks)
+        hipLaunchKernelGGL(k_batch_classify, dim3((unsigned)std::min(kMostBlocks, ncls - first)), dim3(256), 0,
+                           b->stream, (const BatchJob*)b->d_jobs, (const int*)b->d_group_job,
+                           (const int64_t*)b->d_cls_prefix, b->ngroups, first, b->d_mask, b->scan_sums(),
+                           first ? 0 : kTileSums * b->scan.ntiles);
+    for (int64_t first = 0; first < nchunks; first += kMostBlocks)
+        hipLaunchKernelGGL(k_batch_count, dim3((unsigned)std::min(kMostBlocks, nchunks - first)), dim3(256), 0,
+                           b->stream, (const BatchJob*)b->d_jobs, (const int64_t*)b->d_lane_prefix, b->njobs, nlane,
+                           b->chunk, first, nchunks, (const uint64_t*)b->d_mask, b->d_counts, b->d_trims,
+                           b->scan_sums(), b->scan.shift);
     hipLaunchKernelGGL(k_fe_scan<uint32_t>, dim3((unsigned)b->scan.ntiles), dim3(256), 0, b->stream,
                        (const RowCounts*)b->d_counts, b->R, b->d_voff, b->d_toff, (const uint64_t*)b->scan_sums(),
                        b->scan.shift, b->scan.ntiles, b->totals(), b->h_jobout + 4 * b->njobs, ScanMore());
@@ -130,10 +129,10 @@ int enqueue_emit_into(miso_batch* b, int64_t nemit, float* pts, float* nrm, uint
     if (nlane == 0) return MISO_OK;
     const uint64_t* need = nemit < b->njobs ? b->d_jobout + 4 * nemit : b->totals();
     const bool xcd = b->queue_order == MISO_BATCH_QUEUE_XCD;
-    const int64_t items = emit_items(b, nemit), most = int64_t(1) << 23;   // a launch has fewer than 2^32 threads
+    const int64_t items = emit_items(b, nemit);
     auto launch = [&](auto kernel) {
-        for (int64_t first = 0; first < items; first += most)
-            hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(most, items - first)), dim3(256), 0, b->stream,
+        for (int64_t first = 0; first < items; first += kMostBlocks)
+            hipLaunchKernelGGL(kernel, dim3((unsigned)std::min(kMostBlocks, items - first)), dim3(256), 0, b->stream,
                                (const BatchJob*)b->d_jobs, (const int64_t*)b->d_lane_prefix, b->njobs, nlane,
                                (const uint64_t*)b->d_mask, (const RowCounts*)b->d_counts, (const uint64_t*)b->d_voff,
                                (const uint64_t*)b->d_toff, need, cap_v, cap_t, pts, nrm, tris,
@@ -591,6 +590,7 @@ extern "C" int miso_batch_autotune(miso_batch* b, int reps, float* best_ms)
             for (int x : kBlocks)
                 for (int c : kChunk) {
                     if (l == MISO_BATCH_LAUNCH_FUSED && (b->fused_per_cu < 1 || x > b->fused_per_cu)) continue;
+                    if (l == MISO_BATCH_LAUNCH_GRAPHS && x != kBlocks[1]) continue;   // the fused launch's alone
                     if (int rc = miso_batch_set_tuning(b, x, c)) return rc;
                     if (int rc = miso_batch_set_queue_order(b, o)) return rc;
                     if (int rc = miso_batch_set_launch(b, l)) return rc;

@@ -5,14 +5,13 @@
  * The jobs' grid rows are concatenated into one row space: the per-row arrays (sign masks,
  * counts, trims, offsets) of job j start at row_base / mask_base. An item is one block of the
  * single-volume kernels (4 wavefronts of lane rows for counting and emission) of one job, found in the
- * jobs' item prefix. Passes 1 and 2 are persistent kernels whose blocks take chunks of consecutive items
- * in turn (items of one kind cost the same); pass 4, whose items differ, is one block per item, which
- * the dispatcher hands out as blocks end. Classification works on groups of consecutive jobs that read
- * the same volume (one volume at several isovalues): an item is a block of the group's rows, loaded once
- * for all its jobs. Pass 3 is the single-volume scan over the concatenated rows, so job j's output is
- * the contiguous range [voff[row_base_j], voff[row_base_{j+1}]) of one shared buffer; its triangles
- * index its own vertices from 0. k_batch_fused runs the same block functions for all four passes in one
- * cooperative launch, with grid barriers between the passes.
+ * jobs' item prefix. Pass 1 and pass 4 are one block per item, pass 2 one per few consecutive items (their
+ * sums are added up once), and the dispatcher hands the blocks out as others end. Classification works
+ * on groups of consecutive jobs that read the same volume (one volume at several isovalues): an item is
+ * a block of the group's rows, loaded once for all its jobs. Pass 3 is the single-volume scan over the
+ * concatenated rows, so job j's output is the contiguous range [voff[row_base_j], voff[row_base_{j+1}])
+ * of one shared buffer; its triangles index its own vertices from 0. k_batch_fused runs the same block
+ * functions for all four passes in one cooperative launch, with grid barriers between the passes.
  */
 #ifndef MINIISO_FE_BATCH_H
 #define MINIISO_FE_BATCH_H
@@ -58,11 +57,10 @@ __device__ __forceinline__ int find_job(const int64_t* __restrict__ prefix, int 
     return lo;
 }
 
-/* The items of block b of nblocks persistent ones: the chunks b, b + nblocks, ... of `chunk` consecutive
- * items each; item i of job j after next(). Every wavefront walks the same items by itself: no barrier,
- * and no queue's counter to wait for. A counter gives out a ticket every 14 ns: pass 1 of 256 mixed volumes
- * (170,000 small items of a row per wavefront, then) took 600 us with tickets, 385 without (and several
- * rows per wavefront), and the batch 943 us and 668. */
+/* The items of block b of nblocks: the chunks b, b + nblocks, ... of `chunk` consecutive items each; item i
+ * of job j after next(). Every wavefront walks the same items by itself: no barrier, and no queue's counter
+ * to wait for (a counter gives out a ticket every 14 ns: pass 1 of 256 mixed volumes, then 170,000 items,
+ * took 600 us with tickets). */
 struct ItemWalk {
     const int64_t* __restrict__ prefix;
     int64_t nitems, stride, it, end, i;
@@ -150,27 +148,34 @@ __device__ __forceinline__ void batch_classify_item(const BatchJob* __restrict__
         fe_classify_block_n(job_volume(J), J.g, n, sink, blk, INT64_MAX);
 }
 
+/* Pass 1, one item per block, from item `first`. A wavefront's item is one chain of loads (its job, then 2048
+ * voxels), which only other wavefronts' hide: 256 mixed volumes (1.24 GB) take 234 us with a block per item,
+ * 253 with four items per block one after the other, 265 with 2048 blocks that walk all of them; a 256^3
+ * volume at 16 isovalues 41, 59 and 59 us. */
 __global__ __launch_bounds__(256) void k_batch_classify(const BatchJob* __restrict__ jobs,
                                                         const int* __restrict__ group_job,
                                                         const int64_t* __restrict__ prefix, int ngroups,
-                                                        int64_t nitems, int chunk, uint64_t* __restrict__ mask,
+                                                        int64_t first, uint64_t* __restrict__ mask,
                                                         uint64_t* __restrict__ sums, int64_t nsums)
 {
     // pass 2 adds up the scan's tile sums: clear them here
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < nsums; t += (int64_t)gridDim.x * blockDim.x)
         sums[t] = 0;
-    ItemWalk walk(prefix, ngroups, nitems, chunk, blockIdx.x, gridDim.x);
-    while (walk.next()) batch_classify_item(jobs, group_job, mask, walk.j, walk.i);
+    const int64_t it = first + blockIdx.x;
+    const int q = find_job(prefix, ngroups, it);
+    batch_classify_item(jobs, group_job, mask, q, it - prefix[q]);
 }
 
+/* Pass 2, a chunk of items per block, from chunk `first` of nchunks. 256 mixed volumes: 67 us with chunks of
+ * four, 80 with one item per block (an atomic per item and kind), 87 with 2048 blocks that walk all chunks. */
 __global__ __launch_bounds__(256) void k_batch_count(const BatchJob* __restrict__ jobs,
                                                      const int64_t* __restrict__ prefix, int njobs, int64_t nitems,
-                                                     int chunk, const uint64_t* __restrict__ mask,
-                                                     RowCounts* __restrict__ counts, RowTrim* __restrict__ trims,
-                                                     uint64_t* __restrict__ sums, int shift)
+                                                     int chunk, int64_t first, int64_t nchunks,
+                                                     const uint64_t* __restrict__ mask, RowCounts* __restrict__ counts,
+                                                     RowTrim* __restrict__ trims, uint64_t* __restrict__ sums, int shift)
 {
-    batch_count_items(jobs, ItemWalk(prefix, njobs, nitems, chunk, blockIdx.x, gridDim.x), mask, counts, trims, sums,
-                      shift);
+    batch_count_items(jobs, ItemWalk(prefix, njobs, nitems, chunk, first + blockIdx.x, nchunks), mask, counts, trims,
+                      sums, shift);
 }
 
 /* Job j's first vertex, first triangle, vertex and triangle counts (from the scan). */
