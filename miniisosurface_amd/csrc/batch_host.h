@@ -70,13 +70,6 @@ bool geom_lane_rows(const Geom& g)
     return g.W <= 64 && (g.ny + 130) * 3 * g.nx < (int64_t(1) << 32) && planes * g.nx * g.ny < (int64_t(1) << 31);
 }
 
-int64_t geom_rows_per_wave(const Geom& g)
-{
-    int64_t wp = 1;
-    while (wp < g.W) wp <<= 1;
-    return 64 / wp;
-}
-
 void destroy_graphs(miso_batch* b)
 {
     if (b->g_scan) (void)hipGraphExecDestroy(b->g_scan);
@@ -265,7 +258,7 @@ int batch_set_jobs(miso_batch* b, const miso_volume* vols, const float* isovals,
     if (!vols || !isovals) return fail(MISO_ERR_ARG, "volumes or isovalues NULL");
     std::vector<BatchJob> jobs(njobs);
     std::vector<int64_t> lane(njobs + 1, 0);
-    int64_t R = 0, mw = 0;
+    int64_t R = 0, mw = 0, waves = 0;
     for (int64_t j = 0; j < njobs; ++j) {
         const miso_volume* v = &vols[j];
         if (int rc = check_volume(v)) return rc;
@@ -284,8 +277,16 @@ int batch_set_jobs(miso_batch* b, const miso_volume* vols, const float* isovals,
         const int64_t rows = J.g.ny * J.g.nz;
         R += rows;
         mw += rows * J.g.W;
-        const int64_t per_block = 4 * geom_rows_per_wave(J.g);
-        lane[j + 1] = lane[j] + (rows + per_block - 1) / per_block;
+        waves += (rows << fewest_lanes(J.g.W)) >> 6;
+    }
+    // the fewest lanes per row, and more in every job where all jobs together are a small volume (plan_lanes)
+    int more = 0;
+    while (more < 6 && (waves << more) < kFillWaves) ++more;
+    for (int64_t j = 0; j < njobs; ++j) {
+        Geom& g = jobs[j].g;
+        set_lanes(g, std::min(6, fewest_lanes(g.W) + more));
+        const int64_t per_block = 4 * (int64_t)(64 >> g.lg_wp);
+        lane[j + 1] = lane[j] + (g.ny * g.nz + per_block - 1) / per_block;
     }
     // classify groups: runs of consecutive jobs on one volume with the same dimensions (one
     // volume at several isovalues), whose rows pass 1 then loads once for all of them

@@ -80,6 +80,12 @@ int check_volume(const miso_volume* v)
     return MISO_OK;
 }
 
+void set_lanes(Geom& g, int lg_wp)
+{
+    g.lg_wp = lg_wp;
+    g.bo = plan_block_order(g.ny, g.nz, g.W, lg_wp);
+}
+
 Geom make_geom(const miso_volume* v)
 {
     Geom g{};
@@ -95,7 +101,7 @@ Geom make_geom(const miso_volume* v)
     g.nzg = v->nz;
     g.emit_lo = 0;
     g.emit_hi = v->ny * v->nz;
-    g.bo = plan_block_order(g.ny, g.nz, g.W);
+    set_lanes(g, plan_lanes(g.ny, g.nz, g.W));
     return g;
 }
 
@@ -282,15 +288,9 @@ struct RowState {
         return g.W <= 64 && (g.ny + 130) * 3 * g.nx < (int64_t(1) << 32) &&
                planes * g.nx * g.ny < (int64_t(1) << 31);
     }
-    int rows_per_wave() const
-    {
-        int wp = 1;
-        while (wp < g.W) wp <<= 1;
-        return 64 / wp;
-    }
     unsigned lane_row_blocks() const
     {
-        const int64_t per_block = 4 * (int64_t)rows_per_wave();
+        const int64_t per_block = 4 * (int64_t)(64 >> g.lg_wp);
         return (unsigned)((g.ny * g.nz + per_block - 1) / per_block);
     }
 
@@ -928,7 +928,7 @@ int slab_launch_counts(miso_fe_slabs* h, int p, int64_t k0)
     g.nzg = G.nz;
     g.emit_lo = (k0 - d0) * G.ny;
     g.emit_hi = (k1 - d0) * G.ny;
-    g.bo = plan_block_order(g.ny, g.nz, g.W);
+    set_lanes(g, plan_lanes(g.ny, g.nz, g.W));
     s.g = g;
     const int64_t R = g.ny * g.nz;
     s.scan = plan_scan(R);

@@ -100,7 +100,7 @@ __device__ __forceinline__ void batch_count_items(const BatchJob* __restrict__ j
         uint32_t xy, zt;                   // per row, in one lane per row
         const WaveSums w = fe_count_rows_block(mask + J.mask_base, J.g, counts + J.row_base, trims + J.row_base, walk.i,
                                                NoRowExtra(), xy, zt);
-        const RowLanes rl = row_lanes(J.g.W);
+        const RowLanes rl = row_lanes(J.g);
         const int64_t r0 = J.row_base + (walk.i * 4 + wave_in_block()) * rl.rpw;
         // a job's rows start anywhere in a tile, so a wavefront's may lie in two
         const int64_t first = r0 >> shift, last = (r0 + rl.rpw - 1) >> shift;

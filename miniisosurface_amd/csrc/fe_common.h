@@ -44,7 +44,8 @@ struct Geom {
     // triangles of rows [emit_lo, emit_hi). A whole volume has kofs 0, nzg nz and all rows.
     int64_t kofs, nzg;
     int64_t emit_lo, emit_hi;
-    BlockOrder bo;        // planned for ny, nz and W whenever they are set
+    int lg_wp;            // lanes per grid row in the lane-row kernels, 2^lg_wp (plan_lanes)
+    BlockOrder bo;        // planned for ny, nz and lg_wp whenever they are set
 };
 
 struct RowCounts {

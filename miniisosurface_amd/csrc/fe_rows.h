@@ -1,8 +1,8 @@
 /*
  * fe_rows.h -- Flying Edges passes 2 and 4 with (grid row, mask word) pairs on the lanes.
  *
- * A wavefront covers RPW consecutive grid rows of W mask words each (RPW = 64 / Wp, Wp the next
- * power of two >= W, so nx <= 4096 voxels per row); lane (q, w) owns word w of row q. Row
+ * A wavefront covers RPW consecutive grid rows of W mask words each (RPW = 64 / Wp, Wp a power of
+ * two >= W, so nx <= 4096 voxels per row); lane (q, w) owns word w of row q. Row
  * totals and offsets are segmented wave reductions and prefix sums over the Wp lanes of a row.
  * Consecutive grid rows own consecutive vertex blocks, so a wavefront's vertices form one
  * contiguous range of the output, and its triangles one contiguous range too.
@@ -27,10 +27,33 @@ struct RowLanes {
     int w;        // this lane's word within the row
 };
 
-__device__ __forceinline__ RowLanes row_lanes(int64_t W)
+/* lg of the lanes per row: the fewest that hold a row's words (at most 64), and more, so that a wavefront
+ * has fewer rows, where `waves` wavefronts of those would be less than kFillWaves. Passes 2 and 4 of a
+ * small volume are as long as one wavefront's chain of loads, lists and stores (64^3 with 64 rows per
+ * wavefront: 64 wavefronts for 256 CUs). Whole extractions without allocation, with the fewest lanes and at
+ * least 1024, 2048, 4096 or 8192 wavefronts: 64^3 gyroid 154, 54, 55, 62, 62 us; 96^3 noise 105, 64, 61, 67, 80;
+ * 128^3 gyroid 102, 74, 63, 61, 75; 160^3 noise 82, 82, 72, 77, 92; 200^3 gyroid 92, 92, 92, 98, 97. More
+ * wavefronts than that repeat the setup and leave lanes empty. */
+constexpr int64_t kFillWaves = 2048;
+
+inline int fewest_lanes(int64_t W)
+{
+    int lg = 0;
+    while (lg < 6 && (int64_t(1) << lg) < W) ++lg;
+    return lg;
+}
+
+inline int plan_lanes(int64_t ny, int64_t nz, int64_t W)
+{
+    int lg = fewest_lanes(W);
+    while (lg < 6 && ((ny * nz) << lg) >> 6 < kFillWaves) ++lg;
+    return lg;
+}
+
+__device__ __forceinline__ RowLanes row_lanes(const Geom& g)
 {
     RowLanes L;
-    const int lg = W <= 1 ? 0 : 64 - __builtin_clzll((unsigned long long)(W - 1));   // Wp = 2^lg >= W
+    const int lg = g.lg_wp;
     L.Wp = 1 << lg;
     L.rpw = 64 >> lg;
     const int lane = lane_id();
@@ -40,7 +63,7 @@ __device__ __forceinline__ RowLanes row_lanes(int64_t W)
 }
 
 /* the first row of lane-row block blk */
-__device__ __forceinline__ int64_t block_row(int64_t W, int64_t blk) { return blk * 4 * row_lanes(W).rpw; }
+__device__ __forceinline__ int64_t block_row(const Geom& g, int64_t blk) { return blk * 4 * (64 >> g.lg_wp); }
 
 /* This wavefront's index within its 256-thread block, in a scalar register. */
 __device__ __forceinline__ int wave_in_block() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
@@ -336,7 +359,7 @@ __device__ __forceinline__ WaveSums fe_count_rows_block(const uint64_t* __restri
 {
     WaveSums sums{0u, 0u, 0u};
     xy = zt = 0u;
-    const RowLanes rl = row_lanes(g.W);
+    const RowLanes rl = row_lanes(g);
     const int64_t r0 = (blk * 4 + wave_in_block()) * rl.rpw;
     if (r0 >= g.ny * g.nz) return sums;
     const WaveRows A = wave_rows(g, r0, rl.rpw);
@@ -420,7 +443,7 @@ __global__ __launch_bounds__(256) void k_fe_count_rows(const uint64_t* __restric
 {
     uint32_t xy, zt;
     const WaveSums w = fe_count_rows_block(mask, g, counts, trims, blockIdx.x, NoRowExtra(), xy, zt);
-    add_block_sums(w, sums + (block_row(g.W, blockIdx.x) >> shift) * kTileSums);
+    add_block_sums(w, sums + (block_row(g, blockIdx.x) >> shift) * kTileSums);
 }
 
 /* ------------------------------------------------------------------ pass 4: edge points */
@@ -673,7 +696,7 @@ __device__ __forceinline__ bool emit_rows_setup(EmitRows& E, Lds* s_w, const uin
 {
     E.lane = lane_id();
     E.wv = wave_in_block();
-    E.rl = row_lanes(g.W);
+    E.rl = row_lanes(g);
     const RowLanes& rl = E.rl;
     const int64_t R = g.ny * g.nz;
     E.r0 = (blk * 4 + E.wv) * rl.rpw;
@@ -1104,13 +1127,11 @@ __device__ __forceinline__ void fe_emit_rows_block(const uint64_t* __restrict__ 
  * at 1024^3, iso 0.95 took 0.15 ms against 0.08 ms. */
 constexpr uint32_t kBlockOrderTP = 3;
 
-inline BlockOrder plan_block_order(int64_t ny, int64_t nz, int64_t W)
+inline BlockOrder plan_block_order(int64_t ny, int64_t nz, int64_t W, int lg_wp = -1)
 {
     BlockOrder o{0u, 1u, 1u, 0u};
     if (W < 1 || W > 64 || ny >= (1ll << 30)) return o;
-    int64_t wp = 1;
-    while (wp < W) wp <<= 1;
-    const int64_t per_block = 4 * (64 / wp);                // 4 wavefronts of lane rows: 4 .. 256
+    const int64_t per_block = 4 * (64 >> (lg_wp < 0 ? fewest_lanes(W) : lg_wp));   // 4 wavefronts of lane rows: 4 .. 256
     const int64_t n = (ny * nz + per_block - 1) / per_block;
     if (ny % per_block || n > 0xFFFFFFFFll) return o;
     const int64_t G = ny / per_block;                       // blocks per plane

@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256) void k_fe_mc_count_rows(const uint64_t* __rest
 {
     uint32_t xy, zt;
     const WaveSums w = fe_count_rows_block(mask, g, counts, trims, blockIdx.x, OwnedEdges{g, owned}, xy, zt);
-    add_block_sums(w, sums + (block_row(g.W, blockIdx.x) >> shift) * kTileSums);
+    add_block_sums(w, sums + (block_row(g, blockIdx.x) >> shift) * kTileSums);
 }
 
 /* Per case: for each cut edge e, its rank in order of first appearance in the case's triangle
