@@ -131,10 +131,10 @@ __global__ __launch_bounds__(256) void k_batch_zero(uint64_t* __restrict__ words
 
 /* Pass 1 item blk of classify group q: the jobs [group_job[q], group_job[q + 1]), consecutive jobs that
  * read the same volume with the same dimensions (one volume at several isovalues); a block of its rows
- * is loaded once and every job's sign-mask words written. */
+ * is loaded once and every job's sign-mask words written. bits: kFlatBits words of LDS per wavefront. */
 __device__ __forceinline__ void batch_classify_item(const BatchJob* __restrict__ jobs,
                                                     const int* __restrict__ group_job, uint64_t* __restrict__ mask,
-                                                    int q, int64_t blk)
+                                                    int q, int64_t blk, uint32_t* __restrict__ bits)
 {
     const int j0 = group_job[q], n = group_job[q + 1] - j0;
     const BatchJob& J = jobs[j0];
@@ -143,7 +143,7 @@ __device__ __forceinline__ void batch_classify_item(const BatchJob* __restrict__
         m = mask + jobs[j0 + t].mask_base;
     };
     if (J.g.W <= kFlatWords)
-        fe_classify_flat_n(job_volume(J), J.g, n, sink, blk, flat_rows_per_wave(J.g.nx));
+        fe_classify_flat_n(job_volume(J), J.g, n, sink, blk, flat_rows_per_wave(J.g.nx), bits);
     else
         fe_classify_block_n(job_volume(J), J.g, n, sink, blk, INT64_MAX);
 }
@@ -158,12 +158,13 @@ __global__ __launch_bounds__(256) void k_batch_classify(const BatchJob* __restri
                                                         int64_t first, uint64_t* __restrict__ mask,
                                                         uint64_t* __restrict__ sums, int64_t nsums)
 {
+    __shared__ uint32_t s_bits[4][kFlatBits];
     // pass 2 adds up the scan's tile sums: clear them here
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < nsums; t += (int64_t)gridDim.x * blockDim.x)
         sums[t] = 0;
     const int64_t it = first + blockIdx.x;
     const int q = find_job(prefix, ngroups, it);
-    batch_classify_item(jobs, group_job, mask, q, it - prefix[q]);
+    batch_classify_item(jobs, group_job, mask, q, it - prefix[q], s_bits[threadIdx.x >> 6]);
 }
 
 /* Pass 2, a chunk of items per block, from chunk `first` of nchunks. 256 mixed volumes: 67 us with chunks of
@@ -310,7 +311,9 @@ __global__ __launch_bounds__(256) void k_batch_fused(const BatchJob* __restrict_
     __shared__ EmitRowsLds s_w[4];
     s_case[threadIdx.x] = kCaseSlots.v[threadIdx.x];
     ItemWalk walk(cls_prefix, ngroups, ncls, chunk, blockIdx.x, gridDim.x);
-    while (walk.next()) batch_classify_item(jobs, group_job, mask, walk.j, walk.i);
+    // pass 1's bits where pass 4 has its lists
+    uint32_t* bits = reinterpret_cast<uint32_t*>(&s_w[wave_in_block()]);
+    while (walk.next()) batch_classify_item(jobs, group_job, mask, walk.j, walk.i, bits);
     grid.sync();
     batch_count_items(jobs, ItemWalk(lane_prefix, njobs, nlane, chunk, blockIdx.x, gridDim.x), mask, counts, trims,
                       state + 2, shift);

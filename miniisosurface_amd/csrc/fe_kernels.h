@@ -152,17 +152,16 @@ __device__ __forceinline__ void fe_classify_block_n(const float* __restrict__ vo
 constexpr int kFlatWords = 4;
 constexpr int kFlatSteps = 4;
 constexpr int kFlatVoxels = 512 * kFlatSteps;
+constexpr int kFlatBits = kFlatVoxels / 32 + 4;    // LDS words of a wavefront
 __host__ __device__ __forceinline__ int flat_rows_per_wave(int64_t nx) { return kFlatVoxels / (int)nx; }
 
 template <class Sink>
 __device__ __forceinline__ void fe_classify_flat_n(const float* __restrict__ vol, const Geom& g, int n, Sink sink,
-                                                   int64_t blk, int per)
+                                                   int64_t blk, int per, uint32_t* __restrict__ bits)
 {
-    __shared__ uint32_t s_bits[4][kFlatVoxels / 32 + 4];
     const int lane = lane_id(), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int64_t r0 = (blk * 4 + wv) * per, left = g.ny * g.nz - r0;
     if (left <= 0) return;
-    uint32_t* __restrict__ bits = s_bits[wv];
     const int nx = (int)g.nx, W = (int)g.W, rows = (int)(left < per ? left : per), voxels = rows * nx;
     const int64_t there = left * g.nx;                  // voxels to the volume's end
     const float* __restrict__ base = vol + r0 * g.nx;
@@ -219,12 +218,13 @@ __global__ __launch_bounds__(256) void k_fe_classify(const float* __restrict__ v
                                                      uint64_t* __restrict__ mask, int64_t keep_row,
                                                      uint64_t* __restrict__ sums, int64_t nsums)
 {
+    __shared__ uint32_t s_bits[4][kFlatBits];
     // pass 2 adds up the tile sums of pass 3: clear them here
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < nsums; t += (int64_t)gridDim.x * blockDim.x)
         sums[t] = 0;
     auto sink = [&](int, float& is, uint64_t*& m) { is = iso; m = mask; };
     if (g.W <= kFlatWords)
-        fe_classify_flat_n(vol, g, 1, sink, blockIdx.x, flat_rows_per_wave(g.nx));
+        fe_classify_flat_n(vol, g, 1, sink, blockIdx.x, flat_rows_per_wave(g.nx), s_bits[threadIdx.x >> 6]);
     else
         fe_classify_block_n(vol, g, 1, sink, blockIdx.x, keep_row);
 }

@@ -636,7 +636,7 @@ struct CornerCoords {
 };
 
 /* ------------------------------------------------------------------ pass 4: fused emit */
-constexpr int kEmitCellCap = 240;   // active-cell entries per wavefront and round
+constexpr int kEmitCellCap = 576;   // active-cell entries per wavefront and round
 constexpr int kEmitTriCap = 64 * 5; // triangles of one group of 64 cells (at most 5 each)
 constexpr int kIdStride = 7;        // dwords per cell of ids: odd, so that cells spread over the banks
 constexpr int kOriginCap = 640;     // origin entries per wavefront and round
@@ -645,7 +645,10 @@ constexpr int kOriginCap = 640;     // origin entries per wavefront and round
  * l at 2 l + h, followed by the next half's for the corner i + 1; a row that is not there repeats
  * row 0, so that it shows no cut). rank: per half, the id ranks of the eight edge combinations before
  * it, 16 bits each, (0,1) (2,3) (4,5) (6,7). origins: the vertices' list. t: the triangles' cell list
- * and, for the current 64 cells, their ids and the map of their triangles. Four blocks share a CU; a
+ * and, for the current 64 cells, their ids and the map of their triangles. The cell list takes what LDS four
+ * blocks leave: listing is done again for every round (of 240 cells instead of 576: 333x257x190 spaced 123
+ * us against 117, a 256^3 gyroid at 16 isovalues 1061 against 1043, 512^3 466.5 against 463, 1024^3 2.238
+ * ms against 2.228). Four blocks share a CU; a
  * fifth (the list in t's bytes, made again after the triangles) measured 1.48 against 1.445 ms at
  * 1024^3, three 1.73. */
 struct EmitRowsLds {

@@ -154,10 +154,11 @@ __global__ __launch_bounds__(256) void k_edge_order_perm(const RowCounts* __rest
 
 /* LDS of one wavefront of k_mc_ids_rows: as EmitRowsLds. With this alone, not pass 4's whole struct, eight
  * blocks share a CU. */
+constexpr int kMcIdsCells = 240;
 struct McIdsLds {
     uint4 rank[128];
     uint32_t words[4][130];
-    uint16_t cells[kEmitCellCap];
+    uint16_t cells[kMcIdsCells];
 };
 
 /* First-visit order: the map from Flying Edges vertex id to Marching Cubes id. Active cells one per lane
@@ -190,10 +191,10 @@ __global__ __launch_bounds__(256) void k_mc_ids_rows(const uint64_t* __restrict_
     const uint32_t cincl = wave_incl_scan_u32(ncell);
     const uint32_t ctotal = (uint32_t)__builtin_amdgcn_readlane((int)cincl, 63);
     uint64_t mid = moff[E.r0];
-    for (uint32_t win = 0; win < ctotal; win += kEmitCellCap) {
-        list_bits<kEmitCellCap>(E.act, cincl - ncell, win, E.lane, S.cells);
+    for (uint32_t win = 0; win < ctotal; win += kMcIdsCells) {
+        list_bits<kMcIdsCells>(E.act, cincl - ncell, win, E.lane, S.cells);
         wave_sync();
-        const uint32_t n = min((uint32_t)kEmitCellCap, ctotal - win);
+        const uint32_t n = min((uint32_t)kMcIdsCells, ctotal - win);
         for (uint32_t g0 = 0; g0 < n; g0 += 64) {
             const uint32_t idx = g0 + (uint32_t)E.lane;
             const uint32_t ent = idx < n ? (uint32_t)S.cells[idx] : 0u;
