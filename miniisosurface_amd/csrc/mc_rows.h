@@ -152,9 +152,28 @@ __global__ __launch_bounds__(256) void k_edge_order_perm(const RowCounts* __rest
     }
 }
 
-/* LDS of one wavefront of k_mc_ids_rows: as EmitRowsLds. With this alone, not pass 4's whole struct, eight
- * blocks share a CU. */
-constexpr int kMcIdsCells = 240;
+/* The edges that a cell off the near faces may own (5, 6, 11) as a case has them: bits 0, 1, 2 that they are
+ * cut, bits 4, 6, 8 on their places among them in order of first appearance. */
+__device__ __forceinline__ uint16_t inner_order(uint64_t order)
+{
+    const int edge[3] = {5, 6, 11};
+    uint32_t r = 0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        if (!((order >> (48 + edge[a])) & 1ull)) continue;
+        uint32_t before = 0;
+#pragma unroll
+        for (int b = 0; b < 3; ++b)
+            before += ((order >> (48 + edge[b])) & 1ull) && ((order >> (4 * edge[b])) & 0xF) < ((order >> (4 * edge[a])) & 0xF);
+        r |= 1u << a | before << (4 + 2 * a);
+    }
+    return (uint16_t)r;
+}
+
+/* LDS of one wavefront of k_mc_ids_rows: as EmitRowsLds. With this alone, not pass 4's whole struct, seven
+ * blocks share a CU (with 176 or 240 cells eight: 86 us at the 512^3 gyroid against 79, for the second
+ * round of listing). */
+constexpr int kMcIdsCells = 384;
 struct McIdsLds {
     uint4 rank[128];
     uint32_t words[4][130];
@@ -165,7 +184,8 @@ struct McIdsLds {
  * in order, as in pass 4's triangles, from the same words and ranks: a scan of the owned edges' counts
  * gives a cell's first id, the edges' order of first appearance the ids within the cell. Cells off the
  * near faces own at most the three edges that meet at their far corner (5, 6, 11), whose Flying Edges
- * ids run on from cell to cell: the stores of 64 lanes are runs. */
+ * ids run on from cell to cell: the stores of 64 lanes are runs. 64 such cells take their edges' places
+ * from a table by case (with the general order for all of them 84.5 us against 79 at the 512^3 gyroid). */
 template <typename Index>
 __global__ __launch_bounds__(256) void k_mc_ids_rows(const uint64_t* __restrict__ mask, Geom g,
                                                      const RowCounts* __restrict__ counts,
@@ -177,11 +197,13 @@ __global__ __launch_bounds__(256) void k_mc_ids_rows(const uint64_t* __restrict_
 {
     if (need && !output_fits<Index>(need, cap_v, cap_t)) return;
     __shared__ uint64_t s_first[256];
+    __shared__ uint16_t s_inner[256];
     __shared__ McIdsLds s_w[4];
     {
         // by the bits as the mask words give them (make_case_slots)
         const uint32_t c = threadIdx.x;
         s_first[c] = first_appearance(kCaseEdges[(c & 0x33) | (c & 0x44) << 1 | (c & 0x88) >> 1]);
+        s_inner[c] = inner_order(s_first[c]);
     }
     __syncthreads();
     EmitRows E;
@@ -209,7 +231,6 @@ __global__ __launch_bounds__(256) void k_mc_ids_rows(const uint64_t* __restrict_
             }
             const uint4 rk = S.rank[h2];
             const uint32_t cs = (t[0] & 3) | (t[1] & 3) << 2 | (t[2] & 3) << 4 | (t[3] & 3) << 6;
-            const uint64_t order = s_first[cs];
             const int i = (int)(ent & ((64u << E.wp_log2) - 1u));
             int j = E.j0 + (int)(ent >> (6 + E.wp_log2));
             int64_t k = E.k0;
@@ -217,24 +238,37 @@ __global__ __launch_bounds__(256) void k_mc_ids_rows(const uint64_t* __restrict_
                 j -= (int)g.ny;
                 ++k;
             }
+            const uint32_t below = bits_below(b);
+            auto cnt = [&](uint32_t bits) { return (uint32_t)__popc(bits & below); };
+            const uint32_t y1 = (rk.z >> 16) + cnt(w[2] ^ w[3]), z1 = (rk.w >> 16) + cnt(w[1] ^ w[3]);
+            const uint64_t at5 = E.v2 + (y1 + ((t[2] ^ t[3]) & 1u)), at6 = E.v2 + ((rk.y >> 16) + cnt(x[3]));
+            const uint64_t at11 = E.v0 + (z1 + ((t[1] ^ t[3]) & 1u));
+            if (__ballot(idx < n && (i == 0 || j == 0 || k == 0)) == 0ull) {
+                const uint32_t in = idx < n ? (uint32_t)s_inner[cs] : 0u, no = (uint32_t)__popc(in & 7u);
+                const uint32_t incl = wave_incl_scan_u32(no);
+                const uint64_t first = mid + (incl - no);
+                if (in & 1u) fe_to_mc[at5] = (Index)(first + __builtin_amdgcn_ubfe(in, 4, 2));
+                if (in & 2u) fe_to_mc[at6] = (Index)(first + __builtin_amdgcn_ubfe(in, 6, 2));
+                if (in & 4u) fe_to_mc[at11] = (Index)(first + __builtin_amdgcn_ubfe(in, 8, 2));
+                mid += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+                continue;
+            }
+            const uint64_t order = s_first[cs];
             const uint32_t own = idx < n ? (uint32_t)(order >> 48) & 0xFFFu & mc_owned_edges(i == 0, j == 0, k == 0) : 0u;
             const uint32_t no = (uint32_t)__popc(own);
             const uint32_t incl = wave_incl_scan_u32(no);
             uint32_t place = 0;      // bit p: the edge that appears p-th is owned
             for (uint32_t o = own; o; o &= o - 1) place |= 1u << ((order >> (4 * __builtin_ctz(o))) & 0xF);
             const uint64_t first = mid + (incl - no);
-            const uint32_t below = bits_below(b);
-            auto cnt = [&](uint32_t bits) { return (uint32_t)__popc(bits & below); };
             auto put = [&](int e, uint64_t fe) {
                 if (!((own >> e) & 1u)) return;
                 const uint32_t p = (uint32_t)(order >> (4 * e)) & 0xF;
                 fe_to_mc[fe] = (Index)(first + (uint32_t)__popc(place & bits_below(p)));
             };
-            const uint32_t y0 = (rk.z & 0xFFFFu) + cnt(w[0] ^ w[1]), y1 = (rk.z >> 16) + cnt(w[2] ^ w[3]);
-            const uint32_t z0 = (rk.w & 0xFFFFu) + cnt(w[0] ^ w[2]), z1 = (rk.w >> 16) + cnt(w[1] ^ w[3]);
-            put(6, E.v2 + ((rk.y >> 16) + cnt(x[3])));
-            put(5, E.v2 + (y1 + ((t[2] ^ t[3]) & 1u)));
-            put(11, E.v0 + (z1 + ((t[1] ^ t[3]) & 1u)));
+            const uint32_t y0 = (rk.z & 0xFFFFu) + cnt(w[0] ^ w[1]), z0 = (rk.w & 0xFFFFu) + cnt(w[0] ^ w[2]);
+            put(6, at6);
+            put(5, at5);
+            put(11, at11);
             if (own & ~((1u << 5) | (1u << 6) | (1u << 11))) {
                 put(0, E.v0 + ((rk.x & 0xFFFFu) + cnt(x[0])));
                 put(2, E.v0 + ((rk.x >> 16) + cnt(x[1])));
