@@ -232,7 +232,8 @@ int miso_batch_wait(miso_batch* b);
 /* ---------------------------------------------------------------- Flying Edges without allocation */
 /* No counterpart in the reference. For callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): miso_fe_run in one
- * call on a device-resident volume, with no device allocation and no free. The row state of the
+ * call on a device-resident volume, with no device allocation and no free (the first call on a GPU
+ * pins a page of host memory for the counts, kept until the process ends). The row state of the
  * four passes (sign mask, row counts and trims, offsets, scan state, totals) lives in a static
  * device array of the library, 64 MiB per GPU, held from the library's load until the process
  * ends; volumes whose row state exceeds it (one bit per voxel plus about 40 bytes per grid row:
