@@ -785,10 +785,24 @@ __device__ __forceinline__ bool emit_rows_setup(EmitRows& E, Lds* s_w, const uin
 __device__ __forceinline__ uint32_t bits_below(uint32_t b) { return __builtin_amdgcn_ubfe(0xFFFFFFFFu, 0, b); }
 
 /* Appends the positions (lane << 6 | bit) of a lane's set bits to list, from entry `first` on as far
- * as they fall in [win, win + Cap). */
+ * as they fall in [win, win + Cap); total: those of the wavefront, which a list that holds them all takes
+ * without a test per entry. A lane's loop is a chain of branches, and its length the fullest lane's: without
+ * the test 333x257x190 spaced 116.9 -> 113.9 us, 1024^3 2.238 -> 2.215 ms, 1000x900x700 at iso 0.8 608 -> 604. In
+ * its place every lane writing in every step, both halves' bits in one loop, took 2.264 ms at 1024^3. */
 template <int Cap>
-__device__ __forceinline__ void list_bits(uint64_t bits, uint32_t first, uint32_t win, int lane, uint16_t* list)
+__device__ __forceinline__ void list_bits(uint64_t bits, uint32_t first, uint32_t win, uint32_t total, int lane,
+                                          uint16_t* list)
 {
+    if (total <= (uint32_t)Cap) {
+        uint16_t* to = list + first;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint32_t ent = (uint32_t)lane << 6 | (uint32_t)h << 5;
+            for (uint32_t a = h ? (uint32_t)(bits >> 32) : (uint32_t)bits; a; a &= a - 1)
+                *to++ = (uint16_t)(ent | (uint32_t)__builtin_ctz(a));
+        }
+        return;
+    }
     uint32_t p = first - win;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -1004,7 +1018,7 @@ __device__ __forceinline__ void emit_rows_triangles(const EmitRows& E, EmitRowsL
     const uint32_t dv = (uint32_t)(E.v2 - v0);
     Index* __restrict__ out = tris + 3 * E.t0;
     for (uint32_t win = 0; win < ctotal; win += kEmitCellCap) {
-        list_bits<kEmitCellCap>(E.act, cfirst, win, lane, S.t.cells);
+        list_bits<kEmitCellCap>(E.act, cfirst, win, ctotal, lane, S.t.cells);
         wave_sync();
         const uint32_t n = min((uint32_t)kEmitCellCap, ctotal - win);
         for (uint32_t g0 = 0; g0 < n; g0 += 64) {
@@ -1079,7 +1093,7 @@ __device__ __forceinline__ void emit_rows_both(const EmitRows& E, EmitRowsLds& S
     const uint32_t lane = (uint32_t)E.lane;
     VertexStep V;
     uint32_t n = min((uint32_t)kOriginCap, R.n);
-    list_bits<kOriginCap>(E.origins, R.first, 0, E.lane, S.origins);
+    list_bits<kOriginCap>(E.origins, R.first, 0, R.n, E.lane, S.origins);
     wave_sync();
     vertex_load(V, E, S, R, g, lane, n);
     wave_sync();
@@ -1093,7 +1107,7 @@ __device__ __forceinline__ void emit_rows_both(const EmitRows& E, EmitRowsLds& S
         if (win >= R.n) break;
         n = min((uint32_t)kOriginCap, R.n - win);
         wave_sync();
-        list_bits<kOriginCap>(E.origins, R.first, win, E.lane, S.origins);
+        list_bits<kOriginCap>(E.origins, R.first, win, R.n, E.lane, S.origins);
         wave_sync();
         vertex_load(V, E, S, R, g, lane, n);
     }

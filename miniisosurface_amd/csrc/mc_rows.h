@@ -214,7 +214,7 @@ __global__ __launch_bounds__(256) void k_mc_ids_rows(const uint64_t* __restrict_
     const uint32_t ctotal = (uint32_t)__builtin_amdgcn_readlane((int)cincl, 63);
     uint64_t mid = moff[E.r0];
     for (uint32_t win = 0; win < ctotal; win += kMcIdsCells) {
-        list_bits<kMcIdsCells>(E.act, cincl - ncell, win, E.lane, S.cells);
+        list_bits<kMcIdsCells>(E.act, cincl - ncell, win, ctotal, E.lane, S.cells);
         wave_sync();
         const uint32_t n = min((uint32_t)kMcIdsCells, ctotal - win);
         for (uint32_t g0 = 0; g0 < n; g0 += 64) {
