@@ -524,77 +524,6 @@ __device__ __forceinline__ float central(float lo, float hi, float s)
     return (lo - hi) / (2.0f * s);
 }
 
-template <bool Unit>
-__device__ __forceinline__ void edge_finish(const Geom& g, int axis, int i, int j, int k, float w, const float ga[3],
-                                            const float gb[3], float p[3], float nrm[3])
-{
-    float A[3], B[3];
-    if (Unit) {
-        A[0] = (float)i; A[1] = (float)j; A[2] = (float)(k + (int)g.kofs);
-        B[0] = A[0]; B[1] = A[1]; B[2] = A[2];
-        B[axis] = A[axis] + 1.0f;
-    } else {
-        fe_edge_corners(g, axis, i, j, k, A, B);
-    }
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        p[c] = A[c] + w * (B[c] - A[c]);
-        nrm[c] = ga[c] + w * (gb[c] - ga[c]);
-    }
-}
-
-/* x-edge (i,j,k)-(i+1,j,k): the 12 voxels in 5 loads (the row i-1..i+2, and the pairs i..i+1 in
- * rows j-1, j+1 and planes k-1, k+1); edges touching a face take fe_edge_point. */
-template <bool Unit>
-__device__ __forceinline__ void vertex_x(const float* __restrict__ v, const Geom& g, float iso, int i, int j, int k,
-                                         float p[3], float nrm[3])
-{
-    const int nx = (int)g.nx, ny = (int)g.ny, nz = (int)g.nz;
-    if (!(i >= 1 && i <= nx - 3 && j >= 1 && j <= ny - 2 && k >= 1 && k <= nz - 2)) {
-        fe_edge_point<Unit>(v, g, iso, 0, i, j, k, p, nrm);
-        return;
-    }
-    const int sy = nx, sz = nx * ny;
-    const Vox4 r = load_vox<Vox4>(v - 1);
-    const Vox2 ym = load_vox<Vox2>(v - sy), yp = load_vox<Vox2>(v + sy);
-    const Vox2 zm = load_vox<Vox2>(v - sz), zp = load_vox<Vox2>(v + sz);
-    const float w = (iso - r.y) / (r.z - r.y);
-    const float ga[3] = {central<Unit>(r.x, r.z, g.sp[0]), central<Unit>(ym.x, yp.x, g.sp[1]),
-                         central<Unit>(zm.x, zp.x, g.sp[2])};
-    const float gb[3] = {central<Unit>(r.y, r.w, g.sp[0]), central<Unit>(ym.y, yp.y, g.sp[1]),
-                         central<Unit>(zm.y, zp.y, g.sp[2])};
-    edge_finish<Unit>(g, 0, i, j, k, w, ga, gb, p, nrm);
-}
-
-/* y- or z-edge from (i,j,k) along `axis` (1 or 2): the voxels i-1..i+1 of both end rows in two
- * loads, the two further voxels along the edge, and the four across it (axis c, the third). */
-template <bool Unit>
-__device__ __forceinline__ void vertex_yz(const float* __restrict__ v, const Geom& g, float iso, int axis, int i,
-                                          int j, int k, float p[3], float nrm[3])
-{
-    const int nx = (int)g.nx, ny = (int)g.ny, nz = (int)g.nz;
-    const bool ay = axis == 1;
-    const int pa = ay ? j : k, na = ay ? ny : nz, pc = ay ? k : j, nc = ay ? nz : ny;
-    if (!(i >= 1 && i <= nx - 2 && pa >= 1 && pa <= na - 3 && pc >= 1 && pc <= nc - 2)) {
-        fe_edge_point<Unit>(v, g, iso, axis, i, j, k, p, nrm);
-        return;
-    }
-    const int sy = nx, sz = nx * ny;
-    const int sa = ay ? sy : sz, sc = ay ? sz : sy;
-    const float* __restrict__ vb = v + sa;
-    const Vox3 xa = load_vox<Vox3>(v - 1), xb = load_vox<Vox3>(vb - 1);
-    const float am = v[-sa], bp = vb[sa];
-    const float cam = v[-sc], cap = v[sc], cbm = vb[-sc], cbp = vb[sc];
-    const float w = (iso - xa.y) / (xb.y - xa.y);
-    const float spa = ay ? g.sp[1] : g.sp[2], spc = ay ? g.sp[2] : g.sp[1];
-    const float gax = central<Unit>(xa.x, xa.z, g.sp[0]), gbx = central<Unit>(xb.x, xb.z, g.sp[0]);
-    const float gaa = central<Unit>(am, xb.y, spa), gba = central<Unit>(xa.y, bp, spa);
-    const float gac = central<Unit>(cam, cap, spc), gbc = central<Unit>(cbm, cbp, spc);
-    const float ga[3] = {gax, ay ? gaa : gac, ay ? gac : gaa};
-    const float gb[3] = {gbx, ay ? gba : gbc, ay ? gbc : gba};
-    edge_finish<Unit>(g, axis, i, j, k, w, ga, gb, p, nrm);
-}
-
 /* Corner coordinates of the edges from an origin (i,j,k) below the last index of each axis, and the end
  * of edge_point with them: p = a + w (b - a), where b - a is 1 or spacing along the edge and a - a (0, or
  * NaN) across it. Flying Edges' are fe_edge_corners; Marching Cubes' (Mc) those of the cell that first
@@ -662,15 +591,6 @@ struct EmitRowsLds {
     } t;
 };
 static_assert(sizeof(EmitRowsLds) * 4 + 256 * 8 <= 40960, "four blocks of pass 4 share a CU's 160 KB");
-
-/* case of the cell at bit b of a 32-bit half: h[q] holds corner v_q's bits (the case's bit order) */
-__device__ __forceinline__ uint32_t case_of_half(const uint32_t h[8], int b)
-{
-    uint32_t c = __builtin_amdgcn_ubfe(h[0], b, 1);
-#pragma unroll
-    for (int q = 1; q < 8; ++q) c |= __builtin_amdgcn_ubfe(h[q], b, 1) << q;
-    return c;
-}
 
 /* Pass 4 for the (row, word) lane layout in one launch: each wavefront writes the vertices of its
  * rows, then the triangles of its cell rows. */
