@@ -168,7 +168,7 @@ int miso_mc_set_order(miso_mc* h, int order);
 /* No counterpart in the reference, which extracts one volume per process
  * (flyingEdges/serial/main.cpp:110-158). A batch is a fixed list of jobs -- device-resident
  * volumes of any shape (dimensions >= 2, rows of at most 4096 voxels), each with its own
- * isovalue; several jobs may share one volume -- extracted by one persistent launch per pass,
+ * isovalue; several jobs may share one volume -- extracted by one launch per pass,
  * replayed from captured HIP graphs. Each job's result is bit-identical to miso_fe_run on that
  * volume and isovalue; its triangles index its own vertices from 0 (32-bit). */
 typedef struct miso_batch miso_batch;

@@ -2,7 +2,7 @@
 
     b = BatchExtraction([(DeviceVolume, iso), ...])
     b.run()                      # passes 1-4 for every job, replayed from captured HIP graphs
-    b.autotune()                 # picks the persistent kernels' launch shape for this batch
+    b.autotune()                 # picks the launch shape for this batch
     mesh = b.mesh(j)             # job j as vtkio.TriangleMesh (uint64 indices, as the reference)
     pts, nrm, tris = b.device_output(j)   # device pointers into the shared output
 

@@ -324,9 +324,10 @@ struct ScanMore {
 /* Tile `tile` of the scan: first the sums of the tiles before it (wavefront a takes every fourth kind),
  * then its own rows, kScanStep at a time, four per thread. The last tile's block writes totals: V, T,
  * and with xyz the totals of x, y and z after them; V and T also to host (pinned memory), if given.
- * Latency-bound: no tile waits for another one. By event pairs, 8 us at 512^3 and 14.4 us at 1024^3,
- * against 17 and 28 with look-back over tiles of 4096 rows; pass 2, which adds up the sums, takes 2 and
- * 15 us more (27 and 176). A step's sums are of type
+ * Latency-bound: no tile waits for another one. 6 us at 512^3 and 12 us at 1024^3, against 17 and 28 with
+ * look-back over tiles of 4096 rows (event pairs; pass 2, which adds up the sums, then took 2 and 15 us
+ * more). Eight tile sums in flight per lane and the next rows requested a step ahead measured the same. A
+ * step's sums are of type
  * S, 64 bits where 1024 rows of 5 nx triangles may pass 2^32. */
 template <typename S = uint32_t>
 __device__ __forceinline__ void fe_scan_tile(const RowCounts* __restrict__ counts, int64_t R,

@@ -294,7 +294,9 @@ __device__ __forceinline__ uint64_t active_cells(const LaneWords& L, uint64_t eb
  * Corners and x-faces at x = i + 1 are those at x = i of the next cell, so that over the row they count
  * twice but at its two ends: V = sum over the four rows of 2 P - (first voxel) - (last voxel), and the
  * x-faces likewise, which takes one popcount for two. Bits past the row are 0, and no x-pair, ring or
- * inner face has one there. Word halves, so that three-operand logic takes one instruction. */
+ * inner face has one there. Word halves, so that three-operand logic takes one instruction: pass 2 at
+ * 1024^3, bound by its vector instructions, 160 -> 142 us with 342 -> 290 of them per wavefront (before the
+ * row sums 176 us, with every corner and face masked and counted). */
 __device__ __forceinline__ uint32_t word_tri_count(const LaneWords& L, const Geom& g, int w)
 {
     uint32_t P = 0, F = 0, A = 0, Q = 0;       // corners, faces, x-faces and rings, full cells
@@ -753,7 +755,7 @@ __device__ __forceinline__ float of_pair(const Vox2& v)
  * line and four lanes (a 4-byte gather mostly one per lane, so single voxels are read in pairs): 3.6
  * accesses per vertex by origin against 6.1 with an edge per lane (value noise at 1024^3, counted
  * from the mask; all of pass 4, from the L1's counter: 5.5 against 8.8). Pass 4 at 1024^3, with the
- * triangles of emit_rows_triangles: 1.59 -> 1.37-1.40 ms; 512^3 gyroid 0.41 -> 0.34-0.36 ms. Vertices are
+ * triangles of emit_rows_triangles: 1.59 -> 1.37-1.40 ms (now 1.35-1.37); 512^3 gyroid 0.41 -> 0.34 ms. Vertices are
  * stored from the lanes: put in windows of 192 at their place in LDS and stored in 16-byte pieces
  * they took the same time at 1024^3 and 3% more at 512^3, where a wavefront has several windows. */
 
