@@ -1279,7 +1279,8 @@ extern "C" void miso_mc_destroy(miso_mc* h)
  * the process. In host code `scratch` names no device address; the device address is taken per
  * device with hipGetSymbolAddress (scratch_ptr) and only that is passed to kernels. */
 constexpr size_t kScratchBytes = size_t(64) << 20;
-static __device__ __align__(256) uint8_t scratch[kScratchBytes];
+constexpr size_t kScratchRoom = size_t(64) << 10;   // beside what the limit counts (ScratchLayout)
+static __device__ __align__(256) uint8_t scratch[kScratchBytes + kScratchRoom];
 
 namespace {
 
@@ -1320,9 +1321,11 @@ int scratch_ptr(void** out, uint64_t** totals)
 
 size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
-/* Byte offsets of the row state inside the scratch array for geometry g; the total in `end`. */
+/* Byte offsets of the row state inside the scratch array for geometry g, and the bytes that the limit of
+ * kScratchBytes counts: the row state, 16 bytes per 4096 rows, and 24. The tile sums, at most 1024 tiles at that
+ * size, may take up to 40 KiB more, which kScratchRoom holds, so that they move no volume over the limit. */
 struct ScratchLayout {
-    size_t mask, counts, trims, voff, toff, sums, totals, end;
+    size_t mask, counts, trims, voff, toff, sums, totals, counted;
     explicit ScratchLayout(const Geom& g)
     {
         const size_t R = (size_t)(g.ny * g.nz);
@@ -1333,7 +1336,7 @@ struct ScratchLayout {
         toff = align256(voff + R * sizeof(uint64_t));
         sums = align256(toff + R * sizeof(uint64_t));
         totals = align256(sums + (size_t)(kTileSums * plan_scan((int64_t)R).ntiles) * sizeof(uint64_t));
-        end = totals + 5 * sizeof(uint64_t);
+        counted = align256(sums + (1 + 2 * ((R + 4095) / 4096)) * sizeof(uint64_t)) + 2 * sizeof(uint64_t);
     }
 };
 
@@ -1356,11 +1359,11 @@ extern "C" int miso_fe_run_noalloc(const miso_volume* vol, float isoval, void* s
         return fail(MISO_ERR_ARG, "miso_fe_run_noalloc takes rows of at most 4096 voxels (nx = %lld)",
                     (long long)g.nx);
     const ScratchLayout lay(g);
-    if (lay.end > kScratchBytes)
+    if (lay.counted > kScratchBytes)
         return fail(MISO_ERR_ARG,
                     "volume %lld x %lld x %lld needs %zu bytes of row state, above the %zu-byte scratch of "
                     "miso_fe_run_noalloc",
-                    (long long)g.nx, (long long)g.ny, (long long)g.nz, lay.end, kScratchBytes);
+                    (long long)g.nx, (long long)g.ny, (long long)g.nz, lay.counted, kScratchBytes);
     void* base = nullptr;
     if (int rc = scratch_ptr(&base, &s.h_totals)) return rc;
     uint8_t* sp = (uint8_t*)base;
