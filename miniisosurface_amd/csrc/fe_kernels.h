@@ -146,9 +146,10 @@ __device__ __forceinline__ void fe_classify_block_n(const float* __restrict__ vo
  * LDS. A row's words are then cut from the run of bits wherever they start. All steps are in flight at
  * once, and no lane waits at a row's end: with a row's words loaded one voxel per lane, 16 words a
  * wavefront, pass 1 of 256 mixed volumes (32 to 256 a side, 1.24 GB) was bound by its instructions and took
- * 385 us, now 265. 1024 or 4096 voxels a wavefront: the batch 559 and 552 us against 549. Longer rows
- * (up to 512 or 1024 voxels) gain nothing (400x300x280: 212 us either way), and large volumes of them
- * lose the streaming loads of the row kernel (512^3: 103 us against 85). */
+ * 385 us, then 265, and 235 with a block per item. 1024, 1536 or 3072 voxels a wavefront: the batch 500, 493
+ * and 512 us against 495; streaming loads 575 against 552 (neighbouring lanes' halves of a line are read
+ * twice). Longer rows (up to 512 or 1024 voxels) gain nothing (400x300x280: 212 us either way), and large
+ * volumes of them lose the streaming loads of the row kernel (512^3: 103 us against 85). */
 constexpr int kFlatWords = 4;
 constexpr int kFlatSteps = 4;
 constexpr int kFlatVoxels = 512 * kFlatSteps;
