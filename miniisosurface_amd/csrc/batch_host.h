@@ -258,7 +258,8 @@ int batch_set_jobs(miso_batch* b, const miso_volume* vols, const float* isovals,
     if (!vols || !isovals) return fail(MISO_ERR_ARG, "volumes or isovalues NULL");
     std::vector<BatchJob> jobs(njobs);
     std::vector<int64_t> lane(njobs + 1, 0);
-    int64_t R = 0, mw = 0, waves = 0;
+    int64_t R = 0, mw = 0;
+    BatchLanes lanes;
     for (int64_t j = 0; j < njobs; ++j) {
         const miso_volume* v = &vols[j];
         if (int rc = check_volume(v)) return rc;
@@ -277,14 +278,11 @@ int batch_set_jobs(miso_batch* b, const miso_volume* vols, const float* isovals,
         const int64_t rows = J.g.ny * J.g.nz;
         R += rows;
         mw += rows * J.g.W;
-        waves += (rows << fewest_lanes(J.g.W)) >> 6;
+        lanes.add(J.g.ny, J.g.nz, J.g.W);
     }
-    // the fewest lanes per row, and more in every job where all jobs together are a small volume (plan_lanes)
-    int more = 0;
-    while (more < 6 && (waves << more) < kFillWaves) ++more;
     for (int64_t j = 0; j < njobs; ++j) {
         Geom& g = jobs[j].g;
-        set_lanes(g, std::min(6, fewest_lanes(g.W) + more));
+        set_lanes(g, lanes.job(g.W));
         const int64_t per_block = 4 * (int64_t)(64 >> g.lg_wp);
         lane[j + 1] = lane[j] + (g.ny * g.nz + per_block - 1) / per_block;
     }

@@ -43,12 +43,32 @@ inline int fewest_lanes(int64_t W)
     return lg;
 }
 
+/* lg of how many times the fewest: `lanes` is the rows' sum of the fewest */
+inline int more_lanes(int64_t lanes)
+{
+    int more = 0;
+    while (more < 6 && (lanes << more) >> 6 < kFillWaves) ++more;
+    return more;
+}
+
 inline int plan_lanes(int64_t ny, int64_t nz, int64_t W)
 {
-    int lg = fewest_lanes(W);
-    while (lg < 6 && ((ny * nz) << lg) >> 6 < kFillWaves) ++lg;
-    return lg;
+    const int lg = fewest_lanes(W), most = lg + more_lanes((ny * nz) << lg);
+    return most < 6 ? most : 6;
 }
+
+/* The same for a batch: one `more` for every job, from all jobs' lanes together. Added up in wavefronts,
+ * rounded down per job, jobs of less than a wavefront count as nothing however many there are: 20000 of 7x7x7
+ * then got 13 blocks each in the place of one (2521 us against 711). */
+struct BatchLanes {
+    int64_t lanes = 0;
+    void add(int64_t ny, int64_t nz, int64_t W) { lanes += (ny * nz) << fewest_lanes(W); }
+    int job(int64_t W) const
+    {
+        const int lg = fewest_lanes(W) + more_lanes(lanes);
+        return lg < 6 ? lg : 6;
+    }
+};
 
 __device__ __forceinline__ RowLanes row_lanes(const Geom& g)
 {
