@@ -370,8 +370,10 @@ struct McState {
         if (order == MISO_MC_ORDER_EDGE) return s.launch_count();   // no first-visit offsets needed
         if (!s.lane_rows()) {
             if (int rc = s.launch_count()) return rc;
-            hipLaunchKernelGGL(k_mc_count, dim3(s.row_blocks()), dim3(256), 0, s.stream, (const uint64_t*)s.d_mask,
-                               s.g, (const RowCounts*)s.d_counts, d_owned, s.d_sums, s.scan.shift);
+            const int64_t R = s.g.ny * s.g.nz, per = mc_count_rows(R), per_block = kRowsPerBlock * per;
+            hipLaunchKernelGGL(k_mc_count, dim3((unsigned)((R + per_block - 1) / per_block)), dim3(256), 0, s.stream,
+                               (const uint64_t*)s.d_mask, s.g, (const RowCounts*)s.d_counts, d_owned, s.d_sums,
+                               s.scan.shift, (int)per);
         } else {
             hipLaunchKernelGGL(k_fe_mc_count_rows, dim3(s.lane_row_blocks()), dim3(256), 0, s.stream,
                                (const uint64_t*)s.d_mask, s.g, s.d_counts, s.d_trims, s.d_sums, s.scan.shift, d_owned);

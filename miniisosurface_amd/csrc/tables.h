@@ -133,6 +133,19 @@ constexpr CaseSlots make_case_slots()
 }
 static constexpr CaseSlots kCaseSlots = make_case_slots();
 
+/* The cube edges that a case cuts, a bit each: those that its triangles name. */
+struct CaseCuts {
+    uint16_t v[256];
+};
+constexpr CaseCuts make_case_cuts()
+{
+    CaseCuts t{};
+    for (int c = 0; c < 256; ++c)
+        for (int s = 0; s < 3 * (int)(kCaseEdges[c] >> 60); ++s) t.v[c] |= (uint16_t)(1u << ((kCaseEdges[c] >> (4 * s)) & 0xF));
+    return t;
+}
+static constexpr CaseCuts kCaseCuts = make_case_cuts();
+
 MISO_HD constexpr int case_tri_count(uint64_t packed) { return (int)(packed >> 60); }
 
 MISO_HD constexpr int case_edge(uint64_t packed, int slot) { return (int)((packed >> (4 * slot)) & 0xF); }
