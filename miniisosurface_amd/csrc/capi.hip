@@ -299,7 +299,7 @@ struct RowState {
         const int64_t per_block = classify_rows(g);
         const unsigned blocks = (unsigned)((g.ny * g.nz + per_block - 1) / per_block);
         hipLaunchKernelGGL(k_fe_classify, dim3(blocks), dim3(256), 0, stream, d_vol, g, iso, d_mask,
-                           keep_from_row(g), d_sums, kTileSums * scan.ntiles);
+                           keep_from_row(g, lane_rows()), d_sums, kTileSums * scan.ntiles);
         HIPCALL(hipGetLastError());
         return MISO_OK;
     }

@@ -1,7 +1,9 @@
 """CPU: how many lanes a grid row takes (plan_lanes, BatchLanes, miniisosurface_amd/csrc/fe_rows.h). A batch
 of many jobs fills the chip whatever the size of one job, so its rows keep the fewest lanes also where a
 job has less than one wavefront of them; a batch of few small jobs takes more, as one volume of all its rows
-would. The header is compiled for the host with hipcc."""
+would. And which rows pass 1 leaves in the caches (keep_from_row): the last 128 MB where pass 4 takes the rows
+from the end, else those of a volume that is kept whole, or none. The headers are compiled for the host with
+hipcc."""
 import os
 import shutil
 import subprocess
@@ -18,6 +20,15 @@ PROGRAM = r"""
 using namespace miso;
 int main(int argc, char** argv)
 {
+    if (argc == 4) {
+        Geom g{};
+        g.nx = atoll(argv[1]);
+        g.ny = atoll(argv[2]);
+        g.nz = atoll(argv[3]);
+        const long long R = g.ny * g.nz, end = keep_from_row(g, true), whole = keep_from_row(g, false);
+        printf("%lld %lld\n", R - end, R - whole);
+        return 0;
+    }
     const int64_t n = atoll(argv[1]), ny = atoll(argv[2]), nz = atoll(argv[3]), W = atoll(argv[4]);
     BatchLanes all;
     for (int64_t j = 0; j < n; ++j) all.add(ny, nz, W);
@@ -61,3 +72,15 @@ def test_batch_lanes(planner, n, ny, nz, W, lg):
     fewest, job, one = planner(n, ny, nz, W)
     assert job == one           # as one volume with the rows of all jobs
     assert job == lg and lg >= fewest
+
+
+# nx, ny, nz; rows kept where pass 4 starts at the end, and where it does not (all rows or more: the whole volume)
+@pytest.mark.parametrize("nx,ny,nz,end,whole", [
+    (1024, 1024, 1024, 32768, 0),
+    (4097, 64, 64, 8191, 8191),          # 67 MB
+    (65536, 128, 16, 512, 0),
+    (1 << 25, 2, 2, 1, 0),
+    (1 << 23, 2, 2, 4, 4),               # 128 MB
+])
+def test_kept_rows(planner, nx, ny, nz, end, whole):
+    assert planner(nx, ny, nz) == (end, whole)
