@@ -144,12 +144,12 @@ __global__ __launch_bounds__(256) void k_edge_order_perm(const RowCounts* __rest
     const uint32_t n = c.x + c.y + c.z;
     if (n == 0) return;
     const uint64_t f0 = voff[r];
-    const uint64_t bx = xyz[r], by = tot[0] + xyz[R + r], bz = tot[0] + tot[1] + xyz[2 * R + r];
+    // what each axis adds to t, modulo the ids' type: a selection and an addition per id (16x128x65536 noise
+    // 258 us; 410 with each axis's own 64-bit sum)
+    const Index dx = (Index)xyz[r], dy = (Index)(tot[0] + xyz[R + r] - c.x),
+                dz = (Index)(tot[0] + tot[1] + xyz[2 * R + r] - c.x - c.y);
     const uint32_t cxy = c.x + c.y;
-    for (uint32_t t = l; t < n; t += 16) {
-        const uint64_t id = t < c.x ? bx + t : (t < cxy ? by + (t - c.x) : bz + (t - cxy));
-        perm[f0 + t] = (Index)id;
-    }
+    for (uint32_t t = l; t < n; t += 16) perm[f0 + t] = (Index)((t < c.x ? dx : (t < cxy ? dy : dz)) + (Index)t);
 }
 
 /* The edges that a cell off the near faces may own (5, 6, 11) as a case has them: bits 0, 1, 2 that they are
