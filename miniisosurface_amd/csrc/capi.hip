@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "miniiso.h"
+#include "idle_kits.h"
 #include "fe_kernels.h"
 #include "mc_kernels.h"
 #include "fe_rows.h"
@@ -107,88 +108,6 @@ Geom make_geom(const miso_volume* v)
 
 inline bool has_cells(const Geom& g) { return g.nx >= 2 && g.ny >= 2 && g.nz >= 2; }
 
-/* What a handle without a caller's stream takes from the driver whatever its volume: a stream and a pinned
- * page for the totals. Making and destroying them took 80 us, as long as everything that a 128^3 volume
- * needs on the device, so a destroyed handle leaves them, idle, to the next one on its device: at most
- * kIdleKits per device wait here, the rest are destroyed. Any thread may take or leave one. */
-struct Kit {
-    hipStream_t stream = nullptr;
-    uint64_t* totals = nullptr;
-    int dev = 0;
-};
-constexpr int kIdleKits = 4;
-constexpr size_t kPinnedTotals = 2 * sizeof(uint64_t);
-
-struct IdleKits {
-    std::mutex lock;
-    std::vector<Kit> kits;
-};
-IdleKits& idle_kits()
-{
-    static IdleKits* k = new IdleKits();   // never destroyed: handles may outlive static objects
-    return *k;
-}
-
-void destroy_kit(Kit& k)
-{
-    if (k.totals) (void)hipHostFree(k.totals);
-    if (k.stream) (void)hipStreamDestroy(k.stream);
-    k = Kit();
-}
-
-int take_kit(Kit* out)
-{
-    int dev = 0;
-    HIPCALL(hipGetDevice(&dev));
-    IdleKits& idle = idle_kits();
-    for (;;) {
-        Kit k;
-        {
-            std::lock_guard<std::mutex> hold(idle.lock);
-            for (size_t q = idle.kits.size(); q-- > 0 && !k.stream;)
-                if (idle.kits[q].dev == dev) {
-                    k = idle.kits[q];
-                    idle.kits.erase(idle.kits.begin() + (long)q);
-                }
-        }
-        if (!k.stream) break;
-        if (hipStreamQuery(k.stream) == hipSuccess) {
-            *out = k;
-            return MISO_OK;
-        }
-        (void)hipGetLastError();   // not the stream that was left here (the device was reset): forget it
-    }
-    Kit k;
-    k.dev = dev;
-    // a blocking stream: ordered after work on the null stream (where callers that produce a
-    // device volume without naming a stream usually ran)
-    HIPCALL(hipStreamCreateWithFlags(&k.stream, hipStreamDefault));
-    const hipError_t e = hipHostMalloc((void**)&k.totals, kPinnedTotals, hipHostMallocDefault);
-    if (e != hipSuccess) {
-        k.totals = nullptr;
-        destroy_kit(k);
-        HIPCALL(e);
-    }
-    *out = k;
-    return MISO_OK;
-}
-
-/* the stream's work is done, without an error if `clean` */
-void leave_kit(Kit& k, bool clean)
-{
-    if (clean) {
-        IdleKits& idle = idle_kits();
-        std::lock_guard<std::mutex> hold(idle.lock);
-        int same = 0;
-        for (const Kit& q : idle.kits) same += q.dev == k.dev;
-        if (same < kIdleKits) {
-            idle.kits.push_back(k);
-            k = Kit();
-        }
-    }
-    destroy_kit(k);
-}
-
 /* Shared per-extraction device state: volume, sign masks, row counts, offsets, scan state, in one
  * allocation (eight took 30 us of a 128^3 call to make and to free). */
 struct RowState {
@@ -214,7 +133,7 @@ struct RowState {
             stream = (hipStream_t)user_stream;
             HIPCALL(hipHostMalloc((void**)&h_totals, kPinnedTotals, hipHostMallocDefault));
         } else {
-            if (int rc = take_kit(&kit)) return rc;
+            HIPCALL(idle_kits().take(&kit));
             stream = kit.stream;
             h_totals = kit.totals;
         }
@@ -262,7 +181,7 @@ struct RowState {
         if (stream) clean = hipStreamSynchronize(stream) == hipSuccess;
         dev_free(d_all);
         if (kit.stream)
-            leave_kit(kit, clean);
+            idle_kits().leave(kit, clean);
         else if (h_totals)
             (void)hipHostFree(h_totals);
         h_totals = nullptr;
