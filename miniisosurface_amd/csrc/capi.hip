@@ -1208,13 +1208,11 @@ namespace {
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mutex;
 void* g_scratch_ptr[kMaxDevices] = {};
-uint64_t* g_scratch_totals[kMaxDevices] = {};
+KeptPage g_scratch_page[kMaxDevices];
 
-/* The device address of `scratch` on the current device, and a pinned page of the host where pass 3 leaves V
- * and T: looked up and made on the first call there, and kept. Copied back behind pass 4 instead, which takes
- * a copy kernel, the counts cost each call 9 us (64^3 43 against 34 us, 128^3 47 against 38). No page
- * (totals NULL) where the host has none left; the first call may come while the thread captures a
- * graph, which the allocation does not touch. */
+/* The device address of `scratch` on the current device, looked up on the first call there and kept, and a pinned
+ * page of the host where pass 3 leaves V and T. Copied back behind pass 4 instead, which takes a copy kernel, the
+ * counts cost each call 9 us (64^3 43 against 34 us, 128^3 47 against 38). */
 int scratch_ptr(void** out, uint64_t** totals)
 {
     int dev = 0;
@@ -1225,18 +1223,10 @@ int scratch_ptr(void** out, uint64_t** totals)
         void* p = nullptr;
         HIPCALL(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
         if (!p) return fail(MISO_ERR_HIP, "hipGetSymbolAddress returned NULL for the scratch array");
-        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-        if (hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {
-            if (hipHostMalloc((void**)&g_scratch_totals[dev], kPinnedTotals, hipHostMallocDefault) != hipSuccess) {
-                g_scratch_totals[dev] = nullptr;
-                (void)hipGetLastError();
-            }
-            (void)hipThreadExchangeStreamCaptureMode(&mode);
-        }
         g_scratch_ptr[dev] = p;
     }
     *out = g_scratch_ptr[dev];
-    *totals = g_scratch_totals[dev];
+    *totals = g_scratch_page[dev].get();
     return MISO_OK;
 }
 

@@ -9,6 +9,7 @@
  * hipDeviceReset takes a device's streams and allocations away, and what is made after it may have the same
  * handles and addresses. An allocation's buffer id is never given twice in a process, so each kit holds a small
  * allocation on its device and is only handed on while that address still names the allocation (62 ns).
+ * The same test tells whether the pinned page of miso_fe_run_noalloc is still there (KeptPage).
  */
 #ifndef MINIISO_IDLE_KITS_H
 #define MINIISO_IDLE_KITS_H
@@ -134,6 +135,37 @@ inline IdleKits& idle_kits()
     static IdleKits k;
     return k;
 }
+
+/* A pinned page for two totals, made on the first call and kept. */
+class KeptPage {
+    uint64_t* page = nullptr;
+    unsigned long long id = 0;
+
+public:
+    /* NULL where the host has none left; the next call tries again. The call may come while the thread captures a
+     * graph, which the allocation does not touch. */
+    uint64_t* get()
+    {
+        if (page && buffer_id(page) == id) return page;
+        page = nullptr;                 // none yet, or it went with a device reset
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        if (hipHostMalloc((void**)&page, kPinnedTotals, hipHostMallocDefault) != hipSuccess) {
+            page = nullptr;
+            (void)hipGetLastError();
+        }
+        id = buffer_id(page);
+        if (page && !id) {
+            (void)hipHostFree(page);
+            page = nullptr;
+        }
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        return page;
+    }
+};
 
 }  // namespace miso
 

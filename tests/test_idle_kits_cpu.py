@@ -1,5 +1,5 @@
-"""CPU: the streams and pinned pages that destroyed handles leave to the next ones
-(miniisosurface_amd/csrc/idle_kits.h), compiled against a small HIP runtime of this test's own that counts
+"""CPU: the streams and pinned pages that destroyed handles leave to the next ones, and the no-allocation call's
+page (miniisosurface_amd/csrc/idle_kits.h), compiled against a small HIP runtime of this test's own that counts
 what is alive, gives recycled handles and addresses, can refuse a call, leave a stream unfinished and reset its
 device: nothing is lost, nothing is handed on or freed that a reset took away, at most four wait per device."""
 import os
@@ -197,6 +197,8 @@ int main(int, char** argv)
         auto k = take(2);
         for (auto& q : k) { EXPECT(q.stream && q.totals); idle_kits().leave(q, true); }
         EXPECT(alive() == 0 && f.wrong == 0);
+        KeptPage page;
+        EXPECT(!page.get() && alive() == 0);
     } else if (!strcmp(what, "threads")) {
         std::vector<std::thread> t;
         for (int n = 0; n < 8; ++n)
@@ -208,6 +210,21 @@ int main(int, char** argv)
             });
         for (auto& q : t) q.join();
         EXPECT(f.streams.size() <= 4 && alive() == 3 * f.streams.size() && f.wrong == 0);
+    } else if (!strcmp(what, "page")) {
+        KeptPage page;
+        f.refuse_host = 1;
+        EXPECT(!page.get());
+        f.refuse_host = 0;
+        uint64_t* p = page.get();                   // a later call tries again
+        EXPECT(p && f.host_calls == 2);
+        for (int t = 0; t < 5; ++t) EXPECT(page.get() == p);
+        EXPECT(f.host_calls == 2);
+        reset_device(0);
+        void* theirs = nullptr;
+        hipHostMalloc(&theirs, 1, 0);
+        EXPECT(theirs == (void*)p);                 // the address is someone else's now
+        uint64_t* q = page.get();
+        EXPECT(q && q != p && page.get() == q && f.wrong == 0 && f.memory.size() == 2);
     } else {
         return 2;
     }
@@ -231,7 +248,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["bounded", "busy", "reset", "reset alive", "refused", "no ids", "threads"])
+@pytest.mark.parametrize("what", ["bounded", "busy", "reset", "reset alive", "refused", "no ids", "threads", "page"])
 def test_idle_kits(program, what):
     out = subprocess.run([program, what], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0, out.stdout
