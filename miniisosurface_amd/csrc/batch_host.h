@@ -516,6 +516,7 @@ extern "C" int miso_batch_set_tuning(miso_batch* b, int blocks_per_cu, int chunk
     if (blocks_per_cu == b->blocks_per_cu && chunk == b->chunk) return MISO_OK;
     HIPCALL(hipStreamSynchronize(b->stream));
     b->blocks_per_cu = blocks_per_cu;
+    if (chunk == b->chunk) return MISO_OK;      // the fused launch's alone: the graphs stay as they are
     b->chunk = chunk;
     destroy_graphs(b);
     if (b->njobs == 0) return MISO_OK;
