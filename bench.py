@@ -453,8 +453,8 @@ def bench_host_scope(vol, iso, reps=2):
 
 def bench_batched(reps, cpu_threads=None):
     """256 mixed-size Gaussian volumes (dims log-uniform in [32, 256], 1-6 blobs, iso U[0.2, 0.8],
-    seed 0), and one 512^3 gyroid at 16 isovalues in [-1, 1]: the batch (one persistent launch per
-    pass, graph replay, autotuned shape) against the same jobs run one extraction at a time."""
+    seed 0), and one 512^3 gyroid at 16 isovalues in [-1, 1]: the batch (one launch per pass,
+    graph replay, autotuned shape) against the same jobs run one extraction at a time."""
     import numpy as np
     import torch
 

@@ -233,12 +233,13 @@ int miso_batch_wait(miso_batch* b);
 /* No counterpart in the reference. For callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): miso_fe_run in one
  * call on a device-resident volume, with no device allocation and no free (the first call on a GPU
- * pins a page of host memory for the counts, kept until the process ends). The row state of the
+ * pins a page of host memory for the counts, kept for the next ones). The row state of the
  * four passes (sign mask, row counts and trims, offsets, scan state, totals) lives in a static
- * device array of the library, 64 MiB per GPU, held from the library's load until the process
- * ends; volumes whose row state exceeds it (one bit per voxel plus about 40 bytes per grid row:
- * up to about 700^3 voxels) are refused with MISO_ERR_ARG, as are rows of more than 4096 voxels. The caller passes the output buffers: points and normals of cap_vertices * 3 floats,
- * triangles of cap_triangles * 3 uint32 indices (each triangle indexes this mesh's vertices).
+ * device array of the library, 64 MiB per GPU (and 64 KiB for the scan), held from the library's
+ * load until the process ends; volumes whose row state exceeds the 64 MiB (one bit per voxel plus
+ * about 40 bytes per grid row: up to about 700^3 voxels) are refused with MISO_ERR_ARG, as are rows
+ * of more than 4096 voxels. The caller passes the output buffers: points and normals of
+ * cap_vertices * 3 floats, triangles of cap_triangles * 3 uint32 indices (each triangle indexes this mesh's vertices).
  * Kernels run on `stream` (NULL: the null stream); the call returns when they are done, with the
  * mesh's counts in *nverts and *ntris. If the mesh does not fit the buffers, nothing is written
  * to them, the counts are still returned, and the status is MISO_ERR_ARG. Every call on one GPU

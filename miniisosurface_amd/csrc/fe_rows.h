@@ -661,8 +661,9 @@ __device__ __forceinline__ bool emit_rows_setup(EmitRows& E, Lds* s_w, const uin
     E.t0 = toff[E.r0];
     E.k0 = A.k0;
     E.j0 = A.j0;
-    // the row's vertex offset and, in the plane above, that row's, from v0 and v2 (below 2^16: at
-    // most 65 rows of 64 words in all hold 3 * 64 * 65 voxels' edges)
+    // the row's vertex offset and, in the plane above, that row's, from v0 and v2: below 2^16, since the wavefront's at
+    // most 4096 voxels have 12288 edges, and the row after them puts up to 8192 x- and y-edges before its z-edges,
+    // which rank up to 4096 among themselves: 24576
     const int64_t left_above = R - E.r0 - g.ny;             // rows from the one above the wavefront's first
     E.v2 = left_above > 0 ? voff[E.r0 + g.ny] : 0ull;
     uint32_t own = 0, above = 0, above_x = 0;

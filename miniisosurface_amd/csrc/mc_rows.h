@@ -171,14 +171,15 @@ __device__ __forceinline__ uint16_t inner_order(uint64_t order)
 }
 
 /* LDS of one wavefront of k_mc_ids_rows: as EmitRowsLds. With this alone, not pass 4's whole struct, seven
- * blocks share a CU (with 176 or 240 cells eight: 86 us at the 512^3 gyroid against 79, for the second
- * round of listing). */
+ * blocks share a CU. A shorter list only costs a second round of listing: at the 512^3 gyroid the kernel takes
+ * 82 us, 87 with 240 cells (seven blocks too), 87 with 176 (eight). */
 constexpr int kMcIdsCells = 384;
 struct McIdsLds {
     uint4 rank[128];
     uint32_t words[4][130];
     uint16_t cells[kMcIdsCells];
 };
+static_assert((sizeof(McIdsLds) * 4 + 256 * (8 + 2)) * 7 <= 163840, "seven blocks of k_mc_ids_rows share a CU's 160 KB");
 
 /* First-visit order: the map from Flying Edges vertex id to Marching Cubes id. Active cells one per lane
  * in order, as in pass 4's triangles, from the same words and ranks: a scan of the owned edges' counts
