@@ -57,12 +57,13 @@ __device__ __forceinline__ int find_job(const int64_t* __restrict__ prefix, int 
     return lo;
 }
 
-/* The items of block b of nblocks: the chunks b, b + nblocks, ... of `chunk` consecutive items each; item i
- * of job j after next(). Every wavefront walks the same items by itself: no barrier, and no queue's counter
+/* The items of block b of nblocks: the chunks b, b + nblocks, ... of `chunk` consecutive items each, or chunk b
+ * alone (not Again); item i of job j after next(). Every wavefront walks the same items by itself: no barrier, and no queue's counter
  * to wait for (a counter gives out a ticket every 14 ns: pass 1 of 256 mixed volumes, then 170,000 items,
  * took 600 us with tickets). A chunk's job is looked up, not walked to: between two chunks lie as many jobs as
  * items where a job is one item, each a load that waits for the one before (20000 volumes of 3x3x3, fused launch:
  * 2254 us walked, 623 looked up). */
+template <bool Again>
 struct ItemWalk {
     const int64_t* __restrict__ prefix;
     int64_t nitems, stride, it, end, i;
@@ -79,11 +80,12 @@ struct ItemWalk {
     {
         const bool jump = ++it == end;
         if (jump) {
+            if (!Again) return false;
             it += stride;
             end = it + chunk;
         }
         if (it >= nitems) return false;
-        if (it >= prefix[j + 1]) j = jump ? find_job(prefix, njobs, it) : j + 1;   // no job is without items
+        if (it >= prefix[j + 1]) j = Again && jump ? find_job(prefix, njobs, it) : j + 1;   // no job is without items
         i = it - prefix[j];
         return true;
     }
@@ -92,7 +94,8 @@ struct ItemWalk {
 /* Pass 2 of the batch's row blocks of this block's items, into the scan's tile sums: a wavefront keeps the
  * sums of the items it takes one after the other, as long as they lie in one tile, and adds them at
  * once (lane a, 0 .. 3, those of kind a). */
-__device__ __forceinline__ void batch_count_items(const BatchJob* __restrict__ jobs, ItemWalk walk,
+template <class Walk>
+__device__ __forceinline__ void batch_count_items(const BatchJob* __restrict__ jobs, Walk walk,
                                                   const uint64_t* __restrict__ mask, RowCounts* __restrict__ counts,
                                                   RowTrim* __restrict__ trims, uint64_t* __restrict__ sums, int shift)
 {
@@ -179,8 +182,8 @@ __global__ __launch_bounds__(256) void k_batch_count(const BatchJob* __restrict_
                                                      const uint64_t* __restrict__ mask, RowCounts* __restrict__ counts,
                                                      RowTrim* __restrict__ trims, uint64_t* __restrict__ sums, int shift)
 {
-    batch_count_items(jobs, ItemWalk(prefix, njobs, nitems, chunk, first + blockIdx.x, nchunks), mask, counts, trims,
-                      sums, shift);
+    batch_count_items(jobs, ItemWalk<false>(prefix, njobs, nitems, chunk, first + blockIdx.x, nchunks), mask, counts,
+                      trims, sums, shift);
 }
 
 /* Job j's first vertex, first triangle, vertex and triangle counts (from the scan). */
@@ -314,13 +317,13 @@ __global__ __launch_bounds__(256) void k_batch_fused(const BatchJob* __restrict_
     __shared__ uint64_t s_case[256];
     __shared__ EmitRowsLds s_w[4];
     s_case[threadIdx.x] = kCaseSlots.v[threadIdx.x];
-    ItemWalk walk(cls_prefix, ngroups, ncls, chunk, blockIdx.x, gridDim.x);
+    ItemWalk<true> walk(cls_prefix, ngroups, ncls, chunk, blockIdx.x, gridDim.x);
     // pass 1's bits where pass 4 has its lists
     uint32_t* bits = reinterpret_cast<uint32_t*>(&s_w[wave_in_block()]);
     while (walk.next()) batch_classify_item(jobs, group_job, mask, walk.j, walk.i, bits);
     grid.sync();
-    batch_count_items(jobs, ItemWalk(lane_prefix, njobs, nlane, chunk, blockIdx.x, gridDim.x), mask, counts, trims,
-                      state + 2, shift);
+    batch_count_items(jobs, ItemWalk<true>(lane_prefix, njobs, nlane, chunk, blockIdx.x, gridDim.x), mask, counts,
+                      trims, state + 2, shift);
     grid.sync();
     for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x)
         fe_scan_tile(counts, R, voff, toff, state + 2, shift, ntiles, state, host + 4 * (int64_t)njobs, ScanMore(), tile);
